@@ -96,8 +96,6 @@ __device__ __forceinline__ TileCtx tile_ctx(const DeviceView& v, int t) {
 
 __device__ __forceinline__ int row_start(const TileCtx& c, int I) { return c.base + I * c.nT - (I * (I - 1)) / 2; }
 
-__device__ __forceinline__ size_t pslot(int w, int side, int lane) { return ((size_t)w * 2 + side) * kTile + lane; }
-
 // Calls add(item, side) for this wave's items in their fixed order. Systems
 // whose far items carry no partials test 64 candidates per vector load of
 // the item classes and visit only the active ones.
@@ -237,21 +235,19 @@ __device__ __forceinline__ void gather_items(const DeviceView& v, const TileCtx&
 
 // Scalar partials (Born sums) of this wave's items for the lane's atom.
 __device__ __forceinline__ double gather1(const DeviceView& v, const TileCtx& c) {
-  const float* pb = reinterpret_cast<const float*>(v.part);
   double acc = 0.0;
-  gather_items<float>(v, c, [&](int w, int side, int lane) { return pb[pslot(w, side, lane)]; },
+  gather_items<float>(v, c, [&](int w, int side, int lane) { return part1(v, w, side)[lane]; },
                       [&](float x) { acc += (double)x; });
   return acc;
 }
 
 // Chain partials: three float arrays of 64 per (item, side).
 __device__ __forceinline__ double4 gather3(const DeviceView& v, const TileCtx& c) {
-  const float* pc = reinterpret_cast<const float*>(v.part);
   double4 acc = make_double4(0.0, 0.0, 0.0, 0.0);
   gather_items<float3>(
       v, c,
       [&](int w, int side, int lane) {
-        const float* q = pc + ((size_t)w * 2 + side) * (3 * kTile) + lane;
+        const float* q = part3(v, w, side) + lane;
         return make_float3(q[0], q[kTile], q[2 * kTile]);
       },
       [&](float3 p) { acc.x += p.x; acc.y += p.y; acc.z += p.z; });
@@ -260,7 +256,7 @@ __device__ __forceinline__ double4 gather3(const DeviceView& v, const TileCtx& c
 
 __device__ __forceinline__ double4 gather4(const DeviceView& v, const TileCtx& c) {
   double4 acc = make_double4(0.0, 0.0, 0.0, 0.0);
-  gather_items<float4>(v, c, [&](int w, int side, int lane) { return v.part[pslot(w, side, lane)]; },
+  gather_items<float4>(v, c, [&](int w, int side, int lane) { return part4(v, w, side)[lane]; },
                        [&](float4 p) { acc.x += p.x; acc.y += p.y; acc.z += p.z; acc.w += p.w; });
   return acc;
 }

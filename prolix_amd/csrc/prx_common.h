@@ -148,7 +148,7 @@ struct DeviceView {
   // pair work
   const PairItem* items;
   int32_t n_items;
-  float4* part;        // partial sums: item w, side s (0 = i, 1 = j), lane l -> part[(w * 2 + s) * 64 + l]
+  float4* part;        // partial sums, 2 * 64 float4 per item (part1 / part3 / part4 below)
   const int4* tiles;   // per tile: (first atom, atoms in tile, slot, tile index T)
   int32_t n_tiles;
   const unsigned long long* excl_masks;  // 128 per exclusion tile: lane * 2 + {bit0, bit1}
@@ -191,6 +191,21 @@ struct DeviceView {
   // forces stand); 0 for evaluations, which compute every item
   int32_t skip_done;
 };
+
+// Partial sums of item w, side s (0 = i atoms, 1 = j atoms): 64 floats (Born
+// pass), three arrays of 64 floats (chain pass) or 64 float4 (force pass).
+// Every pass starts an item at the same 2 KB stride, so the items of two
+// systems never share bytes: in the fused step kernel systems run different
+// passes at the same time.
+__device__ __forceinline__ float4* part4(const DeviceView& v, int w, int s) {
+  return v.part + ((size_t)w * 2 + s) * kTile;
+}
+__device__ __forceinline__ float* part1(const DeviceView& v, int w, int s) {
+  return reinterpret_cast<float*>(part4(v, w, 0)) + s * kTile;
+}
+__device__ __forceinline__ float* part3(const DeviceView& v, int w, int s) {
+  return reinterpret_cast<float*>(part4(v, w, 0)) + s * (3 * kTile);
+}
 
 // Grid-wide barrier state of the persistent step kernel (device memory).
 struct GridBarrier {

@@ -25,16 +25,11 @@ __device__ __forceinline__ float rot(float x) {
   return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), PRX_DPP_WAVE_ROL1, 0xF, 0xF, true));
 }
 
-// Partial-buffer slot of (item w, side, lane); side 0 = i atoms, 1 = j atoms.
-__device__ __forceinline__ size_t part_slot(int w, int side, int lane) {
-  return ((size_t)w * 2 + side) * kTile + lane;
-}
-
 // Chain partials carry three components: stored as three float arrays of 64
 // per (item, side), each written and read whole by a wave.
 __device__ __forceinline__ void put_part3(const DeviceView& v, int w, int side, int lane, float x, float y,
                                           float z) {
-  float* pc = reinterpret_cast<float*>(v.part) + ((size_t)w * 2 + side) * (3 * kTile);
+  float* pc = part3(v, w, side);
   pc[lane] = x;
   pc[kTile + lane] = y;
   pc[2 * kTile + lane] = z;
@@ -362,14 +357,13 @@ __device__ __forceinline__ void born_tile(const DeviceView& v, const PairItem& i
     if (k != kend) accJ = rot<PRX_ROT_BPERM_BORN>(accJ);
 #endif
   }
-  float* pb = reinterpret_cast<float*>(v.part);  // scalar partials
-  pb[part_slot(w, 0, lane)] = accI;
+  part1(v, w, 0)[lane] = accI;
 #if PRX_LDS_ACC
   wave_lds_sync();
-  pb[part_slot(w, 1, lane)] = L.acc[lane] + L.acc[lane + 64];
+  part1(v, w, 1)[lane] = L.acc[lane] + L.acc[lane + 64];
 #else
   const int home = (lane + kend) & 63;
-  pb[part_slot(w, 1, home)] = accJ;
+  part1(v, w, 1)[home] = accJ;
 #endif
 }
 
@@ -613,16 +607,16 @@ __device__ __forceinline__ void force_tile(const DeviceView& v, const PairItem& 
     }
 #endif
   }
-  v.part[part_slot(w, 0, lane)] = make_float4(fxi, fyi, fzi, -0.5f * dbi);
+  part4(v, w, 0)[lane] = make_float4(fxi, fyi, fzi, -0.5f * dbi);
 #if PRX_LDS_ACC
   wave_lds_sync();
   {
     const float4 a0 = L.acc[lane], a1 = L.acc[lane + 64];
-    v.part[part_slot(w, 1, lane)] = make_float4(a0.x + a1.x, a0.y + a1.y, a0.z + a1.z, -0.5f * (a0.w + a1.w));
+    part4(v, w, 1)[lane] = make_float4(a0.x + a1.x, a0.y + a1.y, a0.z + a1.z, -0.5f * (a0.w + a1.w));
   }
 #else
   const int home = (lane + kend) & 63;
-  v.part[part_slot(w, 1, home)] = make_float4(fxj, fyj, fzj, -0.5f * dbj);
+  part4(v, w, 1)[home] = make_float4(fxj, fyj, fzj, -0.5f * dbj);
 #endif
   if (ENERGY) {
     for (int off = 32; off > 0; off >>= 1) {
