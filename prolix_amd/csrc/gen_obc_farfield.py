@@ -22,7 +22,10 @@ s < 0.6 r, and s <= r/2 excludes under 0.5% of the pairs.
 A second pair of fits covers y in [0, Y_MAX4] (s <= r/4) at degree 4 for
 both (relative error 3.1e-9 and 1.1e-8): the pair kernels use them for work
 items whose tiles are at least 4 s apart in every pair, where they save two
-and three multiply-adds per direction at no loss of accuracy.
+and three multiply-adds per direction at no loss of accuracy. Two more pairs
+do the same further out: degree 3 for s <= r/6.5 and degree 2 for s <= r/14.5,
+each as accurate, so with the distance of two tiles the polynomials get
+shorter and no pair gets less accurate.
 
 Run: python prolix_amd/csrc/gen_obc_farfield.py > prolix_amd/csrc/prx_obc_farfield.h
 """
@@ -35,6 +38,8 @@ DEG_K = 7
 Y_MAX4 = 0.0625  # x <= 0.25
 DEG_H4 = 4
 DEG_K4 = 4
+# (suffix, smallest r / s, degree of h and of k)
+SHORTER = ((3, 6.5, 3), (2, 14.5, 2))
 
 
 def h_series(y):
@@ -78,6 +83,14 @@ def main():
     print(f"__device__ constexpr float kObcH4[{DEG_H4 + 1}] = {{{fmt(ch4)}}};")
     print(f"constexpr int kObcK4Deg = {DEG_K4};")
     print(f"__device__ constexpr float kObcK4[{DEG_K4 + 1}] = {{{fmt(ck4)}}};")
+    for n, ratio, deg in SHORTER:
+        h, eh = fit(h_series, deg, 1.0 / ratio**2)
+        k, ek = fit(k_series, deg, 1.0 / ratio**2)
+        print("// The same for s <= r/%g; max relative error: h %.2e, k %.2e" % (ratio, eh, ek))
+        print(f"#define PRX_OBC_FAR{n}_XMAX {1.0 / ratio:.9g}f")
+        print(f"constexpr int kObcH{n}Deg = {deg}, kObcK{n}Deg = {deg};")
+        print(f"__device__ constexpr float kObcH{n}[{deg + 1}] = {{{fmt(h)}}};")
+        print(f"__device__ constexpr float kObcK{n}[{deg + 1}] = {{{fmt(k)}}};")
 
 
 if __name__ == "__main__":

@@ -28,7 +28,39 @@ struct PairItem {
   int32_t j0;    // global index of the j tile's first atom
   int32_t meta;  // ni (bits 0-6), nj (bits 7-13), flags (bits 14-15), slot (bits 16-31)
   int32_t excl;  // exclusion-mask tile index, or -1
+  int32_t ti, tj;  // global indices of the two tiles (a chunk item's ti is its row's; tj unused)
+  int32_t nsub;    // shares of the item (1, 2 or kUnitWaves, prx_pair_dev.h)
+  int32_t pad;
 };
+// Unit of the pair passes, the work of a group of kUnitWaves waves: the items
+// first .. first + n - 1, each cut into the same number of shares, a share per
+// wave (n * shares <= kUnitWaves).
+constexpr int kUnitWaves = 4;
+struct PairUnit {
+  int32_t first;
+  int16_t n, shares;
+};
+// Shares of the items of a system by its size (item_shares). A wave alone on
+// its SIMD issues at half rate and no other hides its loads, and a system of a few
+// thousand atoms has fewer items than the chip has SIMDs (2,500 atoms: 820 of
+// 1,024), so that a pass takes the time of one item on one wave. Alone, whole
+// items / 2 shares / 4 shares, us a pass (Born, force, chain):
+//     3,000 atoms   24.4 23.4 31.1 / 17.6 16.6 20.2 / 16.0 13.8 17.4
+//     5,000 atoms   27.4 31.9 33.7 / 21.0 25.9 26.5 / 21.2 24.4 25.2
+//     8,000 atoms   40.2 52.5 49.9 / 34.3 47.8 43.3 / 32.3 49.0 40.2
+// In a pack that fills the chip each share more costs 3 to 4% of a pass
+// (the column sums of a share are summed over its lanes; 256 systems of 300 to 5,000
+// atoms: 322, 624, 457 us with these lines, 344, 673, 497 with 4 shares for
+// all), so systems above kQuarterTiles, where most of a pack's items are, take 2,
+// and above kHalfTiles, where one system fills the chip, items stay whole.
+constexpr int kQuarterTiles = 40;
+constexpr int kHalfTiles = 128;
+// Work lists of at least this many items (9 or more per SIMD) run one wave per
+// item, shorter ones a group of waves per unit. 16,110 items of four systems:
+// 35, 54, 52 us a pass with waves, 33, 50, 44 with units; 142,848 items: 319,
+// 609, 445 us with waves, 470, 686, 540 with units.
+constexpr int kWaveItems = 10000;
+
 constexpr int kFlagDiag = 1;
 constexpr int kFlagExcl = 2;
 
@@ -39,13 +71,11 @@ constexpr int kClsNear = 0;      // every pair closer than the cutoff (or no cut
 constexpr int kClsStraddle = 1;  // per-pair r^2 < cutoff^2 test needed
 constexpr int kClsFar = 2;       // every pair at or beyond the cutoff
 constexpr int kClsCutMask = 3;
-// Bit 2: every pair of the item is in the OBC2 far field in both directions
-// (r - s_j > rho_i, s_j <= r/2 and the same with i, j swapped), so the Born
-// and chain passes use the far-field polynomials without a per-pair test.
-constexpr int kClsObcFar = 4;
-// Bit 3: in addition, every pair has s <= r/4 in both directions, where the
-// far-field polynomials of degree 4 are as accurate as the wider fits.
-constexpr int kClsObcFar4 = 8;
+// Bits 2-4: how far into the OBC2 far field every pair of the item is known to
+// be (the tiers of prx_pair_dev.h), so that the Born and chain passes need no
+// per-pair test and a polynomial of the lowest degree that is as accurate.
+constexpr int kClsTierShift = 2;
+constexpr int kClsMask = 31;
 
 __host__ __device__ inline int32_t item_meta(int ni, int nj, int flags, int slot) {
   return ni | (nj << 7) | (flags << 14) | (slot << 16);
@@ -73,6 +103,7 @@ struct SlotConst {
   int32_t caps;         // 1: batched-step safety caps (velocity, displacement, force)
   int32_t tile0;        // global index of the system's first tile
   uint64_t seed;
+  int32_t unit0, n_units;  // the system's units
   // neighbour-list systems (gb_cut with a cutoff): list build and reuse
   int32_t nl;           // 1: pair work from the list (chunk items), 0: all tile pairs
   int32_t tp_base;      // global index of the system's first tile pair (I < J) record
@@ -120,8 +151,8 @@ struct ExceptionEntry { int4 idx; float4 p; };  // idx.xy pair; p = (sigma, eps,
 //    order (nl_entries from the row's entry base, nl_count[I] of them),
 //    evaluated 64 at a time by chunk items (PairItem.j0 < 0, see below).
 // Tile pairs with exclusions and the diagonal tiles stay ordinary items.
-// Chunk item: j0 = -1 - (global entry index of its first j atom); excl = the
-// global tile index of its row; ni = atoms of the i tile.
+// Chunk item: j0 = -1 - (global entry index of its first j atom); excl = -1;
+// ti = the global tile index of its row; ni = atoms of the i tile.
 __host__ __device__ inline bool item_is_chunk(const PairItem& it) { return it.j0 < 0; }
 // Per-tile-pair record: I | J << 16 (local tiles), and the slot (~slot for a
 // pair with exclusions, which the list skips; x = -1 for a free record).
@@ -136,7 +167,7 @@ struct DeviceView {
   float4* pos;         // x, y, z, 0
   float4* mom;         // px, py, pz, 1/m
   float4* force;       // integrator force (float), w unused
-  float4* born4;       // rho, sr, sr^2, sr^3/2       (static)
+  float4* born4;       // rho, sr, sr^2, sr^3/3       (static)
   float4* nb4;         // q, sigma/2, sqrt(eps), 0    (static)
   double4* fin4;       // rho, R, q^2, ace_K          (static, FP64)
   float* sqrt_m;       // sqrt(mass)                  (static)
@@ -148,13 +179,15 @@ struct DeviceView {
   // pair work
   const PairItem* items;
   int32_t n_items;
+  const PairUnit* units;  // nullptr: unit = item, every item cut
+  int32_t n_units;
   float4* part;        // partial sums, 2 * 64 float4 per item (part1 / part3 / part4 below)
   const int4* tiles;   // per tile: (first atom, atoms in tile, slot, tile index T)
   int32_t n_tiles;
   const unsigned long long* excl_masks;  // 128 per exclusion tile: lane * 2 + {bit0, bit1}
   double* e_items;     // 3 per item: GB pairs, Coulomb, LJ
   float4* tbox;        // per tile t: (lo.xyz, max rho) at 2t, (hi.xyz, max s) at 2t + 1
-  int32_t* item_cls;   // per item: class bits (kCls*), written by the Born pass
+  int32_t* item_cls;   // per item: class bits (kCls*) and far-field threshold, written by the Born pass
   // bonded
   BondEntry* bonds; int32_t bond_hw;
   AngleEntry* angles; int32_t angle_hw;

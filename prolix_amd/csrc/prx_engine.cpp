@@ -252,7 +252,10 @@ void validate(const prx_system_desc& d) {
 constexpr size_t kScratchBytes = (size_t)32 << 20;
 constexpr int kScratchMaxAtoms = 8192;
 constexpr int kMaxDevices = 64;
-static __device__ __align__(256) unsigned char scratch[kScratchBytes];
+// The pair items lie behind the region that a system's buffers are held
+// against; in it an item takes 2 KB of partials.
+constexpr size_t kScratchItems = kScratchBytes / (2 * prx::kTile * sizeof(float4));
+static __device__ __align__(256) unsigned char scratch[kScratchBytes + kScratchItems * sizeof(prx::PairItem)];
 
 namespace {
 std::mutex g_scratch_mu;
@@ -354,11 +357,12 @@ struct prx_engine {
   bool has_nl = false;            // a live system uses its neighbour list
   // step path: 0 = auto (the fused kernel when every system fits in
   // kFusedAutoAtoms atoms and none uses a neighbour list, else graphs: on
-  // MI355X the fused kernel beats graphs only there, measured from 138 to
-  // 2,500 atoms), 1 = captured graphs, 2 = the persistent kernel, 3 = the
+  // MI355X the fused kernel beats graphs only on systems of one tile. us a step,
+  // fused / graphs: 64 atoms 32 / 43, 100 atoms 52 / 43, 138 atoms 77 / 44; 192
+  // systems of 64 atoms 34 / 47, of 100 atoms 57 / 54), 1 = captured graphs, 2 = the persistent kernel, 3 = the
   // fused kernel (one workgroup per system)
   int32_t step_mode = 0;
-  static constexpr int32_t kFusedAutoAtoms = 3 * prx::kTile;
+  static constexpr int32_t kFusedAutoAtoms = prx::kTile;
   int32_t max_system_atoms = 0;   // largest live system (rebuild)
   prx::GridBarrier* d_bar = nullptr;
   int persist_blocks = -1;        // co-resident grid of the persistent kernel (0: unavailable)
@@ -375,6 +379,7 @@ struct prx_engine {
   // device buffers owned here
   prx::PairItem* d_items = nullptr;
   int64_t cap_items = 0;
+  prx::PairUnit* d_units = nullptr;
   float4* d_part = nullptr;   // 2 * 64 partials per item
   // positions and forces of prx_energy_forces: an evaluation at arbitrary
   // positions leaves the integrator's state (v.pos, v.force) untouched
@@ -427,7 +432,13 @@ struct prx_engine {
   // holds one fixed set of systems); otherwise rebuild() sizes them.
   void alloc_work(int64_t n_items, int64_t n_tiles) {
     cap_items = n_items;
-    d_items = get<prx::PairItem>(cap_items);
+    if (arena) {  // room for 16 bytes an item is counted here
+      d_units = reinterpret_cast<prx::PairUnit*>(get<float4>(cap_items));
+      d_items = reinterpret_cast<prx::PairItem*>(arena + arena_cap);
+    } else {
+      d_items = get<prx::PairItem>(cap_items);
+      d_units = get<prx::PairUnit>(cap_items);
+    }
     d_e_items = get<double>(cap_items * 3);
     d_part = get<float4>(cap_items * 2 * prx::kTile);
     d_item_cls = get<int32_t>(cap_items);
@@ -540,7 +551,7 @@ struct prx_engine {
     void* ptrs[] = {v.pos, v.mom, v.force, v.born4, v.nb4, v.fin4, v.sqrt_m, v.slot_of, v.gb4, v.fpair, d_part, d_tiles,
                     v.e_atom, v.atom_step, v.bonds, v.angles, v.tors, v.cmaps, v.excs, v.e_bond, v.e_angle,
                     v.e_tors, v.e_cmap, v.e_exc, d_coeff, d_excl, v.slots, d_ranges, d_slot_list,
-                    d_energy_tmp, d_map, d_items, d_e_items, v.rec, v.atom_rec, d_rec_list, v.warn,
+                    d_energy_tmp, d_map, d_items, d_units, d_e_items, v.rec, v.atom_rec, d_rec_list, v.warn,
                     d_tbox, d_item_cls, d_eval_pos, d_eval_force, d_nl_tp, d_nl_mask, d_nl_pref,
                     d_nl_entries, d_nl_xref, d_nl_flag, d_nl_row, d_nl_count, d_nl_col, d_nl_colitems, d_bar};
     for (void* p : ptrs)
@@ -649,7 +660,7 @@ struct prx_engine {
       const double sig = std::max(d.sigmas[i], 1e-6);
       const double m = d.masses ? d.masses[i] : 1.0;
       if (!(m > 0.0)) throw std::invalid_argument("masses must be positive");
-      born4[i] = make_float4((float)rho, (float)sr, (float)(sr * sr), (float)(0.5 * sr * sr * sr));
+      born4[i] = make_float4((float)rho, (float)sr, (float)(sr * sr), (float)(sr * sr * sr / 3.0));
       nb4[i] = make_float4((float)q, (float)(0.5 * sig), (float)std::sqrt(std::max(d.epsilons[i], 0.0)), 0.0f);
       const double rn = (R - off) / 10.0 + 0.009;
       const double aceK = d.implicit_solvent
@@ -874,6 +885,7 @@ struct prx_engine {
     // allocation-free entry point has synchronised its stream already)
     if (!arena) HIPCHECK(hipDeviceSynchronize());
     std::vector<prx::PairItem> items;
+    std::vector<prx::PairUnit> units;
     std::vector<int32_t> ranges;
     std::vector<int32_t> map;
     std::vector<int4> tiles;
@@ -881,6 +893,7 @@ struct prx_engine {
     std::vector<int2> nl_col;
     std::vector<int32_t> nl_colitems;
     offsets.assign(1, 0);
+    bool all_cut = true;
     max_system_atoms = 0;
     has_nl = false;
     for (int32_t sid : order) {
@@ -888,8 +901,12 @@ struct prx_engine {
       const int32_t ib = (int32_t)items.size();
       s.c.item_base = ib;
       s.c.tile0 = (int32_t)tiles.size();
-      push_const(sid, s.c);
       const int nT = (s.n + prx::kTile - 1) / prx::kTile;
+      const int32_t n_it = (int32_t)s.items.size();
+      s.c.unit0 = (int32_t)units.size();
+      all_cut = prx::append_units(s.items, ib, units) && all_cut;
+      s.c.n_units = (int32_t)units.size() - s.c.unit0;
+      push_const(sid, s.c);
       for (int T = 0; T < nT; ++T) {
         tiles.push_back(make_int4(s.a0 + T * prx::kTile, std::min(prx::kTile, s.n - T * prx::kTile), sid, T));
         if (s.nl) {
@@ -904,9 +921,10 @@ struct prx_engine {
       }
       has_nl = has_nl || s.nl;
       items.insert(items.end(), s.items.begin(), s.items.end());
-      if (s.nl)  // chunk items name their row's global tile
-        for (size_t k = items.size() - s.items.size(); k < items.size(); ++k)
-          if (prx::item_is_chunk(items[k])) items[k].excl += s.c.tile0;
+      for (size_t k = items.size() - s.items.size(); k < items.size(); ++k) {
+        items[k].ti += s.c.tile0;
+        items[k].tj += s.c.tile0;
+      }
       const int32_t r[14] = {ib, (int32_t)items.size(), s.a0, s.n, (int32_t)s.bond_b, (int32_t)(s.bond_b + s.bond_n),
                              (int32_t)s.ang_b, (int32_t)(s.ang_b + s.ang_n), (int32_t)s.tors_b,
                              (int32_t)(s.tors_b + s.tors_n), (int32_t)s.cmap_b, (int32_t)(s.cmap_b + s.cmap_n),
@@ -923,7 +941,9 @@ struct prx_engine {
       if (d_part) HIPCHECK(hipFree(d_part));
       cap_items = std::max<int64_t>((int64_t)items.size(), cap_items * 3 / 2);
       if (d_item_cls) HIPCHECK(hipFree(d_item_cls));
+      if (d_units) HIPCHECK(hipFree(d_units));
       d_items = dalloc<prx::PairItem>(cap_items);
+      d_units = dalloc<prx::PairUnit>(cap_items);  // a unit holds an item at least
       d_e_items = dalloc<double>(cap_items * 3);
       d_part = dalloc<float4>(cap_items * 2 * prx::kTile);
       d_item_cls = dalloc<int32_t>(cap_items);
@@ -959,11 +979,15 @@ struct prx_engine {
       HIPCHECK(hipMemcpy(d_tiles, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice));
     if (!items.empty())
       HIPCHECK(hipMemcpy(d_items, items.data(), items.size() * sizeof(prx::PairItem), hipMemcpyHostToDevice));
+    if (!units.empty())
+      HIPCHECK(hipMemcpy(d_units, units.data(), units.size() * sizeof(prx::PairUnit), hipMemcpyHostToDevice));
     if (!ranges.empty())
       HIPCHECK(hipMemcpy(d_ranges, ranges.data(), ranges.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     if (!map.empty()) HIPCHECK(hipMemcpy(d_map, map.data(), map.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     v.items = d_items;
     v.n_items = (int32_t)items.size();
+    v.units = all_cut ? nullptr : d_units;
+    v.n_units = (int32_t)units.size();
     v.e_items = d_e_items;
     v.part = d_part;
     v.tiles = d_tiles;
@@ -1122,10 +1146,10 @@ struct prx_engine {
     return true;
   }
 
-  // The persistent kernel: at most one item per wave and one tile per block
-  // in each pass, within the co-resident grid.
+  // The persistent kernel: at most one unit and one tile per block in each
+  // pass, within the co-resident grid.
   void steps_persistent(int n_steps, hipStream_t s) {
-    const int64_t want = std::max<int64_t>({(int64_t)v.n_tiles, ((int64_t)v.n_items + 3) / 4, 1});
+    const int64_t want = std::max<int64_t>({(int64_t)v.n_tiles, (int64_t)v.n_units, 1});
     const int blocks = (int)std::min<int64_t>(want, persist_blocks);
     for (int left = n_steps; left > 0;) {
       const int k = std::min(left, kPersistChunk);

@@ -32,8 +32,9 @@ namespace prx {
 
 namespace {
 
-constexpr int kFusedGroups = 2;                  // tile gathers side by side
+constexpr int kFusedGroups = 2;                  // groups of four waves: units and tile gathers side by side
 constexpr int kFusedWaves = kGW * kFusedGroups;  // 8
+static_assert(kGW == kUnitWaves, "a group runs a unit or a tile gather");
 constexpr int kFusedThreads = kFusedWaves * 64;
 
 // The bonded entries of one system (its ranges in each kind's arena).
@@ -45,31 +46,36 @@ __device__ __forceinline__ void bonded_slot(const DeviceView& v, const int32_t* 
   for (int e = R[12] + (int)threadIdx.x; e < R[13]; e += kFusedThreads) do_exception<false>(v, e);
 }
 
-// One round of tile gathers: group g of four waves gathers tile t + g, or,
-// past the last tile, takes the one barrier that gather would have held.
-// Then the round's barrier, before the workgroup memory is used again.
-template <class F>
-__device__ __forceinline__ void gather_round(int t, int t1, int grp, F&& gather) {
-  if (t + grp < t1)
-    gather(t + grp);
-  else
-    __syncthreads();
+// One round of units or tile gathers: group g of four waves takes unit or tile
+// t + g, or, past the last one, the barriers that it would have held (two a
+// unit, one a gather). Then the round's barrier, before the workgroup memory is
+// used again.
+template <int BARRIERS, class F>
+__device__ __forceinline__ void group_round(int t, int t1, int grp, F&& work) {
+  if (t + grp < t1) {
+    work(t + grp);
+  } else {
+    for (int k = 0; k < BARRIERS; ++k) __syncthreads();
+  }
   __syncthreads();
 }
 
 // Block b: the b-th listed system, ranges row b (item_b, item_e, a0, n, then
 // the bonded ranges).
 __global__ __launch_bounds__(kFusedThreads) void k_fused_steps(DeviceView v, const int32_t* ranges, int n_steps) {
-  __shared__ PassLds lds[kFusedWaves];
+  __shared__ UnitLds<kPairLds> ulds[kFusedGroups];
   __shared__ GatherLds glds[kFusedGroups];
-  PassLds& L = lds[threadIdx.x >> 6];
   const int32_t* R = ranges + (size_t)blockIdx.x * kRangeInts;
-  const int item_b = R[0], item_e = R[1], a0 = R[2], n = R[3];
+  const int a0 = R[2], n = R[3];
   if (n <= 0) return;
-  const int t0 = v.slots[v.slot_of[a0]].tile0;
+  const SlotConst& S = v.slots[v.slot_of[a0]];
+  const int u0 = S.unit0, u1 = u0 + S.n_units;
+  const int t0 = S.tile0;
   const int t1 = t0 + (n + kTile - 1) / kTile;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int grp = wave / kGW;
+  const int uw = unit_wave();
+  UnitLds<kPairLds>& L = ulds[grp];
   GatherLds& G = glds[grp];
 
   // B A O A of the first step from the stored force, then the tile boxes
@@ -79,20 +85,20 @@ __global__ __launch_bounds__(kFusedThreads) void k_fused_steps(DeviceView v, con
   __syncthreads();
 
   for (int k = 0; k < n_steps; ++k) {
-    for (int w = item_b + wave; w < item_e; w += kFusedWaves) born_item(v, w, L.born);
     bonded_slot(v, R);
-    __syncthreads();
+    for (int u = u0; u < u1; u += kFusedGroups)
+      group_round<2>(u, u1, grp, [&](int uu) { pair_unit<true, BornPass>(v, uu, uw, L); });
     for (int t = t0; t < t1; t += kFusedGroups)
-      gather_round(t, t1, grp, [&](int tt) { born_gather_tile(v, tt, G); });
-    for (int w = item_b + wave; w < item_e; w += kFusedWaves) force_item<false>(v, w, L.pair);
-    __syncthreads();
+      group_round<1>(t, t1, grp, [&](int tt) { born_gather_tile(v, tt, G); });
+    for (int u = u0; u < u1; u += kFusedGroups)
+      group_round<2>(u, u1, grp, [&](int uu) { pair_unit<true, ForcePass<false>>(v, uu, uw, L); });
     for (int t = t0; t < t1; t += kFusedGroups)
-      gather_round(t, t1, grp, [&](int tt) { force_gather_tile<false>(v, tt, G); });
-    for (int w = item_b + wave; w < item_e; w += kFusedWaves) chain_item(v, w, L.pair);
-    __syncthreads();
+      group_round<1>(t, t1, grp, [&](int tt) { force_gather_tile<false>(v, tt, G); });
+    for (int u = u0; u < u1; u += kFusedGroups)
+      group_round<2>(u, u1, grp, [&](int uu) { pair_unit<true, ChainPass>(v, uu, uw, L); });
     const int mode = k + 1 == n_steps ? 2 : 1;  // the last step stops after B(F)
     for (int t = t0; t < t1; t += kFusedGroups)
-      gather_round(t, t1, grp, [&](int tt) { chain_gather_tile(v, tt, mode, G); });
+      group_round<1>(t, t1, grp, [&](int tt) { chain_gather_tile(v, tt, mode, G); });
   }
 }
 

@@ -249,6 +249,9 @@ void build_exclusions(const prx_system_desc& d, ExclPlan& plan) {
   }
 }
 
+// Shares of every item of a system of nT tiles.
+static int item_shares(int nT) { return nT <= kQuarterTiles ? kUnitWaves : (nT <= kHalfTiles ? 2 : 1); }
+
 void build_items(int n_atoms, int a0, int slot, const ExclPlan& plan, int excl_base,
                  std::vector<PairItem>& out) {
   const int nT = (n_atoms + kTile - 1) / kTile;
@@ -270,8 +273,20 @@ void build_items(int n_atoms, int a0, int slot, const ExclPlan& plan, int excl_b
       p.j0 = a0 + J * kTile;
       p.meta = item_meta(ni, nj, flags, slot);
       p.excl = ex;
+      p.ti = I;
+      p.tj = J;
+      p.nsub = item_shares(nT);
+      p.pad = 0;
       out.push_back(p);
     }
+}
+
+bool append_units(const std::vector<PairItem>& items, int base, std::vector<PairUnit>& out) {
+  if (items.empty()) return true;
+  const int shares = items[0].nsub, per = kUnitWaves / shares, n = (int)items.size();
+  for (int k = 0; k < n; k += per)
+    out.push_back({base + k, (int16_t)std::min(per, n - k), (int16_t)shares});
+  return shares == kUnitWaves;
 }
 
 namespace {
@@ -330,6 +345,10 @@ void build_items_nl(int n_atoms, int a0, int slot, const ExclPlan& plan, int exc
       p.j0 = a0 + J * kTile;
       p.meta = item_meta(n_of(I), n_of(J), flags, slot);
       p.excl = ex;
+      p.ti = I;
+      p.tj = J;
+      p.nsub = item_shares(nT);
+      p.pad = 0;
       out.cols[J].push_back((int32_t)out.items.size());
       out.items.push_back(p);
     }
@@ -354,7 +373,11 @@ void build_items_nl(int n_atoms, int a0, int slot, const ExclPlan& plan, int exc
       p.i0 = a0 + I * kTile;
       p.j0 = (int32_t)(-1 - (ent_b + ent + c));
       p.meta = item_meta(n_of(I), kTile, 0, slot);
-      p.excl = I;
+      p.excl = -1;
+      p.ti = I;
+      p.tj = I;
+      p.nsub = item_shares(nT);
+      p.pad = 0;
       out.items.push_back(p);
     }
     ent += cap;

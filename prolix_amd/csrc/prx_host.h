@@ -18,9 +18,14 @@ struct ExclPlan {
 void cmap_coefficients(const double* grid_psi_phi, int G, double* out);
 // Exclusion classes and 64x64 tile masks of one system (throws std::invalid_argument).
 void build_exclusions(const prx_system_desc& d, ExclPlan& plan);
-// Tile pairs I <= J of one system placed at arena offset a0.
+// Tile pairs I <= J of one system placed at arena offset a0; ti and tj are the
+// system's own tile indices (the engine adds its first global tile).
 void build_items(int n_atoms, int a0, int slot, const ExclPlan& plan, int excl_base,
                  std::vector<PairItem>& out);
+
+// Appends the units of one system's items, whose first has index base. True if
+// each is one item in kUnitWaves shares.
+bool append_units(const std::vector<PairItem>& items, int base, std::vector<PairUnit>& out);
 
 // Work layout of a neighbour-list system (relative to the system: item
 // indices from its first item, entries from its entry base, tiles local).
@@ -34,8 +39,7 @@ struct NlPlan {
 // Tile-pair count and list capacity of a neighbour-list system, without building it.
 void nl_sizes(int n_atoms, const ExclPlan& plan, int64_t* n_tp, int64_t* n_entries, int64_t* n_items);
 // Items for arena offset a0 and entry base ent_b: chunk items carry
-// j0 = -1 - (ent_b + first entry) and excl = local row tile (the engine adds
-// the system's first global tile).
+// j0 = -1 - (ent_b + first entry); ti and tj are local as in build_items.
 void build_items_nl(int n_atoms, int a0, int slot, const ExclPlan& plan, int excl_base, int64_t ent_b,
                     NlPlan& out);
 

@@ -15,3 +15,13 @@ constexpr int kObcH4Deg = 4;
 __device__ constexpr float kObcH4[5] = {0.66666666872154989f, 0.79999836766752519f, 0.85734960136170812f, 0.87978772663299587f, 1.0697785612734509f};
 constexpr int kObcK4Deg = 4;
 __device__ constexpr float kObcK4[5] = {1.3333333480933838f, 2.3999882868211322f, 3.4300527588646554f, 4.3793952777570881f, 6.5973534742035334f};
+// The same for s <= r/6.5; max relative error: h 3.53e-09, k 1.07e-08
+#define PRX_OBC_FAR3_XMAX 0.153846154f
+constexpr int kObcH3Deg = 3, kObcK3Deg = 3;
+__device__ constexpr float kObcH3[4] = {0.66666666431269472f, 0.80000317176590752f, 0.85647660317730745f, 0.93342088098950193f};
+__device__ constexpr float kObcK3[4] = {1.3333333190797376f, 2.4000191945887033f, 3.4245432458952312f, 4.7131794432933019f};
+// The same for s <= r/14.5; max relative error: h 4.52e-09, k 1.13e-08
+#define PRX_OBC_FAR2_XMAX 0.0689655172f
+constexpr int kObcH2Deg = 2, kObcK2Deg = 2;
+__device__ constexpr float kObcH2[3] = {0.66666666968101695f, 0.79998860299052732f, 0.86352069034728762f};
+__device__ constexpr float kObcK2[3] = {1.3333333484308443f, 2.399942928361444f, 3.460496959115233f};

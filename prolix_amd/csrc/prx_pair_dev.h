@@ -1,39 +1,35 @@
 // Device code of the pair passes, shared by prx_pair.hip (one kernel per
-// pass) and prx_persist.hip (every pass of a step in one persistent kernel).
-// born_item / force_item / chain_item are one wave's work on one item.
+// pass), prx_persist.hip and prx_fused.hip (every pass of a step in one kernel).
+// BornPass, ForcePass and ChainPass are a wave's work on an item, or on a share
+// of one ("Items to waves" below).
+//
+// A 64x64 item is 8x8 patches of 8x8 pairs. Lane l = 8 q + p takes the pair
+// (row 8 b + q of tile I, column 8 a + p of tile J) of patch (b, a). Rows are
+// read from LDS once per b and columns once per patch; the sums of the wave's
+// eight columns (a = 0..7) stay in registers for the whole item, those of a row
+// are added over the eight lanes p by DPP once per eight patches, and the
+// columns' over q once at the end, so that no sum moves between lanes in the
+// loop. Near pairs, which need square root, logarithm and clamps, are taken out
+// of the loop: it marks their patches, and they are listed and evaluated 64 at
+// a time behind it.
+//
+// What bounds it: VALU issue. gfx950 issues a plain FP32 instruction of one
+// wave every 4.4 cycles and, with two or more waves per SIMD, one every 2.2
+// cycles; transcendentals take 8.4, DPP operands 4.2, and the LDS of a CU
+// takes 6 cycles per ds_bpermute and 8 per 16-byte read of a wave. One j atom
+// per lane and iteration (64 rotations of the j sums through DPP or
+// ds_bpermute, 1-2 LDS reads an iteration) bound the force pass by LDS: 40 of
+// its 40 cycles per CU and iteration. A patch takes 26 (Born, average of its
+// classes), 48 (force) and 37 (chain) VALU instructions, where an iteration
+// took 40 to 50. 256 systems of 300 to 5,000 atoms, us a pass (Born, force,
+// chain): 376, 609, 486 then, 322, 624, 457 now; one system of 2,500 atoms: 23.3,
+// 23.2, 32.7 then, 14.1, 11.8, 15.3 now.
 #pragma once
 
 #include "prx_common.h"
 #include "prx_obc_farfield.h"
 
 namespace prx {
-
-// DPP wave_rol:1 (lane l reads lane l + 1 mod 64). After k rotations lane l
-// holds the value that started in lane (l + k) & 63.
-#define PRX_DPP_WAVE_ROL1 0x134
-
-// BPERM moves the value through the LDS crossbar (ds_bpermute_b32: lane l
-// reads lane (l + 1) & 63), which takes no VALU issue slot; otherwise the DPP
-// wave rotate. Chosen per pass (PRX_ROT_BPERM_BORN / _FORCE / _CHAIN below).
-template <bool BPERM>
-__device__ __forceinline__ float rot(float x) {
-  if (BPERM) {
-    const int src = ((int)(threadIdx.x + 1) & 63) << 2;
-    return __int_as_float(__builtin_amdgcn_ds_bpermute(src, __float_as_int(x)));
-  }
-  // Every lane has a valid source under a full-wave rotate, so no "old" value is needed.
-  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(x), PRX_DPP_WAVE_ROL1, 0xF, 0xF, true));
-}
-
-// Chain partials carry three components: stored as three float arrays of 64
-// per (item, side), each written and read whole by a wave.
-__device__ __forceinline__ void put_part3(const DeviceView& v, int w, int side, int lane, float x, float y,
-                                          float z) {
-  float* pc = part3(v, w, side);
-  pc[lane] = x;
-  pc[kTile + lane] = y;
-  pc[2 * kTile + lane] = z;
-}
 
 __device__ __forceinline__ float frcp(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ float frsq(float x) { return __builtin_amdgcn_rsqf(x); }
@@ -51,85 +47,105 @@ __device__ __forceinline__ void wave_lds_sync() {
 // defaults below apply to anything it leaves unset.
 #include "prx_tuned.h"
 
-// How each pass rotates its j accumulators: 1 = LDS crossbar, 0 = DPP (rot);
-// the chain pass's three also split 1 + 2 (value 2) or 2 + 1 (value 3).
-#ifndef PRX_ROT_BPERM_BORN
-#define PRX_ROT_BPERM_BORN 0
+// Unroll depth of the row loop (over b) of the three pair passes.
+#ifndef PRX_UNROLL_BORN
+#define PRX_UNROLL_BORN 1
 #endif
-#ifndef PRX_ROT_BPERM_FORCE
-#define PRX_ROT_BPERM_FORCE 0
+#ifndef PRX_UNROLL_FORCE
+#define PRX_UNROLL_FORCE 1
 #endif
-#ifndef PRX_ROT_BPERM_CHAIN
-#define PRX_ROT_BPERM_CHAIN 0
+#ifndef PRX_UNROLL_CHAIN
+#define PRX_UNROLL_CHAIN 1
 #endif
-
-// Work items (waves) per workgroup of the pair kernels.
-#ifndef PRX_PAIR_WAVES
-#define PRX_PAIR_WAVES 4
+// XCD-aware unit order (unit_id below).
+#ifndef PRX_XCD_MAP
+#define PRX_XCD_MAP 1
 #endif
-constexpr int kWavesPerBlock = PRX_PAIR_WAVES;
-
-// Minimum waves per SIMD the compiler must fit the force and chain kernels'
-// registers to (0: no constraint; their unrolled loops otherwise take what
-// they need and run at lower occupancy).
+// Minimum waves per SIMD the compiler must fit the pair kernels' registers to
+// (0: no constraint).
 #ifndef PRX_MIN_WAVES
 #define PRX_MIN_WAVES 0
 #endif
 #if PRX_MIN_WAVES > 0
 #define PRX_OCCUPANCY __attribute__((amdgpu_waves_per_eu(PRX_MIN_WAVES)))
+#define PRX_FORCE_OCCUPANCY(ENERGY) PRX_OCCUPANCY
 #else
 #define PRX_OCCUPANCY
-#endif
-constexpr int kPairThreads = 64 * kWavesPerBlock;
-static_assert(kWavesPerBlock >= 1 && kWavesPerBlock <= 8, "PRX_PAIR_WAVES out of range");
-
-// LDS j accumulators are read and written through volatile pointers: the
-// compiler keeps those accesses in program order (the next iteration's read of
-// an entry another lane just wrote stays behind that write) while the
-// read-only j data loads remain free to move.
-typedef float v4f __attribute__((ext_vector_type(4)));
-
-// Build-time tuning knobs (defaults are the measured best on MI355X):
-// unroll depth of the three pair loops, and where the j-side accumulators
-// live: 0 = registers rotated by DPP; 1 = LDS, stored twice over like the j
-// data: lane l adds iteration k's term to entry l + k (an immediate offset;
-// no two lanes share an entry in one iteration, and a wave's LDS operations
-// complete in issue order, so the read-add-write needs only a compiler
-// ordering), and atom j's sum is entry j plus entry j + 64.
-#ifndef PRX_UNROLL_BORN
-#define PRX_UNROLL_BORN 8
-#endif
-#ifndef PRX_UNROLL_FORCE
-#define PRX_UNROLL_FORCE 4
-#endif
-#ifndef PRX_UNROLL_CHAIN
-#define PRX_UNROLL_CHAIN 8
-#endif
-#ifndef PRX_LDS_ACC
-#define PRX_LDS_ACC 0
+// The force pass takes 96 VGPRs, 128 with energies, without a spill (its free
+// choice is 144: 64 systems of up to 5,000 atoms 526 us an evaluation, 519 with 128).
+#define PRX_FORCE_OCCUPANCY(ENERGY) __attribute__((amdgpu_waves_per_eu(ENERGY ? 4 : 5)))
 #endif
 #define PRX_PRAGMA(x) _Pragma(#x)
 #define PRX_UNROLL(n) PRX_PRAGMA(unroll n)
 
-// Work item of this wave. Workgroups are dispatched to the 8 XCDs round-robin
-// (block b to XCD b mod 8), and each XCD has its own L2. With PRX_XCD_MAP the
-// blocks are renumbered so that XCD x runs one contiguous run of items
-// (consecutive items share their i tile and neighbouring j tiles, which then
-// hit in that XCD's L2): block b = 8k + x becomes x * per + min(x, rem) + k,
-// a bijection on [0, n_blocks) with per = n_blocks / 8, rem = n_blocks % 8.
-#ifndef PRX_XCD_MAP
-#define PRX_XCD_MAP 1
-#endif
-constexpr int kXcds = 8;
+constexpr int kEdge = 8;  // edge of a patch
 
-__device__ __forceinline__ int wave_id() {
-  int b = (int)blockIdx.x;
-#if PRX_XCD_MAP
-  const int nb = (int)gridDim.x, per = nb / kXcds, rem = nb % kXcds;
-  const int x = b % kXcds, k = b / kXcds;
-  b = x * per + min(x, rem) + k;
-#endif
-  return __builtin_amdgcn_readfirstlane((int)(b * (blockDim.x >> 6) + (threadIdx.x >> 6)));
+// Index x, hidden from the optimiser and ready only once y is: the columns are
+// read from LDS at such an index, so that column a is read while column a - 1
+// is evaluated. Left alone, the compiler reads all eight ahead of the row loop
+// and keeps them, 8 x 8 to 12 registers that cost half the waves.
+__device__ __forceinline__ int after(int x, float y) {
+  asm volatile("" : "+v"(x) : "v"(y));
+  return x;
+}
+
+// Position of the lanes past the end of a ragged tile: so far away that every
+// pair term underflows to zero or is multiplied by a zero parameter, and
+// different for every lane, so that no such pair has r = 0.
+__device__ __forceinline__ float4 pad_pos(int lane) { return make_float4(1e15f + 1e13f * (float)lane, 0.f, 0.f, 0.f); }
+
+// ---------------------------------------------------------------------------
+// Cross-lane sums
+// ---------------------------------------------------------------------------
+template <int CTRL>
+__device__ __forceinline__ float dpp(float x) {
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
+}
+constexpr int kDppHalfMirror = 0x141;  // lane p of 8 reads lane 7 - p
+constexpr int kDppXor2 = 0x4E;         // quad_perm [2, 3, 0, 1]
+constexpr int kDppXor1 = 0xB1;         // quad_perm [1, 0, 3, 2]
+constexpr int kDppRor8 = 0x128;        // lane l of 16 reads lane l + 8 mod 16
+
+// Sum over the eight lanes p; every lane gets it.
+__device__ __forceinline__ float sum_p(float x) {
+  x += dpp<kDppHalfMirror>(x);
+  x += dpp<kDppXor2>(x);
+  x += dpp<kDppXor1>(x);
+  return x;
+}
+
+// Sums over the eight lanes p of four values at once: lane p gets the
+// sum of value comp_p(p). Each exchange halves the values a lane still
+// carries: 4 DPP adds and 6 selects where four sums one by one take 12 DPP adds.
+__device__ __forceinline__ int comp_p(int p) { return (p & 2) + ((p >> 2) & 1); }
+__device__ __forceinline__ float sum_p4(float c0, float c1, float c2, float c3, int p) {
+  const bool hi = (p & 4) != 0, mid = (p & 2) != 0;
+  const float r0 = (hi ? c1 : c0) + dpp<kDppHalfMirror>(hi ? c0 : c1);
+  const float r1 = (hi ? c3 : c2) + dpp<kDppHalfMirror>(hi ? c2 : c3);
+  const float r = (mid ? r1 : r0) + dpp<kDppXor2>(mid ? r0 : r1);
+  return r + dpp<kDppXor1>(r);
+}
+// x and y with their halves (of 64 lanes) or rows of 16 exchanged:
+// swap32: (x.lo, y.lo), (x.hi, y.hi); swap16: the same within each half.
+__device__ __forceinline__ float add_swap32(float x, float y) {
+  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float add_swap16(float x, float y) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+// Sums over the eight lane groups q of the eight columns v[a] of lane p: lane
+// 8 q + p gets the sum of column a = q, which is atom (lane) of the tile.
+__device__ __forceinline__ float sum_q(const float (&v)[kEdge], int lane) {
+  float h[4], g[2];
+#pragma unroll
+  for (int a = 0; a < 4; ++a) h[a] = add_swap32(v[a], v[a + 4]);
+#pragma unroll
+  for (int a = 0; a < 2; ++a) g[a] = add_swap16(h[a], h[a + 2]);
+  const bool odd = (lane & 8) != 0;
+  return (odd ? g[1] : g[0]) + dpp<kDppRor8>(odd ? g[0] : g[1]);
 }
 
 // The j atoms of an item: a tile (gj = j0 + lane), or for a chunk item of a
@@ -148,8 +164,7 @@ __device__ __forceinline__ JSrc j_source(const DeviceView& v, const PairItem& it
     return j;
   }
   const int e0 = -1 - it.j0;
-  const int tI = it.excl;
-  j.nj = max(0, min(kTile, v.nl_count[tI] - (e0 - v.nl_row[tI].y)));
+  j.nj = max(0, min(kTile, v.nl_count[it.ti] - (e0 - v.nl_row[it.ti].y)));
   j.gj = j.nj > 0 ? v.nl_entries[e0 + min(lane, j.nj - 1)] : 0;
   return j;
 }
@@ -223,158 +238,351 @@ __device__ __forceinline__ bool obc_far(float r, float rho, float s) {
   return (r - s > rho) && (s <= PRX_OBC_FAR_XMAX * r);
 }
 
-// Written with u = 1/r^2 and the per-atom constants s^2 and s^3/2 (born4.z, .w):
-//   I = (s^3/2) u^2 h(s^2 u),   dI/dr = -2 (s^3/2) u^2 r^-1 k(s^2 u),
-// so each direction costs one product for the argument, the Horner chain and
-// two products; u^2 and u^2/r are shared by both directions of a pair.
-// F4: the degree-4 fits on y <= 1/16 (s <= r/4), for items whose every pair
-// is that far apart (kClsObcFar4); else the fits on y <= 1/4.
-template <bool F4 = false>
-__device__ __forceinline__ float obc_far_I(float s2, float s3h, float u, float u2) {
-  const float y = s2 * u;
-  float h;
-  if (F4) {
-    h = kObcH4[kObcH4Deg];
-#pragma unroll
-    for (int k = kObcH4Deg - 1; k >= 0; --k) h = fmaf(h, y, kObcH4[k]);
-  } else {
-    h = kObcH[kObcHDeg];
-#pragma unroll
-    for (int k = kObcHDeg - 1; k >= 0; --k) h = fmaf(h, y, kObcH[k]);
+// How the Born and chain passes treat an item: every pair tested (kMixed), or
+// every pair known to be in the far field (kFar) and at least 4, 6.5 or 14.5 s
+// apart (kFar4, kFar3, kFar2: the polynomial's degree).
+enum { kMixed = 0, kFar = 1, kFar4 = 2, kFar3 = 3, kFar2 = 4 };
+
+// With u = 1/r^2 the far field is a polynomial in u whose coefficients belong
+// to the descreening atom alone,
+//   I = u^2 sum_k w_k u^k,           w_k = (s^3/3) s^(2k) h_k / h_0,
+//   dI/dr = u^2 r^-1 sum_k w_k u^k,  w_k = -4 (s^3/3) s^(2k) k_k / k_0
+// (h_0 = 2/3, k_0 = 4/3: the leading coefficient, all that counts far away, is s^3/3 of
+// the atom's data, rounded once),
+// so they are formed once per atom and item, and a direction of a pair costs
+// one Horner chain in u and one fused multiply-add into its sum (against
+// y = s^2 u, the chain in y, two products and an add: 5 against 8 operations
+// a direction for the degree-4 fits).
+template <int CLS>
+struct BornW {
+  static constexpr int N = (CLS == kFar2 ? kObcH2Deg : CLS == kFar3 ? kObcH3Deg : CLS == kFar4 ? kObcH4Deg : kObcHDeg) + 1;
+  __device__ static constexpr float c(int k) {
+    return k == 0 ? 1.0f : 1.5f * (CLS == kFar2 ? kObcH2[k] : CLS == kFar3 ? kObcH3[k] : CLS == kFar4 ? kObcH4[k] : kObcH[k]);
   }
-  return (s3h * u2) * h;
-}
-
-// -2 k(y): the factor -2 scales every coefficient exactly, so this is -2 times
-// the Horner value of k bit for bit.
-template <bool F4 = false>
-__device__ __forceinline__ float obc_far_km2(float y) {
-  float q;
-  if (F4) {
-    q = -2.0f * kObcK4[kObcK4Deg];
-#pragma unroll
-    for (int k = kObcK4Deg - 1; k >= 0; --k) q = fmaf(q, y, -2.0f * kObcK4[k]);
-  } else {
-    q = -2.0f * kObcK[kObcKDeg];
-#pragma unroll
-    for (int k = kObcKDeg - 1; k >= 0; --k) q = fmaf(q, y, -2.0f * kObcK[k]);
+};
+template <int CLS>
+struct ChainW {
+  static constexpr int N = (CLS == kFar2 ? kObcK2Deg : CLS == kFar3 ? kObcK3Deg : CLS == kFar4 ? kObcK4Deg : kObcKDeg) + 1;
+  __device__ static constexpr float c(int k) {
+    return k == 0 ? -4.0f : -3.0f * (CLS == kFar2 ? kObcK2[k] : CLS == kFar3 ? kObcK3[k] : CLS == kFar4 ? kObcK4[k] : kObcK[k]);
   }
-  return q;
+};
+
+// w[k] of one atom.
+template <class W>
+__device__ __forceinline__ void obc_weights(float s2, float s33, float (&w)[W::N]) {
+  float m = s33;
+#pragma unroll
+  for (int k = 0; k < W::N; ++k) {
+    w[k] = m * W::c(k);
+    m *= s2;
+  }
 }
 
-__device__ __forceinline__ float obc_far_dI(float s2, float s3h, float u, float u2r) {
-  return (s3h * u2r) * obc_far_km2(s2 * u);
+// sum_k w_k u^k / s33 for an atom whose weights are not formed: y = s^2 u.
+template <class W>
+__device__ __forceinline__ float obc_poly(float y) {
+  float h = W::c(W::N - 1);
+#pragma unroll
+  for (int k = W::N - 2; k >= 0; --k) h = fmaf(h, y, W::c(k));
+  return h;
 }
 
-// Chain-rule scalar of a pair with both directions in the far field:
-//   (c_i dI(rho_i, s_j)/dr + c_j dI(rho_j, s_i)/dr) / r
-//     = -2 u^3 (c_i s_j^3/2 k(s_j^2 u) + c_j s_i^3/2 k(s_i^2 u)),   u = 1/r^2.
-template <bool F4 = false>
-__device__ __forceinline__ float chain_far(float u, float sj2, float ci_s3hj, float si2, float cj_s3hi) {
-  return (u * u * u) * fmaf(ci_s3hj, obc_far_km2<F4>(sj2 * u), cj_s3hi * obc_far_km2<F4>(si2 * u));
+template <int N>
+__device__ __forceinline__ float horner(const float (&w)[N], float u) {
+  float h = w[N - 1];
+#pragma unroll
+  for (int k = N - 2; k >= 0; --k) h = fmaf(h, u, w[k]);
+  return h;
 }
 
 // ---------------------------------------------------------------------------
 // Pass 1: Born sums
 // ---------------------------------------------------------------------------
 
-// LDS slice of one wave: j data staged twice (2 x 64 entries).
-struct BornLds {  // (x, y, z, s^2), (s^3/2, rho, s, 0); j accumulators
-  float4 a[128];
-  float4 b[128];
-#if PRX_LDS_ACC
-  float acc[128];
-#endif
+// One wave's LDS in float4: the rows (tile I) and columns (tile J) of its item,
+// two per atom, and a scratch list of 64 for the near pairs and the column sums
+// (force: with the energies). 5 KB let eight waves of a SIMD run.
+constexpr int kBornLds = 5 * kTile, kForceLds = 5 * kTile + 2, kChainLds = 5 * kTile;
+constexpr int kPairLds = kForceLds;  // of any pass
+typedef float4 Tile4[kTile];
+
+// An atom of the Born pass. Short: the tiers of at most five coefficients,
+// (x, y, z, w0), (w1, w2, w3, w4). The others keep (x, y, z, s^2), (s^3/3, rho,
+// s, -): a row's weights are formed once per row of patches, a column takes
+// obc_poly in y, two products more a pair than with weights but 16 bytes less
+// per atom and read.
+template <int CLS>
+struct BornAtom {
+  static constexpr int N = BornW<CLS>::N;
+  static constexpr bool kShort = N <= 5;
+  float x, y, z, s2, s33;
+  float w[N];  // row, or short
+
+  __device__ __forceinline__ static void stage(Tile4* t, int lane, const float4& p, const float4& b, float) {
+    if constexpr (kShort) {
+      float w[N];
+      obc_weights<BornW<CLS>>(b.z, b.w, w);
+      t[0][lane] = make_float4(p.x, p.y, p.z, w[0]);
+      t[1][lane] = make_float4(w[1], w[2], N > 3 ? w[3 % N] : 0.0f, N > 4 ? w[4 % N] : 0.0f);
+    } else {
+      t[0][lane] = make_float4(p.x, p.y, p.z, b.z);
+      t[1][lane] = make_float4(b.w, b.x, b.y, 0.0f);
+    }
+  }
+  // row: with its weights
+  __device__ __forceinline__ void read(const Tile4* t, int e, bool row) {
+    const float4 a = t[0][e];
+    x = a.x; y = a.y; z = a.z;
+    if constexpr (kShort) {
+      const float4 b = t[1][e];
+      w[0] = a.w; w[1] = b.x; w[2] = b.y;
+      if constexpr (N > 3) w[3] = b.z;
+      if constexpr (N > 4) w[4] = b.w;
+    } else {
+      s2 = a.w;
+      s33 = t[1][e].x;
+      if (row) obc_weights<BornW<CLS>>(s2, s33, w);
+    }
+  }
+  // sum_k w_k u^k
+  __device__ __forceinline__ float sum(float u, bool row) const {
+    if (kShort || row) return horner(w, u);
+    return s33 * obc_poly<BornW<CLS>>(s2 * u);
+  }
 };
 
-// FAR: every pair of the item is in the far field (no per-pair test); F4:
-// and at least 4 s apart (the degree-4 fits).
-template <bool GENERAL, bool DIAG, bool FAR, bool F4 = false>
-__device__ __forceinline__ void born_tile(const DeviceView& v, const PairItem& it, const JSrc& js, int lane, int w,
-                                          float cut2, BornLds& L) {
-  const int ni = item_ni(it.meta), nj = js.nj;
-  const int gi = it.i0 + min(lane, ni - 1);
-  const int gj = js.gj;
-  const float4 pi = v.pos[gi], bi = v.born4[gi];
-  {
-    const float4 pj = v.pos[gj], bj = v.born4[gj];
-    // the far-field loop reads only a and b.x
-    const float4 a = make_float4(pj.x, pj.y, pj.z, bj.z);
-    const float4 b = make_float4(bj.w, bj.x, bj.y, 0.0f);
-    L.a[lane] = a; L.a[lane + 64] = a;
-    L.b[lane] = b; L.b[lane + 64] = b;
-#if PRX_LDS_ACC
-    L.acc[lane] = 0.0f;
-    L.acc[lane + 64] = 0.0f;
-#endif
-  }
-  wave_lds_sync();
-  float accI = 0.0f, accJ = 0.0f;
-  const bool ivalid = lane < ni;
-  constexpr int kbeg = DIAG ? 1 : 0, kend = DIAG ? 32 : 63;
-  PRX_UNROLL(PRX_UNROLL_BORN)
-  for (int k = kbeg; k <= kend; ++k) {
-    const float4 ja = L.a[lane + k];
-    const float xj = ja.x, yj = ja.y, zj = ja.z, sj2 = ja.w, sj3h = L.b[lane + k].x;
-    const float dx = xj - pi.x, dy = yj - pi.y, dz = zj - pi.z;
-    const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-    BornPair bp;
-    if (FAR) {
-      const float u = frcp(r2), u2 = u * u;
-      bp.I1 = obc_far_I<F4>(sj2, sj3h, u, u2);
-      bp.I2 = obc_far_I<F4>(bi.z, bi.w, u, u2);
-    } else {
-      const float rinv = frsq(r2);
-      const float u = rinv * rinv, u2 = u * u;
-      const float rhoj = L.b[lane + k].y, sj = L.b[lane + k].z;
-      const float r = r2 * rinv;
-      const bool far1 = obc_far(r, bi.x, sj), far2 = obc_far(r, rhoj, bi.y);
-      if (__all(far1 && far2)) {
-        bp.I1 = obc_far_I(sj2, sj3h, u, u2);
-        bp.I2 = obc_far_I(bi.z, bi.w, u, u2);
-      } else {
-        bp = born_pair(r, rinv, bi.x, bi.y, bi.z, rhoj, sj, sj2);
-        bp.I1 = far1 ? obc_far_I(sj2, sj3h, u, u2) : bp.I1;
-        bp.I2 = far2 ? obc_far_I(bi.z, bi.w, u, u2) : bp.I2;
+// The largest float below x > 0: r^2 < x is r^2 <= prev_below(x).
+__device__ __forceinline__ float prev_below(float x) { return __int_as_float(__float_as_int(x) - 1); }
+
+// The near pairs of a mixed item: those within lim2, of the patches marked in
+// near (bit 8 b + a).
+//
+// Off the diagonal they are few (on proteins a tenth of the patches hold one,
+// and three lanes of 64 in those: 20 to 40 pairs an item). They are listed
+// first and then evaluated 64 at a time, a pair per lane, by eval(row, col),
+// which stores its terms in scratch[lane].xyz; then every lane adds, in list
+// order, the terms of its row 8 p + q and of its column (lane) by
+// take(terms, mine_r, mine_c), factors of 1 or 0.
+template <class Eval, class Take>
+__device__ __forceinline__ void near_list(const Tile4* ti, const Tile4* tj, unsigned long long near, int lane,
+                                          bool cut, float lim2, float4* scratch, Eval&& eval, Take&& take) {
+  const int p = lane & 7, q = lane >> 3, my_row = kEdge * p + q;
+  unsigned short* const list = reinterpret_cast<unsigned short*>(scratch);
+  int count = 0;
+  while (near != 0 || count > 0) {
+    while (near != 0 && count < 64) {
+      const int k = __builtin_ctzll(near), row = (k & 56) + q, col = kEdge * (k & 7) + p;
+      near &= near - 1;
+      const float4 a = ti[0][row], b = tj[0][col];
+      const float dx = b.x - a.x, dy = b.y - a.y, dz = b.z - a.z;
+      const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+      const bool on = cut ? r2 <= lim2 : !(r2 > lim2);
+      const unsigned long long m = __ballot(on);
+      const int at = count + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
+                                                            __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+      if (on) list[at] = (unsigned short)(row << 6 | col);
+      count += __popcll(m);
+    }
+    if (count == 0) break;
+    wave_lds_sync();
+    const int n = min(count, 64);
+    const int e = list[min(lane, n - 1)], rest = list[64 + lane];
+    wave_lds_sync();
+    eval(e >> 6, e & 63);  // writes scratch[lane].xyz
+    scratch[lane].w = __int_as_float(lane < n ? e : -1);
+    wave_lds_sync();
+    constexpr int kBatch = 4;  // entries read before any is added
+    for (int k = 0; k < n; k += kBatch) {
+      float4 c[kBatch];
+#pragma unroll
+      for (int m = 0; m < kBatch; ++m) c[m] = scratch[k + m];
+#pragma unroll
+      for (int m = 0; m < kBatch; ++m) {
+        const int ce = __float_as_int(c[m].w);
+        take(c[m], (ce >> 6) == my_row ? 1.0f : 0.0f, ce >= 0 && (ce & 63) == lane ? 1.0f : 0.0f);
       }
     }
-    if (GENERAL) {
-      const int orig = (lane + k) & 63;
-      bool valid = ivalid && orig < nj;
-      if (DIAG && k == 32) valid = valid && lane < 32;
-      if (cut2 > 0.0f) valid = valid && r2 < cut2;
-      bp.I1 = valid ? bp.I1 : 0.0f;
-      bp.I2 = valid ? bp.I2 : 0.0f;
-    }
-    accI += bp.I1;
-#if PRX_LDS_ACC
-    {
-      volatile float* acc = L.acc;
-      acc[lane + k] = acc[lane + k] + bp.I2;
-    }
-#else
-    accJ += bp.I2;
-    if (k != kend) accJ = rot<PRX_ROT_BPERM_BORN>(accJ);
-#endif
+    wave_lds_sync();
+    count -= n;
+    if (lane < count) list[lane] = (unsigned short)rest;
   }
-  part1(v, w, 0)[lane] = accI;
-#if PRX_LDS_ACC
-  wave_lds_sync();
-  part1(v, w, 1)[lane] = L.acc[lane] + L.acc[lane + 64];
-#else
-  const int home = (lane + kend) & 63;
-  part1(v, w, 1)[home] = accJ;
-#endif
+}
+
+// On the diagonal a fifth of the pairs are near (14 to 20 per atom): each lane
+// walks the near atoms of its own atom (lane), on both sides of the diagonal,
+// so nothing is summed across lanes; eval(atoms, on) adds to the lane's sums. Of a
+// unit's waves, sub = 0 .. nsub - 1, each takes the atoms 8 b + q' of its rows.
+template <class Eval>
+__device__ __forceinline__ void near_diag(const Tile4* t, int lane, int ni, int sub, int nsub, bool cut, float lim2,
+                                          Eval&& eval) {
+  const float4 me = t[0][lane];
+  unsigned long long near = 0;
+  for (int b = sub; kEdge * b < ni; b += nsub) {
+    unsigned bits = 0;
+#pragma unroll
+    for (int k = 0; k < kEdge; ++k) {
+      const float4 o = t[0][kEdge * b + k];
+      // the sign of the difference as in the pair loop: later atom minus earlier
+      const float dx = o.x - me.x, dy = o.y - me.y, dz = o.z - me.z;
+      const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+      const bool on = (cut ? r2 <= lim2 : !(r2 > lim2)) && kEdge * b + k != lane && kEdge * b + k < ni;
+      bits |= on ? 1u << k : 0u;
+    }
+    near |= (unsigned long long)bits << (kEdge * b);
+  }
+  if (lane >= ni) near = 0;
+  while (__any(near != 0)) {  // two atoms at a time: one is a chain of dependent steps
+    int o[2];
+    bool on[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      on[k] = near != 0;
+      o[k] = on[k] ? __builtin_ctzll(near) : lane;
+      near &= near - 1;
+    }
+    eval(o, on);
+  }
+}
+
+// I(r; rho_i, s_j) alone, for a near or a far pair.
+__device__ __forceinline__ float born_one(float r2, float rho_i, float s_j, float s2_j, float s33_j) {
+  const float rinv = frsq(r2), r = r2 * rinv, u = rinv * rinv;
+  const float U = r + s_j;
+  const float L = fmaxf(fmaxf(rho_i, fabsf(r - s_j)), 1e-4f), Uc = fmaxf(U, 1e-4f);
+  const float inv = frcp(L * Uc), iL = Uc * inv, iU = L * inv;
+  const float rs = fminf(rinv, 1e4f);
+  const float a = iL - iU, b = -a * (iL + iU), c = fmaf(-s2_j, rs, r);
+  const float I = fmaf(0.5f, a, fmaf(0.25f * kLn2 * flog2(L * iU), rs, 0.125f * c * b));
+  return obc_far(r, rho_i, s_j) ? (u * u) * (s33_j * obc_poly<BornW<kMixed>>(s2_j * u)) : (U > rho_i ? I : 0.0f);
+}
+
+__device__ __forceinline__ void born_near(float4* L, float4* scratch, unsigned long long near, int lane, int ni, bool diag, bool cut,
+                                          float lim2, int sub, int nsub, float& rows, float& cols) {
+  Tile4* ti = reinterpret_cast<Tile4*>(L);
+  Tile4* tj = ti + 2;
+  if (diag) {
+    const float4 me = ti[0][lane];
+    const float rhoi = ti[1][lane].y;
+    near_diag(ti, lane, ni, sub, nsub, cut, lim2, [&](const int (&o)[2], const bool (&on)[2]) {
+      float I[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const float4 a = ti[0][o[k]], b = ti[1][o[k]];
+        const float dx = a.x - me.x, dy = a.y - me.y, dz = a.z - me.z;
+        I[k] = born_one(fmaf(dx, dx, fmaf(dy, dy, dz * dz)), rhoi, b.z, a.w, b.x);
+      }
+#pragma unroll
+      for (int k = 0; k < 2; ++k) cols += on[k] ? I[k] : 0.0f;
+    });
+    return;
+  }
+  near_list(
+      ti, tj, near, lane, cut, lim2, scratch,
+      [&](int row, int col) {
+        const float4 ai = ti[0][row], bi = ti[1][row], aj = tj[0][col], bj = tj[1][col];
+        const float rhoi = bi.y, si = bi.z, rhoj = bj.y, sj = bj.z;
+        const float dx = aj.x - ai.x, dy = aj.y - ai.y, dz = aj.z - ai.z;
+        const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+        const float rinv = frsq(r2);
+        const float u = rinv * rinv, u2 = u * u, r = r2 * rinv;
+        const BornPair bp = born_pair(r, rinv, rhoi, si, ai.w, rhoj, sj, aj.w);
+        const float I1 = obc_far(r, rhoi, sj) ? u2 * (bj.x * obc_poly<BornW<kMixed>>(aj.w * u)) : bp.I1;
+        const float I2 = obc_far(r, rhoj, si) ? u2 * (bi.x * obc_poly<BornW<kMixed>>(ai.w * u)) : bp.I2;
+        *reinterpret_cast<float2*>(&scratch[lane]) = make_float2(I1, I2);
+      },
+      [&](const float4& c, float mr, float mc) {
+        rows = fmaf(mr, c.x, rows);
+        cols = fmaf(mc, c.y, cols);
+      });
+}
+
+// The atoms of an item's tiles (or of one of them), loaded together: lane = atom.
+struct ItemAtoms {
+  float4 pi, bi, pj, bj;
+  float ci, cj;
+};
+template <bool CHAIN>
+__device__ __forceinline__ ItemAtoms load_atoms(const DeviceView& v, const PairItem& it, const JSrc& js, int lane,
+                                                bool rows, bool cols) {
+  const int gi = it.i0 + min(lane, item_ni(it.meta) - 1), gj = js.gj;
+  ItemAtoms t;
+  t.ci = t.cj = 0.0f;
+  if (rows) {
+    t.pi = v.pos[gi]; t.bi = v.born4[gi];
+    if (CHAIN) t.ci = v.gb4[gi].w;
+  }
+  if (cols) {
+    t.pj = v.pos[gj]; t.bj = v.born4[gj];
+    if (CHAIN) t.cj = v.gb4[gj].w;
+  }
+  return t;
+}
+// Lanes past the end of a ragged tile: far away, and without any term.
+__device__ __forceinline__ void pad_atoms(ItemAtoms& t, int lane, int ni, int nj) {
+  const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (lane >= ni) { t.pi = pad_pos(lane); t.bi = zero; t.ci = 0.0f; }
+  if (lane >= nj) { t.pj = pad_pos(lane); t.bj = zero; t.cj = 0.0f; }
+}
+
+// The far pairs of rows b = sub, sub + nsub, ... of an item. rows: lane 8 q + p
+// gets the sum of row 8 p + q; cols: lane l that of column l over these rows.
+// CUT: pairs with r^2 >= cut2 add nothing. FULL: both tiles hold 64 atoms.
+// thr2: above it every pair of the item is in the far field; a mixed item
+// adds only the pairs above it here and marks the patches of the others in
+// near, so that the loop has no branch and the registers of the far field alone.
+template <int CLS, bool DIAG, bool CUT, bool FULL>
+__device__ __forceinline__ void born_tile(const float4* L, int ni, int nj, int lane, float cut2, float thr2, int sub,
+                                          int nsub, float& rows, float& cols, unsigned long long& near) {
+  const Tile4* ti = reinterpret_cast<const Tile4*>(L);
+  const Tile4* tj = ti + 2;
+  const int p = lane & 7, q = lane >> 3;
+  float accj[kEdge] = {};
+  const int nb = FULL ? kEdge : (ni + kEdge - 1) / kEdge, na = FULL ? kEdge : (nj + kEdge - 1) / kEdge;
+  PRX_UNROLL(PRX_UNROLL_BORN)
+  for (int b = sub; b < nb; b += nsub) {
+    BornAtom<CLS> i;
+    float acci = 0.0f;
+    i.read(ti, kEdge * b + q, true);
+    unsigned marks = 0;
+    int col = p;
+#pragma unroll
+    for (int a = 0; a < kEdge; ++a) {
+      if (!FULL && a >= na) break;
+      if (DIAG && a < b) continue;
+      BornAtom<CLS> j;
+      col = after(col, a < 2 ? acci : accj[a - 2]);
+      j.read(tj, col + kEdge * a, false);
+      const float dx = j.x - i.x, dy = j.y - i.y, dz = j.z - i.z;
+      float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+      if (DIAG && a == b) r2 = p > q ? r2 : 1e30f;  // each unordered pair once: no term at 1e15 A
+      bool on = true;
+      if (CUT) on = r2 < cut2;
+      if (CLS == kMixed) {
+        const bool close = !(r2 > thr2);
+        if (!DIAG) marks |= (__ballot(on && close) != 0 ? 1u : 0u) << a;
+        on = on && !close;
+      }
+      float u = frcp(r2);
+      if (CUT || CLS == kMixed) u = on ? u : 0.0f;
+      const float u2 = u * u;
+      acci = fmaf(u2, j.sum(u, false), acci);
+      accj[a] = fmaf(u2, i.sum(u, true), accj[a]);
+    }
+    const float r = sum_p(acci);
+    rows = p == b ? r : rows;
+    if (CLS == kMixed && !DIAG) near |= (unsigned long long)marks << (kEdge * b);
+  }
+  cols = sum_q(accj, lane);
 }
 
 // Class bits of an item from its tiles' bounding boxes (wave-uniform). The
-// OBC2 far-field bit needs the box distance above every pair's threshold,
+// far-field tier needs the box distance above every pair's threshold,
 // max(s_j + rho_i, s_i + rho_j, 2 s) over the two tiles, with a 1e-4
-// relative margin on the squared distance; the s <= r/4 bit also needs it
-// above 4 s.
-__device__ __forceinline__ int classify(const DeviceView& v, const SlotConst& S, const PairItem& it) {
-  const int tI = S.tile0 + ((it.i0 - S.a0) >> 6);
-  const int tJ = S.tile0 + ((it.j0 - S.a0) >> 6);
+// relative margin on the squared distance; the finer tiers also need it above
+// 4, 6.5 and 14.5 s.
+__device__ __forceinline__ int classify(const DeviceView& v, const SlotConst& S, const PairItem& it, float& thr2) {
+  const int tI = it.ti, tJ = it.tj;
   const float4 li = v.tbox[2 * tI], hi = v.tbox[2 * tI + 1];
   const float4 lj = v.tbox[2 * tJ], hj = v.tbox[2 * tJ + 1];
   const float gx = fmaxf(0.0f, fmaxf(lj.x - hi.x, li.x - hj.x));
@@ -386,9 +594,13 @@ __device__ __forceinline__ int classify(const DeviceView& v, const SlotConst& S,
   const float dmin2 = gx * gx + gy * gy + gz * gz;
   const float dmax2 = ex * ex + ey * ey + ez * ez;
   const float thr = fmaxf(fmaxf(hj.w + li.w, hi.w + lj.w), fmaxf(hi.w, hj.w) * (1.0f / PRX_OBC_FAR_XMAX));
-  int cls = (tI != tJ && dmin2 > thr * thr * 1.0001f) ? kClsObcFar : 0;
-  const float thr4 = fmaxf(hi.w, hj.w) * (1.0f / PRX_OBC_FAR4_XMAX);
-  if (cls && dmin2 > thr4 * thr4 * 1.0001f) cls |= kClsObcFar4;
+  thr2 = thr * thr * 1.0001f;
+  const float smax = fmaxf(hi.w, hj.w), d2 = dmin2 * (1.0f / 1.0001f);
+  const float t4 = smax * (1.0f / PRX_OBC_FAR4_XMAX), t3 = smax * (1.0f / PRX_OBC_FAR3_XMAX);
+  const float t2 = smax * (1.0f / PRX_OBC_FAR2_XMAX);
+  int tier = kMixed;
+  if (tI != tJ && dmin2 > thr2) tier = d2 > t2 * t2 ? kFar2 : d2 > t3 * t3 ? kFar3 : d2 > t4 * t4 ? kFar4 : kFar;
+  int cls = tier << kClsTierShift;
   if (S.cutoff2 > 0.0f) {
     if (dmin2 >= S.cutoff2 * 1.00001f)
       cls |= kClsFar;
@@ -401,8 +613,8 @@ __device__ __forceinline__ int classify(const DeviceView& v, const SlotConst& S,
 // Class of a chunk item: every listed pair may straddle the cutoff; the OBC2
 // far-field bit comes from the i tile's box and the box of the chunk's j
 // atoms (a wave reduction over the lanes' atoms), as for a tile pair.
-__device__ __forceinline__ int classify_chunk(const DeviceView& v, const PairItem& it, const JSrc& js, int lane) {
-  const float4 p = v.pos[js.gj], b = v.born4[js.gj];
+__device__ __forceinline__ int classify_chunk(const DeviceView& v, const PairItem& it, const float4& p,
+                                              const float4& b, float& thr2) {
   float lx = p.x, ly = p.y, lz = p.z, hx = p.x, hy = p.y, hz = p.z, mr = b.x, ms = b.y;
   for (int off = 32; off > 0; off >>= 1) {
     lx = fminf(lx, __shfl_xor(lx, off));
@@ -414,14 +626,16 @@ __device__ __forceinline__ int classify_chunk(const DeviceView& v, const PairIte
     mr = fmaxf(mr, __shfl_xor(mr, off));
     ms = fmaxf(ms, __shfl_xor(ms, off));
   }
-  const int tI = it.excl;
-  const float4 li = v.tbox[2 * tI], hi = v.tbox[2 * tI + 1];
+  const float4 li = v.tbox[2 * it.ti], hi = v.tbox[2 * it.ti + 1];
   const float gx = fmaxf(0.0f, fmaxf(lx - hi.x, li.x - hx));
   const float gy = fmaxf(0.0f, fmaxf(ly - hi.y, li.y - hy));
   const float gz = fmaxf(0.0f, fmaxf(lz - hi.z, li.z - hz));
   const float dmin2 = gx * gx + gy * gy + gz * gz;
   const float thr = fmaxf(fmaxf(ms + li.w, hi.w + mr), fmaxf(hi.w, ms) * (1.0f / PRX_OBC_FAR_XMAX));
-  return kClsStraddle | (dmin2 > thr * thr * 1.0001f ? kClsObcFar : 0);
+  thr2 = thr * thr * 1.0001f;
+  const float t4 = fmaxf(hi.w, ms) * (1.0f / PRX_OBC_FAR4_XMAX);
+  const int tier = !(dmin2 > thr2) ? kMixed : (dmin2 * (1.0f / 1.0001f) > t4 * t4 ? kFar4 : kFar);
+  return kClsStraddle | (tier << kClsTierShift);
 }
 
 // A system at its step limit, in a step graph (DeviceView::skip_done).
@@ -429,377 +643,725 @@ __device__ __forceinline__ bool skip_item(const DeviceView& v, const SlotConst& 
   return v.skip_done && S.step_limit != 0u && slot_done(S, v.atom_step[it.i0]);
 }
 
-// The Born pass of work item w, by one wave.
-__device__ __forceinline__ void born_item(const DeviceView& v, int w, BornLds& L) {
-  const PairItem it = v.items[w];
-  const int lane = threadIdx.x & 63;
-  const int fl = item_flags(it.meta);
-  const SlotConst& S = v.slots[item_slot(it.meta)];
-  if (skip_item(v, S, it)) return;
-  const JSrc js = j_source(v, it, lane);
-  if (item_is_chunk(it)) {  // neighbour-list chunk: always the masked path with the cutoff test
-    if (js.nj == 0) {
-      if (lane == 0) v.item_cls[w] = kClsFar;
-      return;
-    }
-    const int cls = classify_chunk(v, it, js, lane);
-    if (lane == 0) v.item_cls[w] = cls;
-    if (cls & kClsObcFar)
-      born_tile<true, false, true>(v, it, js, lane, w, S.cutoff2, L);
+// item_cls holds an item's class (low bits) and, in the others, the Born
+// pass's far-field threshold thr^2 as a float rounded up: a pair with r^2 above
+// it is in the far field in both directions.
+__device__ __forceinline__ int pack_cls(int cls, float thr2) {
+  return ((__float_as_int(thr2) + kClsMask) & ~kClsMask) | cls;
+}
+__device__ __forceinline__ float cls_thr2(int packed) { return __int_as_float(packed & ~kClsMask); }
+
+// Runs f.run<CLS, DIAG, CUT, FULL>() for an item of class tier. Ragged and
+// cut items take the degree-4 polynomials at best: they are few, and every
+// variant costs instruction cache.
+template <class F>
+__device__ __forceinline__ void by_class(int tier, bool diag, bool cut, bool full, F&& f) {
+  if (diag) {
+    if (cut)
+      f.template run<kMixed, true, true, false>();
     else
-      born_tile<true, false, false>(v, it, js, lane, w, S.cutoff2, L);
-    return;
-  }
-  const bool full = item_ni(it.meta) == kTile && js.nj == kTile;
-  const int cls = classify(v, S, it);
-  if (lane == 0) v.item_cls[w] = cls;
-  const int ccut = cls & kClsCutMask;
-  if (S.gb_cut && ccut == kClsFar) return;  // no partials: the gathers skip this item
-  const float cut2 = (S.gb_cut && ccut == kClsStraddle) ? S.cutoff2 : 0.0f;
-  if (fl & kFlagDiag) {
-    born_tile<true, true, false>(v, it, js, lane, w, cut2, L);
-  } else if (cls & kClsObcFar4) {
-    if (full && cut2 == 0.0f)
-      born_tile<false, false, true, true>(v, it, js, lane, w, 0.0f, L);
+      f.template run<kMixed, true, false, false>();
+  } else if (cut) {
+    if (tier >= kFar4)
+      f.template run<kFar4, false, true, false>();
+    else if (tier == kFar)
+      f.template run<kFar, false, true, false>();
     else
-      born_tile<true, false, true, true>(v, it, js, lane, w, cut2, L);
-  } else if (cls & kClsObcFar) {
-    if (full && cut2 == 0.0f)
-      born_tile<false, false, true>(v, it, js, lane, w, 0.0f, L);
+      f.template run<kMixed, false, true, false>();
+  } else if (!full) {
+    if (tier >= kFar4)
+      f.template run<kFar4, false, false, false>();
+    else if (tier == kFar)
+      f.template run<kFar, false, false, false>();
     else
-      born_tile<true, false, true>(v, it, js, lane, w, cut2, L);
-  } else if (full && cut2 == 0.0f) {
-    born_tile<false, false, false>(v, it, js, lane, w, 0.0f, L);
+      f.template run<kMixed, false, false, false>();
   } else {
-    born_tile<true, false, false>(v, it, js, lane, w, cut2, L);
+    if (tier == kFar2)
+      f.template run<kFar2, false, false, true>();
+    else if (tier == kFar3)
+      f.template run<kFar3, false, false, true>();
+    else if (tier == kFar4)
+      f.template run<kFar4, false, false, true>();
+    else if (tier == kFar)
+      f.template run<kFar, false, false, true>();
+    else
+      f.template run<kMixed, false, false, true>();
   }
 }
+
+// An item's rows and/or columns into LDS in the form of its class (template
+// ATOM); done with before the pairs, so that the loaded atoms hold no registers
+// there.
+template <template <int> class ATOM>
+struct StageRun {
+  const ItemAtoms& t;
+  int lane;
+  bool rows, cols;
+  float4* L;
+  template <int CLS, bool DIAG, bool CUT, bool FULL>
+  __device__ __forceinline__ void run() {
+    Tile4* ti = reinterpret_cast<Tile4*>(L);
+    if (rows) ATOM<CLS>::stage(ti, lane, t.pi, t.bi, t.ci);
+    if (cols) ATOM<CLS>::stage(ti + 2, lane, t.pj, t.bj, t.cj);
+  }
+};
+
+struct BornRun {
+  const float4* L;
+  int ni, nj, lane;
+  float cut2, thr2;
+  int sub, nsub;
+  float rows, cols;
+  unsigned long long near;
+  template <int CLS, bool DIAG, bool CUT, bool FULL>
+  __device__ __forceinline__ void run() {
+    born_tile<CLS, DIAG, CUT, FULL>(L, ni, nj, lane, cut2, thr2, sub, nsub, rows, cols, near);
+  }
+};
+
+// Column sums of a share of a Born item (lane = column), added share by share.
+struct BornSum {
+  float c = 0.0f;
+  __device__ __forceinline__ void add(const BornSum& o) { c += o.c; }
+  __device__ __forceinline__ void store(const DeviceView& v, int w, int lane) const { part1(v, w, 1)[lane] = c; }
+  __device__ __forceinline__ void to_lds(float4* at, int lane) const { reinterpret_cast<float*>(at)[lane] = c; }
+  __device__ __forceinline__ void from_lds(const float4* at, int lane) { c = reinterpret_cast<const float*>(at)[lane]; }
+};
+
+// The Born pass over one item. stage() prepares it (rows and/or cols: which of
+// its tiles this wave brings into LDS at L); false: the item has no work, and no
+// partials. run() evaluates share sub of its rows: stores their sums and
+// returns the columns'. scratch: 64 float4 of this wave's own.
+struct BornPass {
+  typedef BornSum Sum;
+  static constexpr int kLds = kBornLds;
+  int w, lane, ni, nj, tier, nsub;
+  float cut2, thr2, lim2;
+  bool diag, full, cut;
+
+  __device__ __forceinline__ bool stage(const DeviceView& v, int w_, const PairItem& it, bool rows, bool cols,
+                                        float4* L) {
+    w = w_;
+    lane = threadIdx.x & 63;
+    const SlotConst& S = v.slots[item_slot(it.meta)];
+    if (skip_item(v, S, it)) return false;
+    const bool chunk = item_is_chunk(it);
+    const JSrc js = j_source(v, it, lane);
+    ItemAtoms t = load_atoms<false>(v, it, js, lane, rows, cols || chunk);
+    diag = (item_flags(it.meta) & kFlagDiag) != 0;
+    ni = item_ni(it.meta);
+    nj = js.nj;
+    full = ni == kTile && nj == kTile;
+    nsub = it.nsub;
+    thr2 = 0.0f;
+    int cls;
+    if (chunk) {  // neighbour-list chunk: always with the cutoff test
+      if (nj == 0) {
+        if (lane == 0 && rows) v.item_cls[w] = kClsFar;
+        return false;
+      }
+      cls = classify_chunk(v, it, t.pj, t.bj, thr2);
+    } else {
+      cls = classify(v, S, it, thr2);
+    }
+    if (lane == 0 && rows) v.item_cls[w] = pack_cls(cls, thr2);
+    const int ccut = cls & kClsCutMask;
+    if (S.gb_cut && ccut == kClsFar) return false;  // no partials: the gathers skip this item
+    cut = S.gb_cut && ccut == kClsStraddle;
+    cut2 = S.cutoff2;
+    lim2 = cut ? fminf(thr2, prev_below(cut2)) : thr2;
+    tier = cls >> kClsTierShift;
+    if (!full) pad_atoms(t, lane, ni, nj);
+    StageRun<BornAtom> put{t, lane, rows, cols, L};
+    by_class(tier, diag, cut, full, put);
+    return true;
+  }
+
+  __device__ __forceinline__ BornSum run(const DeviceView& v, int sub, float4* L,
+                                         float4* scratch) const {
+    const int p = lane & 7, q = lane >> 3;
+    BornRun f{L, ni, nj, lane, cut2, thr2, sub, nsub, 0.0f, 0.0f, 0};
+    by_class(tier, diag, cut, full, f);
+    if (f.near != 0 || diag) born_near(L, scratch, f.near, lane, ni, diag, cut, lim2, sub, nsub, f.rows, f.cols);
+    if ((p & (nsub - 1)) == sub) part1(v, w, 0)[kEdge * p + q] = f.rows;
+    BornSum s;
+    s.c = f.cols;
+    return s;
+  }
+};
 
 // ---------------------------------------------------------------------------
 // Pass 2: GB + Coulomb + LJ
 // ---------------------------------------------------------------------------
 
-// LJC = false: GB only (items entirely beyond the LJ/Coulomb cutoff).
-// GENERAL tiles test r^2 < cut2 per pair when cut2 > 0, on LJ/Coulomb and, if
-// gb_cut, on GB too.
-struct PairLds {  // two float4 of j data per entry; j accumulators
-  float4 a[128];
-  float4 b[128];
-#if PRX_LDS_ACC
-  float4 acc[128];
-#endif
+// Column sums of a share: force, sum of g B_i of lane's atom; e: an energy
+// summed over the wave, GB in lanes 0-15, Coulomb in 32-47, LJ in the others
+// (sum_energies).
+template <bool ENERGY>
+struct ForceSum {
+  float x = 0.0f, y = 0.0f, z = 0.0f, g = 0.0f;
+  double e = 0.0;
+  __device__ __forceinline__ void add(const ForceSum& o) {
+    x += o.x; y += o.y; z += o.z; g += o.g;
+    if (ENERGY) e += o.e;
+  }
+  __device__ __forceinline__ void store(const DeviceView& v, int w, int lane) const {
+    part4(v, w, 1)[lane] = make_float4(x, y, z, g);
+    if (ENERGY && lane < 48 && (lane & 15) == 0) v.e_items[(size_t)w * 3 + (lane == 0 ? 0 : (lane == 32 ? 1 : 2))] = e;
+  }
+  __device__ __forceinline__ void to_lds(float4* at, int lane) const {
+    at[lane] = make_float4(x, y, z, g);
+    if (ENERGY && (lane & 15) == 0) reinterpret_cast<double*>(at + kTile)[lane >> 4] = e;
+  }
+  __device__ __forceinline__ void from_lds(const float4* at, int lane) {
+    const float4 f = at[lane];
+    x = f.x; y = f.y; z = f.z; g = f.w;
+    if (ENERGY) e = reinterpret_cast<const double*>(at + kTile)[lane >> 4];
+  }
 };
 
-template <bool GENERAL, bool DIAG, bool ENERGY, bool LJC>
-__device__ __forceinline__ void force_tile(const DeviceView& v, const PairItem& it, const JSrc& js, int lane, int w,
-                                           float cut2, bool gb_cut, PairLds& L) {
-  const int ni = item_ni(it.meta), nj = js.nj;
-  const SlotConst& S = v.slots[item_slot(it.meta)];
-  const float kc = S.k_coulomb, gb2 = S.gb2;
-  const bool has_cut = GENERAL && cut2 > 0.0f;
-  const bool gb_has_cut = has_cut && gb_cut;
-  const bool has_excl = GENERAL && LJC && !item_is_chunk(it) && it.excl >= 0;  // a chunk's excl is its row tile
-  const int gi = it.i0 + min(lane, ni - 1);
-  const int gj = js.gj;
-  const float4 pi = v.pos[gi], nbi = v.nb4[gi], gbi = v.gb4[gi];
-  const float q_kc = kc * nbi.x, q_gb = gb2 * nbi.x;
-  {
-    const float4 pj = v.pos[gj], nbj = v.nb4[gj], gbj = v.gb4[gj];
-    const float4 a = make_float4(pj.x, pj.y, pj.z, nbj.x);    // x, y, z, q
-    const float4 b = make_float4(nbj.y, nbj.z, gbj.x, gbj.y);  // sigma/2, sqrt(eps), B, a
-    L.a[lane] = a; L.a[lane + 64] = a;
-    L.b[lane] = b; L.b[lane + 64] = b;
-#if PRX_LDS_ACC
-    L.acc[lane] = make_float4(0.f, 0.f, 0.f, 0.f);
-    L.acc[lane + 64] = make_float4(0.f, 0.f, 0.f, 0.f);
-#endif
-  }
-  wave_lds_sync();
-  float fxi = 0.f, fyi = 0.f, fzi = 0.f, dbi = 0.f;
-  float fxj = 0.f, fyj = 0.f, fzj = 0.f, dbj = 0.f;
-  double egb = 0.0, ecl = 0.0, elj = 0.0;
-  unsigned long long m0 = 0, m1 = 0;
-  if (has_excl) {
-    m0 = v.excl_masks[(size_t)it.excl * 128 + lane * 2];
-    m1 = v.excl_masks[(size_t)it.excl * 128 + lane * 2 + 1];
-  }
-  const bool ivalid = lane < ni;
-  constexpr int kbeg = DIAG ? 1 : 0, kend = DIAG ? 32 : 63;
-  PRX_UNROLL(PRX_UNROLL_FORCE)
-  for (int k = kbeg; k <= kend; ++k) {
-    const float4 ja = L.a[lane + k];
-    const float4 jb = L.b[lane + k];
-    const float xj = ja.x, yj = ja.y, zj = ja.z, qj = ja.w, hsj = jb.x, sej = jb.y, Bj = jb.z, aj = jb.w;
-    const float dx = xj - pi.x, dy = yj - pi.y, dz = zj - pi.z;
-    const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-    const float rinv = frsq(r2);
-    const float rinv2 = rinv * rinv;
-    // Coulomb + LJ (q_kc = k_coulomb q_i, q_gb = gb2 q_i are per-lane constants)
-    float ec = 0.0f, el = 0.0f, fl = 0.0f;
-    if (LJC) {
-      ec = (q_kc * qj) * rinv;
-      const float sg = nbi.y + hsj;
-      const float ep = nbi.z * sej;
-      const float s2 = sg * sg * rinv2;
-      const float s6 = s2 * s2 * s2;
-      el = 4.0f * ep * (s6 * s6 - s6);
-      fl = ep * s6 * fmaf(48.0f, s6, -24.0f);
-    }
-    // GB over every pair
-    const float BB = gbi.x * Bj;
-    const float x = r2 * (gbi.y * aj);  // r^2 log2(e) / (4 B_i B_j)
-    const float ex = fexp2(-x);
-    const float f2 = fmaf(BB, ex, r2);
-    const float finv = frsq(f2);
-    const float eg = (q_gb * qj) * finv;
-    const float t = eg * (finv * finv);                // gb2 qq / f^3
-    const float te = t * ex;
-    float fgb = fmaf(-0.25f, te, t);                   // -dE/dr / r
-    float g = te * fmaf(x, kLn2, 1.0f);                // dE/dB_i = -g B_j / 2, dE/dB_j = -g B_i / 2
-    if (GENERAL) {
-      const int orig = (lane + k) & 63;
-      bool valid = ivalid && orig < nj;
-      if (DIAG && k == 32) valid = valid && lane < 32;
-      float sv = 1.0f, se = 1.0f;
-      if (has_excl) {
-        const int cls = (int)((m0 >> orig) & 1ull) | ((int)((m1 >> orig) & 1ull) << 1);
-        sv = cls == 0 ? 1.0f : (cls == 1 ? S.excl_v[1] : (cls == 2 ? S.excl_v[2] : S.excl_v[3]));
-        se = cls == 0 ? 1.0f : (cls == 1 ? S.excl_e[1] : (cls == 2 ? S.excl_e[2] : S.excl_e[3]));
-      }
-      bool clv = valid && (sv != 0.0f || se != 0.0f);
-      if (has_cut) clv = clv && r2 < cut2;
-      const bool gv = gb_has_cut ? (valid && r2 < cut2) : valid;
-      ec = clv ? ec * se : 0.0f;
-      el = clv ? el * sv : 0.0f;
-      fl = clv ? fl * sv : 0.0f;
-      fgb = gv ? fgb : 0.0f;
-      g = gv ? g : 0.0f;
-      if (ENERGY) egb += gv ? (double)eg : 0.0;
-    } else {
-      if (ENERGY) egb += (double)eg;
-    }
-    if (ENERGY && LJC) { ecl += (double)ec; elj += (double)el; }
-    float fr = LJC ? fmaf(ec + fl, rinv2, fgb) : fgb;
-    if (GENERAL) {
-      // An idle lane of a ragged tile may pair an atom with itself (r = 0):
-      // 0 * inf there is NaN, so the final scalar is selected, not just its parts.
-      const int orig = (lane + k) & 63;
-      bool valid = ivalid && orig < nj;
-      if (DIAG && k == 32) valid = valid && lane < 32;
-      fr = valid ? fr : 0.0f;
-    }
-    // F_i = -fr * (x_j - x_i)
-    fxi = fmaf(-fr, dx, fxi); fyi = fmaf(-fr, dy, fyi); fzi = fmaf(-fr, dz, fzi);
-    dbi = fmaf(g, Bj, dbi);
-#if PRX_LDS_ACC
-    {
-      volatile v4f* acc = reinterpret_cast<volatile v4f*>(L.acc);
-      v4f t = acc[lane + k];
-      t.x = fmaf(fr, dx, t.x); t.y = fmaf(fr, dy, t.y); t.z = fmaf(fr, dz, t.z); t.w = fmaf(g, gbi.x, t.w);
-      acc[lane + k] = t;
-    }
-#else
-    fxj = fmaf(fr, dx, fxj); fyj = fmaf(fr, dy, fyj); fzj = fmaf(fr, dz, fzj);
-    dbj = fmaf(g, gbi.x, dbj);
-    if (k != kend) {
-      fxj = rot<PRX_ROT_BPERM_FORCE>(fxj); fyj = rot<PRX_ROT_BPERM_FORCE>(fyj);
-      fzj = rot<PRX_ROT_BPERM_FORCE>(fzj); dbj = rot<PRX_ROT_BPERM_FORCE>(dbj);
-    }
-#endif
-  }
-  part4(v, w, 0)[lane] = make_float4(fxi, fyi, fzi, -0.5f * dbi);
-#if PRX_LDS_ACC
-  wave_lds_sync();
-  {
-    const float4 a0 = L.acc[lane], a1 = L.acc[lane + 64];
-    part4(v, w, 1)[lane] = make_float4(a0.x + a1.x, a0.y + a1.y, a0.z + a1.z, -0.5f * (a0.w + a1.w));
-  }
-#else
-  const int home = (lane + kend) & 63;
-  part4(v, w, 1)[home] = make_float4(fxj, fyj, fzj, -0.5f * dbj);
-#endif
-  if (ENERGY) {
-    for (int off = 32; off > 0; off >>= 1) {
-      egb += __shfl_xor(egb, off);
-      ecl += __shfl_xor(ecl, off);
-      elj += __shfl_xor(elj, off);
-    }
-    if (lane == 0) {
-      v.e_items[(size_t)w * 3 + 0] = egb;
-      v.e_items[(size_t)w * 3 + 1] = ecl;
-      v.e_items[(size_t)w * 3 + 2] = elj;
-    }
-  }
+// Three doubles summed over the wave, in the lanes of ForceSum::e: each
+// exchange puts two values' sums into the halves of one register.
+template <bool HALF>
+__device__ __forceinline__ double add_swap(double x, double y) {
+  const auto swap = [](unsigned p, unsigned q) {
+    if constexpr (HALF)
+      return __builtin_amdgcn_permlane32_swap(p, q, false, false);
+    else
+      return __builtin_amdgcn_permlane16_swap(p, q, false, false);
+  };
+  const auto lo = swap((unsigned)__double2loint(x), (unsigned)__double2loint(y));
+  const auto hi = swap((unsigned)__double2hiint(x), (unsigned)__double2hiint(y));
+  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+template <int CTRL>
+__device__ __forceinline__ double add_dpp(double x) {
+  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xF, 0xF, true);
+  return x + __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double sum_energies(double gb, double cl, double lj) {
+  double e = add_swap<false>(add_swap<true>(gb, cl), add_swap<true>(lj, lj));
+  e = add_dpp<kDppRor8>(e);
+  e = add_dpp<kDppRor8 - 4>(e);
+  e = add_dpp<kDppRor8 - 6>(e);
+  return add_dpp<kDppRor8 - 7>(e);
 }
 
-// The force pass of work item w, by one wave.
-template <bool ENERGY>
-__device__ __forceinline__ void force_item(const DeviceView& v, int w, PairLds& L) {
-  const PairItem it = v.items[w];
-  const int lane = threadIdx.x & 63;
-  const int fl = item_flags(it.meta);
-  const SlotConst& S = v.slots[item_slot(it.meta)];
-  if (!ENERGY && skip_item(v, S, it)) return;
-  const int cls = S.cutoff2 > 0.0f ? (v.item_cls[w] & kClsCutMask) : kClsNear;
-  if (cls == kClsFar) {
-    if (S.gb_cut) {
-      if (ENERGY && lane == 0) {
-        v.e_items[(size_t)w * 3 + 0] = 0.0;
-        v.e_items[(size_t)w * 3 + 1] = 0.0;
-        v.e_items[(size_t)w * 3 + 2] = 0.0;
-      }
-      return;
+// What the pass takes from its system's constants and its item.
+struct ForceConst {
+  float kc, gb2, cut2;  // cut2 > 0: the test r^2 < cut2 per pair
+  bool gb_cut;          // of GB too
+  float ev[4], ee[4];   // scales by exclusion class
+  const unsigned long long* excl;  // the tile's exclusion masks, or nullptr
+};
+
+// LJC = false: GB only (items entirely beyond the LJ/Coulomb cutoff). GEN:
+// ragged tiles, exclusions, and with cut2 > 0 the test r^2 < cut2 per pair, on
+// LJ/Coulomb and, if gb_cut, on GB too.
+template <bool GEN, bool DIAG, bool ENERGY, bool LJC>
+__device__ __forceinline__ void force_tile(const ForceConst& S, int ni, int nj, int lane, float* side0, int sub,
+                                           int nsub, const float4* L, ForceSum<ENERGY>& out) {
+  const Tile4* ti = reinterpret_cast<const Tile4*>(L);
+  const Tile4* tj = ti + 2;
+  const float kc = S.kc, gb2 = S.gb2, cut2 = S.cut2;
+  const bool has_cut = GEN && cut2 > 0.0f, gb_cut = S.gb_cut;
+  const bool has_excl = GEN && LJC && S.excl != nullptr;
+  const int p = lane & 7, q = lane >> 3;
+  float fxj[kEdge] = {}, fyj[kEdge] = {}, fzj[kEdge] = {}, dbj[kEdge] = {};
+  double egb = 0.0, ecl = 0.0, elj = 0.0;
+  const int nb = GEN ? (ni + kEdge - 1) / kEdge : kEdge, na = GEN ? (nj + kEdge - 1) / kEdge : kEdge;
+  const int comp = comp_p(p);
+  PRX_UNROLL(PRX_UNROLL_FORCE)
+  for (int b = sub; b < nb; b += nsub) {
+    const int row = kEdge * b + q;
+    const float4 ia = ti[0][row], ib = ti[1][row];
+    const float q_kc = kc * ia.w, q_gb = gb2 * ia.w;
+    float fxi = 0.f, fyi = 0.f, fzi = 0.f, dbi = 0.f;
+    unsigned long long m0 = 0, m1 = 0;  // the row's exclusion classes, column p of each patch at bit 8 a
+    if (has_excl) {
+      m0 = S.excl[row * 2] >> p;
+      m1 = S.excl[row * 2 + 1] >> p;
     }
-    // GB over every pair, nothing else (a far item is never diagonal)
-    const JSrc js = j_source(v, it, lane);
-    if (item_ni(it.meta) == kTile && js.nj == kTile)
-      force_tile<false, false, ENERGY, false>(v, it, js, lane, w, 0.0f, false, L);
-    else
-      force_tile<true, false, ENERGY, false>(v, it, js, lane, w, 0.0f, false, L);
-    return;
+    int col = p;
+#pragma unroll
+    for (int a = 0; a < kEdge; ++a) {
+      if (GEN && a >= na) break;
+      if (DIAG && a < b) continue;
+      col = after(col, a < 2 ? fxi : fxj[a - 2]);
+      const float4 ja = tj[0][col + kEdge * a], jb = tj[1][col + kEdge * a];
+      const float dx = ja.x - ia.x, dy = ja.y - ia.y, dz = ja.z - ia.z;
+      float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+      const bool once = !DIAG || a != b || p > q;  // each unordered pair once
+      if (DIAG && a == b) r2 = once ? r2 : 1e30f;
+      const bool in = !has_cut || r2 < cut2;
+      if (has_cut && gb_cut && !__any(in)) continue;
+      float lc = 0.0f, rinv2 = 0.0f;  // -dE/dr r of Coulomb + LJ
+      if (LJC && (!has_cut || __any(in))) {
+        const float rinv = frsq(r2);
+        rinv2 = rinv * rinv;
+        float ec = (q_kc * ja.w) * rinv;
+        const float sg = ib.x + jb.x;
+        const float ep = ib.y * jb.y;
+        const float s2 = sg * sg * rinv2;
+        const float s6 = s2 * s2 * s2;
+        float el = ep * fmaf(s6, s6, -s6);  // / 4
+        float fl = ep * s6 * fmaf(48.0f, s6, -24.0f);
+        if (GEN) {
+          if (has_excl) {
+            const unsigned e0 = (unsigned)(m0 >> (kEdge * a)) & 1u, e1 = (unsigned)(m1 >> (kEdge * a)) & 1u;
+            const unsigned cls = e0 | (e1 << 1);
+            if (__any(cls != 0u)) {
+              const float sv = cls == 0 ? 1.0f : (cls == 1 ? S.ev[1] : (cls == 2 ? S.ev[2] : S.ev[3]));
+              const float se = cls == 0 ? 1.0f : (cls == 1 ? S.ee[1] : (cls == 2 ? S.ee[2] : S.ee[3]));
+              const bool some = sv != 0.0f || se != 0.0f;
+              ec = some ? ec * se : 0.0f;
+              el = some ? el * sv : 0.0f;
+              fl = some ? fl * sv : 0.0f;
+            }
+          }
+          if (has_cut) {
+            ec = in ? ec : 0.0f;
+            el = in ? el : 0.0f;
+            fl = in ? fl : 0.0f;
+          }
+        }
+        if (ENERGY) {
+          ecl += once ? (double)ec : 0.0;
+          elj += once ? (double)el : 0.0;
+        }
+        lc = ec + fl;
+      }
+      // GB over every pair
+      const float BB = ib.z * jb.z;
+      const float x = r2 * (ib.w * jb.w);  // r^2 log2(e) / (4 B_i B_j)
+      const float ex = fexp2(-x);
+      const float f2 = fmaf(BB, ex, r2);
+      const float finv = frsq(f2);
+      const float eg = (q_gb * ja.w) * finv;
+      const float t = eg * (finv * finv);  // gb2 qq / f^3
+      const float te = t * ex;
+      float fgb = fmaf(-0.25f, te, t);     // -dE/dr / r
+      float g = te * fmaf(x, kLn2, 1.0f);  // dE/dB_i = -g B_j / 2, dE/dB_j = -g B_i / 2
+      if (GEN && has_cut && gb_cut) {
+        fgb = in ? fgb : 0.0f;
+        g = in ? g : 0.0f;
+        if (ENERGY) egb += in && once ? (double)eg : 0.0;
+      } else if (ENERGY) {
+        egb += once ? (double)eg : 0.0;
+      }
+      const float fr = LJC ? fmaf(lc, rinv2, fgb) : fgb;
+      // F_i = -fr * (x_j - x_i)
+      fxi = fmaf(-fr, dx, fxi); fyi = fmaf(-fr, dy, fyi); fzi = fmaf(-fr, dz, fzi);
+      dbi = fmaf(g, jb.z, dbi);
+      fxj[a] = fmaf(fr, dx, fxj[a]); fyj[a] = fmaf(fr, dy, fyj[a]); fzj[a] = fmaf(fr, dz, fzj[a]);
+      dbj[a] = fmaf(g, ib.z, dbj[a]);
+    }
+    const float t = sum_p4(fxi, fyi, fzi, -0.5f * dbi, p);
+    if ((p & 1) == 0) side0[row * 4 + comp] = t;
   }
-  const JSrc js = j_source(v, it, lane);
-  const bool full = item_ni(it.meta) == kTile && js.nj == kTile;
-  const float cut2 = cls == kClsStraddle ? S.cutoff2 : 0.0f;
-  const bool gb_cut = S.gb_cut != 0;
-  if (fl & kFlagDiag) {
-    force_tile<true, true, ENERGY, true>(v, it, js, lane, w, cut2, gb_cut, L);
-  } else if (full && !(fl & kFlagExcl) && cut2 == 0.0f) {
-    force_tile<false, false, ENERGY, true>(v, it, js, lane, w, 0.0f, false, L);
-  } else {
-    force_tile<true, false, ENERGY, true>(v, it, js, lane, w, cut2, gb_cut, L);
-  }
+  out.x = sum_q(fxj, lane);
+  out.y = sum_q(fyj, lane);
+  out.z = sum_q(fzj, lane);
+  out.g = -0.5f * sum_q(dbj, lane);
+  if (ENERGY) out.e = sum_energies(egb, ecl, 4.0 * elj);
 }
+
+// The force pass over one item (as BornPass).
+template <bool ENERGY>
+struct ForcePass {
+  typedef ForceSum<ENERGY> Sum;
+  static constexpr int kLds = kForceLds;
+  int w, lane, ni, nj, cls, nsub, flags;
+  ForceConst K;
+  float* side0;
+  bool full;
+
+  __device__ __forceinline__ bool stage(const DeviceView& v, int w_, const PairItem& it, bool rows, bool cols,
+                                        float4* L) {
+    w = w_;
+    lane = threadIdx.x & 63;
+    const SlotConst& S = v.slots[item_slot(it.meta)];
+    if (!ENERGY && skip_item(v, S, it)) return false;
+    cls = S.cutoff2 > 0.0f ? (v.item_cls[w] & kClsCutMask) : kClsNear;
+    if (cls == kClsFar && S.gb_cut) {
+      if (ENERGY && lane < 3 && rows) v.e_items[(size_t)w * 3 + lane] = 0.0;
+      return false;
+    }
+    const JSrc js = j_source(v, it, lane);
+    ni = item_ni(it.meta);
+    nj = js.nj;
+    full = ni == kTile && nj == kTile;
+    nsub = it.nsub;
+    flags = item_flags(it.meta);
+    side0 = reinterpret_cast<float*>(part4(v, w, 0));
+    K.kc = S.k_coulomb;
+    K.gb2 = S.gb2;
+    K.cut2 = cls == kClsStraddle ? S.cutoff2 : 0.0f;
+    K.gb_cut = S.gb_cut != 0;
+    K.excl = it.excl >= 0 ? v.excl_masks + (size_t)it.excl * 128 : nullptr;
+    for (int k = 1; k < 4; ++k) {
+      K.ev[k] = S.excl_v[k];
+      K.ee[k] = S.excl_e[k];
+    }
+    // (x, y, z, q), (sigma/2, sqrt(eps), B, a) of the rows and the columns
+    const int gi = it.i0 + min(lane, ni - 1), gj = js.gj;
+    float4 pi, ci, bi, pj, cj, bj;
+    if (rows) { pi = v.pos[gi]; ci = v.nb4[gi]; bi = v.gb4[gi]; }
+    if (cols) { pj = v.pos[gj]; cj = v.nb4[gj]; bj = v.gb4[gj]; }
+    Tile4* t = reinterpret_cast<Tile4*>(L);
+    // past the end of a ragged tile: no charge, no well depth, B = 1 and an exponent of 0
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f), one = make_float4(1.f, 0.f, 0.f, 0.f);
+    if (rows) {
+      if (!full && lane >= ni) { pi = pad_pos(lane); ci = zero; bi = one; }
+      t[0][lane] = make_float4(pi.x, pi.y, pi.z, ci.x);
+      t[1][lane] = make_float4(ci.y, ci.z, bi.x, bi.y);
+    }
+    if (cols) {
+      if (!full && lane >= nj) { pj = pad_pos(lane); cj = zero; bj = one; }
+      t[2][lane] = make_float4(pj.x, pj.y, pj.z, cj.x);
+      t[3][lane] = make_float4(cj.y, cj.z, bj.x, bj.y);
+    }
+    return true;
+  }
+
+  __device__ __forceinline__ Sum run(const DeviceView&, int sub, float4* L, float4*) const {
+    Sum f;
+    if (cls == kClsFar) {  // GB over every pair, nothing else (a far item is never diagonal)
+      if (full)
+        force_tile<false, false, ENERGY, false>(K, ni, nj, lane, side0, sub, nsub, L, f);
+      else
+        force_tile<true, false, ENERGY, false>(K, ni, nj, lane, side0, sub, nsub, L, f);
+    } else if (flags & kFlagDiag) {
+      force_tile<true, true, ENERGY, true>(K, ni, nj, lane, side0, sub, nsub, L, f);
+    } else if (full && !(flags & kFlagExcl) && K.cut2 == 0.0f) {
+      force_tile<false, false, ENERGY, true>(K, ni, nj, lane, side0, sub, nsub, L, f);
+    } else {
+      force_tile<true, false, ENERGY, true>(K, ni, nj, lane, side0, sub, nsub, L, f);
+    }
+    return f;
+  }
+};
 
 // ---------------------------------------------------------------------------
 // Pass 3: chain rule through the Born radii
 // ---------------------------------------------------------------------------
 
-template <bool GENERAL, bool DIAG, bool FAR, bool F4 = false>
-__device__ __forceinline__ void chain_tile(const DeviceView& v, const PairItem& it, const JSrc& js, int lane, int w,
-                                           float cut2, PairLds& L) {
-  const int ni = item_ni(it.meta), nj = js.nj;
-  const int gi = it.i0 + min(lane, ni - 1);
-  const int gj = js.gj;
-  const float4 pi = v.pos[gi], bi = v.born4[gi];
-  const float ci = v.gb4[gi].w;
-  {
-    const float4 pj = v.pos[gj], bj = v.born4[gj];
-    const float4 a = make_float4(pj.x, pj.y, pj.z, bj.z);          // x, y, z, s^2
-    const float4 b = make_float4(bj.w, v.gb4[gj].w, bj.x, bj.y);     // s^3/2, c, rho, s
-    L.a[lane] = a; L.a[lane + 64] = a;
-    L.b[lane] = b; L.b[lane + 64] = b;
-#if PRX_LDS_ACC
-    L.acc[lane] = make_float4(0.f, 0.f, 0.f, 0.f);
-    L.acc[lane + 64] = make_float4(0.f, 0.f, 0.f, 0.f);
-#endif
-  }
-  wave_lds_sync();
-  float fxi = 0.f, fyi = 0.f, fzi = 0.f, fxj = 0.f, fyj = 0.f, fzj = 0.f;
-  const bool ivalid = lane < ni;
-  constexpr int kbeg = DIAG ? 1 : 0, kend = DIAG ? 32 : 63;
-  PRX_UNROLL(PRX_UNROLL_CHAIN)
-  for (int k = kbeg; k <= kend; ++k) {
-    const float4 ja = L.a[lane + k];
-    const float2 jb = *reinterpret_cast<const float2*>(&L.b[lane + k]);  // the far field needs only these
-    const float xj = ja.x, yj = ja.y, zj = ja.z, sj2 = ja.w, sj3h = jb.x, cj = jb.y;
-    const float dx = xj - pi.x, dy = yj - pi.y, dz = zj - pi.z;
-    const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-    float gsc;  // (c_i dI(r; rho_i, s_j)/dr + c_j dI(r; rho_j, s_i)/dr) / r; F_i = gsc (x_j - x_i)
-    if (FAR) {
-      gsc = chain_far<F4>(frcp(r2), sj2, ci * sj3h, bi.z, cj * bi.w);
+// An atom of the chain pass: short (x, y, z, c), (w0, w1, w2, w3), else
+// (x, y, z, c), (s^2, s^3/3, rho, s), as BornAtom.
+template <int CLS>
+struct ChainAtom {
+  static constexpr bool kShort = ChainW<CLS>::N <= 4;
+  float x, y, z, c, s2, s33;
+  float w[ChainW<CLS>::N];
+
+  __device__ __forceinline__ static void stage(Tile4* t, int lane, const float4& p, const float4& b, float c) {
+    t[0][lane] = make_float4(p.x, p.y, p.z, c);
+    if constexpr (kShort) {
+      float w[ChainW<CLS>::N];
+      obc_weights<ChainW<CLS>>(b.z, b.w, w);
+      t[1][lane] = make_float4(w[0], w[1], w[2], ChainW<CLS>::N > 3 ? w[3 % ChainW<CLS>::N] : 0.0f);
     } else {
-      const float rinv = frsq(r2);
-      const float rhoj = L.b[lane + k].z, sj = L.b[lane + k].w;  // near field only
-      const float r = r2 * rinv;
-      const bool far1 = obc_far(r, bi.x, sj), far2 = obc_far(r, rhoj, bi.y);
-      const float u = rinv * rinv;
-      if (__all(far1 && far2)) {
-        gsc = chain_far(u, sj2, ci * sj3h, bi.z, cj * bi.w);
-      } else {
-        const float u2r = u * u * rinv, rs = fminf(rinv, 1e4f);
-        const float d1 = far1 ? obc_far_dI(sj2, sj3h, u, u2r) : born_dr(r, rs, bi.x, sj, sj2);
-        const float d2 = far2 ? obc_far_dI(bi.z, bi.w, u, u2r) : born_dr(r, rs, rhoj, bi.y, bi.z);
-        gsc = fmaf(ci, d1, cj * d2) * rinv;
-      }
+      t[1][lane] = make_float4(b.z, b.w, b.x, b.y);
     }
-    if (GENERAL) {
-      const int orig = (lane + k) & 63;
-      bool valid = ivalid && orig < nj;
-      if (DIAG && k == 32) valid = valid && lane < 32;
-      if (cut2 > 0.0f) valid = valid && r2 < cut2;
-      gsc = valid ? gsc : 0.0f;
+  }
+  __device__ __forceinline__ void read(const Tile4* t, int e, bool row) {
+    const float4 a = t[0][e];
+    x = a.x; y = a.y; z = a.z; c = a.w;
+    if constexpr (kShort) {
+      const float4 b = t[1][e];
+      w[0] = b.x; w[1] = b.y; w[2] = b.z;
+      if constexpr (ChainW<CLS>::N > 3) w[3] = b.w;
+    } else {
+      const float2 b = *reinterpret_cast<const float2*>(&t[1][e]);
+      s2 = b.x;
+      s33 = b.y;
+      if (row) obc_weights<ChainW<CLS>>(s2, s33, w);
     }
-    fxi = fmaf(gsc, dx, fxi); fyi = fmaf(gsc, dy, fyi); fzi = fmaf(gsc, dz, fzi);
-#if PRX_LDS_ACC
-    {
-      volatile v4f* acc = reinterpret_cast<volatile v4f*>(L.acc);
-      v4f t = acc[lane + k];
-      t.x = fmaf(-gsc, dx, t.x); t.y = fmaf(-gsc, dy, t.y); t.z = fmaf(-gsc, dz, t.z);
-      acc[lane + k] = t;
-    }
-#else
-    fxj = fmaf(-gsc, dx, fxj); fyj = fmaf(-gsc, dy, fyj); fzj = fmaf(-gsc, dz, fzj);
-    if (k != kend) {
-      // PRX_ROT_BPERM_CHAIN 2 or 3: the first one or two by the crossbar, the rest by DPP
-      fxj = rot<(PRX_ROT_BPERM_CHAIN >= 1)>(fxj);
-      fyj = rot<(PRX_ROT_BPERM_CHAIN == 1 || PRX_ROT_BPERM_CHAIN == 3)>(fyj);
-      fzj = rot<(PRX_ROT_BPERM_CHAIN == 1)>(fzj);
-    }
-#endif
   }
-  put_part3(v, w, 0, lane, fxi, fyi, fzi);
-#if PRX_LDS_ACC
-  wave_lds_sync();
-  {
-    const float4 a0 = L.acc[lane], a1 = L.acc[lane + 64];
-    put_part3(v, w, 1, lane, a0.x + a1.x, a0.y + a1.y, a0.z + a1.z);
+  // f sum_k w_k u^k
+  __device__ __forceinline__ float sum(float f, float u, bool row) const {
+    if (kShort || row) return f * horner(w, u);
+    return (f * s33) * obc_poly<ChainW<CLS>>(s2 * u);
   }
-#else
-  const int home = (lane + kend) & 63;
-  put_part3(v, w, 1, home, fxj, fyj, fzj);
-#endif
-}
-
-// The chain pass of work item w, by one wave.
-__device__ __forceinline__ void chain_item(const DeviceView& v, int w, PairLds& L) {
-  const PairItem it = v.items[w];
-  const int lane = threadIdx.x & 63;
-  const int fl = item_flags(it.meta);
-  const SlotConst& S = v.slots[item_slot(it.meta)];
-  if (skip_item(v, S, it)) return;
-  const int cls = v.item_cls[w];
-  float cut2 = 0.0f;
-  if (S.gb_cut) {
-    if ((cls & kClsCutMask) == kClsFar) return;
-    if ((cls & kClsCutMask) == kClsStraddle) cut2 = S.cutoff2;
-  }
-  const JSrc js = j_source(v, it, lane);
-  const bool full = item_ni(it.meta) == kTile && js.nj == kTile;
-  if (fl & kFlagDiag) {
-    chain_tile<true, true, false>(v, it, js, lane, w, cut2, L);
-  } else if (cls & kClsObcFar4) {
-    if (full && cut2 == 0.0f)
-      chain_tile<false, false, true, true>(v, it, js, lane, w, 0.0f, L);
-    else
-      chain_tile<true, false, true, true>(v, it, js, lane, w, cut2, L);
-  } else if (cls & kClsObcFar) {
-    if (full && cut2 == 0.0f)
-      chain_tile<false, false, true>(v, it, js, lane, w, 0.0f, L);
-    else
-      chain_tile<true, false, true>(v, it, js, lane, w, cut2, L);
-  } else if (full && cut2 == 0.0f) {
-    chain_tile<false, false, false>(v, it, js, lane, w, 0.0f, L);
-  } else {
-    chain_tile<true, false, false>(v, it, js, lane, w, cut2, L);
-  }
-}
-
-
-// One wave's LDS slice in a kernel that runs every pass.
-union PassLds {
-  BornLds born;
-  PairLds pair;
 };
+
+// gsc of a near or far pair (chain_tile); a = (x, y, z, c), b = (s^2, s^3/3, rho, s).
+__device__ __forceinline__ float chain_one(float r2, float ci, const float4& bi, float cj, const float4& bj) {
+  const float rinv = frsq(r2), u = rinv * rinv, u2r = u * u * rinv, r = r2 * rinv, rs = fminf(rinv, 1e4f);
+  const float d1 = obc_far(r, bi.z, bj.w) ? u2r * (bj.y * obc_poly<ChainW<kMixed>>(bj.x * u))
+                                          : born_dr(r, rs, bi.z, bj.w, bj.x);
+  const float d2 = obc_far(r, bj.z, bi.w) ? u2r * (bi.y * obc_poly<ChainW<kMixed>>(bi.x * u))
+                                          : born_dr(r, rs, bj.z, bi.w, bi.x);
+  return fmaf(ci, d1, cj * d2) * rinv;
+}
+
+__device__ __forceinline__ void chain_near(float4* L, float4* scratch, unsigned long long near, int lane, int ni, bool diag, bool cut,
+                                           float lim2, int sub, int nsub, float3& rows, float3& cols) {
+  Tile4* ti = reinterpret_cast<Tile4*>(L);
+  Tile4* tj = ti + 2;
+  if (diag) {
+    const float4 me = ti[0][lane], mb = ti[1][lane];
+    near_diag(ti, lane, ni, sub, nsub, cut, lim2, [&](const int (&o)[2], const bool (&on)[2]) {
+      float g[2], dx[2], dy[2], dz[2];
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const float4 a = ti[0][o[k]], b = ti[1][o[k]];
+        dx[k] = a.x - me.x; dy[k] = a.y - me.y; dz[k] = a.z - me.z;
+        const float r2 = fmaf(dx[k], dx[k], fmaf(dy[k], dy[k], dz[k] * dz[k]));
+        g[k] = chain_one(on[k] ? r2 : 1.0f, me.w, mb, a.w, b);
+      }
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const float f = on[k] ? g[k] : 0.0f;
+        cols.x = fmaf(f, dx[k], cols.x);
+        cols.y = fmaf(f, dy[k], cols.y);
+        cols.z = fmaf(f, dz[k], cols.z);
+      }
+    });
+    return;
+  }
+  near_list(
+      ti, tj, near, lane, cut, lim2, scratch,
+      [&](int row, int col) {
+        const float4 ai = ti[0][row], bi = ti[1][row], aj = tj[0][col], bj = tj[1][col];
+        const float dx = aj.x - ai.x, dy = aj.y - ai.y, dz = aj.z - ai.z;
+        const float gsc = chain_one(fmaf(dx, dx, fmaf(dy, dy, dz * dz)), ai.w, bi, aj.w, bj);
+        scratch[lane].x = gsc * dx;
+        scratch[lane].y = gsc * dy;
+        scratch[lane].z = gsc * dz;
+      },
+      [&](const float4& c, float mr, float mc) {
+        rows.x = fmaf(mr, c.x, rows.x); rows.y = fmaf(mr, c.y, rows.y); rows.z = fmaf(mr, c.z, rows.z);
+        cols.x = fmaf(-mc, c.x, cols.x); cols.y = fmaf(-mc, c.y, cols.y); cols.z = fmaf(-mc, c.z, cols.z);
+      });
+}
+
+// As born_tile. Per pair: F_i = gsc (x_j - x_i), gsc = (c_i dI(rho_i, s_j)/dr +
+// c_j dI(rho_j, s_i)/dr) / r, in the far field u^3 (c_i P_j(u) + c_j P_i(u)).
+template <int CLS, bool DIAG, bool CUT, bool FULL>
+__device__ __forceinline__ void chain_tile(const float4* L, int ni, int nj, int lane, float cut2, float thr2, int sub,
+                                           int nsub, float3& rows, float3& cols, unsigned long long& near) {
+  const Tile4* ti = reinterpret_cast<const Tile4*>(L);
+  const Tile4* tj = ti + 2;
+  const int p = lane & 7, q = lane >> 3;
+  float fxj[kEdge] = {}, fyj[kEdge] = {}, fzj[kEdge] = {};
+  const int nb = FULL ? kEdge : (ni + kEdge - 1) / kEdge, na = FULL ? kEdge : (nj + kEdge - 1) / kEdge;
+  PRX_UNROLL(PRX_UNROLL_CHAIN)
+  for (int b = sub; b < nb; b += nsub) {
+    ChainAtom<CLS> i;
+    float fxi = 0.f, fyi = 0.f, fzi = 0.f;
+    i.read(ti, kEdge * b + q, true);
+    unsigned marks = 0;
+    int col = p;
+#pragma unroll
+    for (int a = 0; a < kEdge; ++a) {
+      if (!FULL && a >= na) break;
+      if (DIAG && a < b) continue;
+      ChainAtom<CLS> j;
+      col = after(col, a < 2 ? fxi : fxj[a - 2]);
+      j.read(tj, col + kEdge * a, false);
+      const float dx = j.x - i.x, dy = j.y - i.y, dz = j.z - i.z;
+      float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+      if (DIAG && a == b) r2 = p > q ? r2 : 1e30f;
+      bool on = true;
+      if (CUT) on = r2 < cut2;
+      if (CLS == kMixed) {
+        const bool close = !(r2 > thr2);
+        if (!DIAG) marks |= (__ballot(on && close) != 0 ? 1u : 0u) << a;
+        on = on && !close;
+      }
+      float u = frcp(r2);
+      if (CUT || CLS == kMixed) u = on ? u : 0.0f;
+      const float gsc = (u * u * u) * (j.sum(i.c, u, false) + i.sum(j.c, u, true));
+      fxi = fmaf(gsc, dx, fxi); fyi = fmaf(gsc, dy, fyi); fzi = fmaf(gsc, dz, fzi);
+      fxj[a] = fmaf(-gsc, dx, fxj[a]); fyj[a] = fmaf(-gsc, dy, fyj[a]); fzj[a] = fmaf(-gsc, dz, fzj[a]);
+    }
+    const float x = sum_p(fxi), y = sum_p(fyi), z = sum_p(fzi);
+    rows.x = p == b ? x : rows.x; rows.y = p == b ? y : rows.y; rows.z = p == b ? z : rows.z;
+    if (CLS == kMixed && !DIAG) near |= (unsigned long long)marks << (kEdge * b);
+  }
+  cols = make_float3(sum_q(fxj, lane), sum_q(fyj, lane), sum_q(fzj, lane));
+}
+
+struct ChainRun {
+  const float4* L;
+  int ni, nj, lane;
+  float cut2, thr2;
+  int sub, nsub;
+  float3 rows, cols;
+  unsigned long long near;
+  template <int CLS, bool DIAG, bool CUT, bool FULL>
+  __device__ __forceinline__ void run() {
+    chain_tile<CLS, DIAG, CUT, FULL>(L, ni, nj, lane, cut2, thr2, sub, nsub, rows, cols, near);
+  }
+};
+
+__device__ __forceinline__ void put_part3(const DeviceView& v, int w, int side, int at, float x, float y, float z) {
+  float* pc = part3(v, w, side);
+  pc[at] = x;
+  pc[kTile + at] = y;
+  pc[2 * kTile + at] = z;
+}
+
+struct ChainSum {
+  float x = 0.0f, y = 0.0f, z = 0.0f;
+  __device__ __forceinline__ void add(const ChainSum& o) { x += o.x; y += o.y; z += o.z; }
+  __device__ __forceinline__ void store(const DeviceView& v, int w, int lane) const { put_part3(v, w, 1, lane, x, y, z); }
+  __device__ __forceinline__ void to_lds(float4* at, int lane) const { at[lane] = make_float4(x, y, z, 0.0f); }
+  __device__ __forceinline__ void from_lds(const float4* at, int lane) {
+    const float4 f = at[lane];
+    x = f.x; y = f.y; z = f.z;
+  }
+};
+
+// The chain pass over one item (as BornPass).
+struct ChainPass {
+  typedef ChainSum Sum;
+  static constexpr int kLds = kChainLds;
+  int w, lane, ni, nj, tier, nsub;
+  float cut2, thr2, lim2;
+  bool diag, full, cut;
+
+  __device__ __forceinline__ bool stage(const DeviceView& v, int w_, const PairItem& it, bool rows, bool cols,
+                                        float4* L) {
+    w = w_;
+    lane = threadIdx.x & 63;
+    const SlotConst& S = v.slots[item_slot(it.meta)];
+    if (skip_item(v, S, it)) return false;
+    const int packed = v.item_cls[w], cls = packed & kClsMask;
+    thr2 = cls_thr2(packed);
+    cut = false;
+    if (S.gb_cut) {
+      if ((cls & kClsCutMask) == kClsFar) return false;
+      cut = (cls & kClsCutMask) == kClsStraddle;
+    }
+    cut2 = S.cutoff2;
+    lim2 = cut ? fminf(thr2, prev_below(cut2)) : thr2;
+    tier = cls >> kClsTierShift;
+    const JSrc js = j_source(v, it, lane);
+    ItemAtoms t = load_atoms<true>(v, it, js, lane, rows, cols);
+    diag = (item_flags(it.meta) & kFlagDiag) != 0;
+    ni = item_ni(it.meta);
+    nj = js.nj;
+    full = ni == kTile && nj == kTile;
+    nsub = it.nsub;
+    if (!full) pad_atoms(t, lane, ni, nj);
+    StageRun<ChainAtom> put{t, lane, rows, cols, L};
+    by_class(tier, diag, cut, full, put);
+    return true;
+  }
+
+  __device__ __forceinline__ ChainSum run(const DeviceView& v, int sub, float4* L,
+                                          float4* scratch) const {
+    const int p = lane & 7, q = lane >> 3;
+    const float3 zero = make_float3(0.f, 0.f, 0.f);
+    ChainRun f{L, ni, nj, lane, cut2, thr2, sub, nsub, zero, zero, 0};
+    by_class(tier, diag, cut, full, f);
+    if (f.near != 0 || diag) chain_near(L, scratch, f.near, lane, ni, diag, cut, lim2, sub, nsub, f.rows, f.cols);
+    if ((p & (nsub - 1)) == sub) put_part3(v, w, 0, kEdge * p + q, f.rows.x, f.rows.y, f.rows.z);
+    ChainSum s;
+    s.x = f.cols.x; s.y = f.cols.y; s.z = f.cols.z;
+    return s;
+  }
+};
+
+// ---------------------------------------------------------------------------
+// Items to waves
+// ---------------------------------------------------------------------------
+// The items of a small system are cut into shares by rows (PairItem.nsub: share
+// s has the rows b = s, s + nsub, ... of the patches), whose column sums are
+// added in their order. How many depends on the system's own size alone, so
+// its sums are the same in any pack and on either path:
+// - pair_wave: one wave takes an item, its shares one after the other. For work
+//   lists that fill the chip: a wave's registers and LDS are free as soon as its
+//   own item is done, and no wave waits for another.
+// - pair_unit: a group of kUnitWaves waves takes a unit (prx_common.h): a wave
+//   per share. The first two waves of an item bring its two tiles into LDS,
+//   for all. For short work lists, whose time is that of one item.
+// SYNC: every unit holds exactly two workgroup barriers, also one of whole
+// items or of items without work, so that groups of one workgroup meet the same
+// barriers whatever their units are; without it only cut items hold them.
+
+template <class Pass>
+__device__ __forceinline__ void pair_wave(const DeviceView& v, int w, float4* L) {
+  const PairItem it = v.items[w];
+  Pass f;
+  if (!f.stage(v, w, it, true, true, L)) return;
+  wave_lds_sync();
+  typename Pass::Sum s;
+  for (int sub = 0; sub < it.nsub; ++sub) s.add(f.run(v, sub, L, L + 4 * kTile));
+  s.store(v, w, f.lane);
+}
+
+// Workgroup memory of one group: per wave two tiles (used by the first wave of
+// each item) and the wave's scratch, which takes its column sums at the end.
+template <int N>
+struct UnitLds {
+  float4 wave[kUnitWaves][N];
+};
+
+// k: the wave's index in the group.
+template <bool SYNC, class Pass, class Lds>
+__device__ __forceinline__ void pair_unit(const DeviceView& v, int unit, int k, Lds& L) {
+  const PairUnit u = v.units != nullptr ? v.units[unit] : PairUnit{unit, 1, kUnitWaves};
+  const int sh = u.shares;
+  const int m = sh == kUnitWaves ? 0 : (sh == 1 ? k : k / 2), sub = k - m * sh;
+  const int w = u.first + m;
+  float4* const tiles = L.wave[m * sh];
+  float4* const own = L.wave[k] + 4 * kTile;
+  const bool meet = SYNC || sh > 1;
+  PairItem it;
+  Pass f;
+  bool on = m < u.n;
+  if (on) {
+    it = v.items[w];
+    on = f.stage(v, w, it, sub == 0, sub == (sh > 1 ? 1 : 0), tiles);
+  }
+  if (meet)
+    __syncthreads();
+  else
+    wave_lds_sync();
+  typename Pass::Sum s;
+  if (on) {
+    s.add(f.run(v, sub, tiles, own));
+    if (sub > 0) s.to_lds(own, f.lane);
+  }
+  if (meet) __syncthreads();
+  if (!on || sub > 0) return;
+  for (int n = 1; n < sh; ++n) {
+    typename Pass::Sum o;
+    o.from_lds(L.wave[k + n] + 4 * kTile, f.lane);
+    s.add(o);
+  }
+  s.store(v, w, f.lane);
+}
+
+// Item or unit of block b of nb. Workgroups are dispatched to the 8 XCDs round-robin
+// (block b to XCD b mod 8), and each XCD has its own L2. With PRX_XCD_MAP the
+// blocks are renumbered so that XCD x runs one contiguous run of them
+// (consecutive items share their i tile and neighbouring j tiles, which then
+// hit in that XCD's L2, and so do the partials for the tile gathers): block
+// b = 8k + x becomes x * per + min(x, rem) + k, a bijection on [0, nb) with
+// per = nb / 8, rem = nb % 8. Not with neighbour lists: there most chunk items
+// are empty, and more so in the first rows, so that one XCD of eight would get
+// more than twice the average work (20,000 atoms cut at 20 A, Born, force, chain:
+// 51, 55, 58 us; 45, 42, 50 in plain order).
+constexpr int kXcds = 8;
+
+__device__ __forceinline__ int unit_id(const DeviceView& v, int b, int nb) {
+#if PRX_XCD_MAP
+  if (v.nl_tp_hw > 0) return b;
+  const int per = nb / kXcds, rem = nb % kXcds;
+  const int x = b % kXcds, k = b / kXcds;
+  b = x * per + min(x, rem) + k;
+#endif
+  return b;
+}
+
+// Wave of this thread within its group of kUnitWaves (wave-uniform).
+__device__ __forceinline__ int unit_wave() {
+  return __builtin_amdgcn_readfirstlane((int)((threadIdx.x >> 6) & (kUnitWaves - 1)));
+}
 
 }  // namespace prx

@@ -28,7 +28,7 @@ namespace prx {
 
 namespace {
 
-constexpr int kPersistThreads = 256;
+constexpr int kPersistThreads = 64 * kUnitWaves;  // one unit of the pair passes per block
 constexpr int kPersistWaves = kPersistThreads / 64;
 constexpr unsigned kSpinLimit = 1u << 24;  // polls of ~0.1 us each: seconds, far above any pass
 
@@ -68,8 +68,8 @@ __device__ __forceinline__ bool grid_sync(GridBarrier* bar, unsigned& gen) {
 
 __global__ __launch_bounds__(kPersistThreads) void k_persist_steps(DeviceView v, const int32_t* ranges, int n_slots,
                                                                     int n_steps, int has_nl, GridBarrier* bar) {
-  __shared__ PassLds lds[kPersistWaves];
-  PassLds& L = lds[threadIdx.x >> 6];
+  __shared__ UnitLds<kPairLds> L;
+  const int uw = unit_wave();
   __shared__ GatherLds G;
   unsigned gen = 0;  // the barrier's generation, tracked by thread 0
   const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * kPersistWaves + (threadIdx.x >> 6)));
@@ -98,7 +98,10 @@ __global__ __launch_bounds__(kPersistThreads) void k_persist_steps(DeviceView v,
       for (int w = wave; w < v.nl_tp_hw; w += n_waves) nl_fill_wave(v, w);
       if (!grid_sync(bar, gen)) return;
     }
-    for (int w = wave; w < v.n_items; w += n_waves) born_item(v, w, L.born);
+    for (int u = blockIdx.x; u < v.n_units; u += gridDim.x) {
+      pair_unit<true, BornPass>(v, u, uw, L);
+      __syncthreads();
+    }
     for (int e = tid; e < n_bonded; e += n_threads) bonded_entry<false>(v, e);
     if (!grid_sync(bar, gen)) return;
     for (int t = blockIdx.x; t < v.n_tiles; t += gridDim.x) {
@@ -106,14 +109,20 @@ __global__ __launch_bounds__(kPersistThreads) void k_persist_steps(DeviceView v,
       __syncthreads();
     }
     if (!grid_sync(bar, gen)) return;
-    for (int w = wave; w < v.n_items; w += n_waves) force_item<false>(v, w, L.pair);
+    for (int u = blockIdx.x; u < v.n_units; u += gridDim.x) {
+      pair_unit<true, ForcePass<false>>(v, u, uw, L);
+      __syncthreads();
+    }
     if (!grid_sync(bar, gen)) return;
     for (int t = blockIdx.x; t < v.n_tiles; t += gridDim.x) {
       force_gather_tile<false>(v, t, G);
       __syncthreads();
     }
     if (!grid_sync(bar, gen)) return;
-    for (int w = wave; w < v.n_items; w += n_waves) chain_item(v, w, L.pair);
+    for (int u = blockIdx.x; u < v.n_units; u += gridDim.x) {
+      pair_unit<true, ChainPass>(v, u, uw, L);
+      __syncthreads();
+    }
     if (!grid_sync(bar, gen)) return;
     const int mode = k + 1 == n_steps ? 2 : 1;  // the last step stops after B(F)
     for (int t = blockIdx.x; t < v.n_tiles; t += gridDim.x) {

@@ -1,34 +1,4 @@
 // Generated by prolix_amd/tune.py -- pair-kernel settings measured fastest on
-// the 256-system batched mix (mean ms per captured step).
-// Chain unroll, same box, two runs each (ms per mix step; chain pass in-graph):
-// w2_ub8_uf4_uc4_x1_bpb0_bpf1_bpc2_mw0: 1.6459 1.6465; chain 0.4943 0.4944
-// w2_ub8_uf4_uc4_x1_bpb0_bpf1_bpc2_mw6: 1.6462 1.6470; chain 0.4927 0.4961
-// w2_ub8_uf4_uc8_x1_bpb0_bpf1_bpc2_mw0: 1.6513 1.6515; chain 0.5011 0.5004
+// the 256-system batched mix (mean ms per captured step). None differs from its
+// default in prx_pair_dev.h.
 #pragma once
-#ifndef PRX_PAIR_WAVES
-#define PRX_PAIR_WAVES 2
-#endif
-#ifndef PRX_UNROLL_BORN
-#define PRX_UNROLL_BORN 8
-#endif
-#ifndef PRX_UNROLL_FORCE
-#define PRX_UNROLL_FORCE 4
-#endif
-#ifndef PRX_UNROLL_CHAIN
-#define PRX_UNROLL_CHAIN 4
-#endif
-#ifndef PRX_XCD_MAP
-#define PRX_XCD_MAP 1
-#endif
-#ifndef PRX_ROT_BPERM_BORN
-#define PRX_ROT_BPERM_BORN 0
-#endif
-#ifndef PRX_ROT_BPERM_FORCE
-#define PRX_ROT_BPERM_FORCE 1
-#endif
-#ifndef PRX_ROT_BPERM_CHAIN
-#define PRX_ROT_BPERM_CHAIN 2
-#endif
-#ifndef PRX_MIN_WAVES
-#define PRX_MIN_WAVES 0
-#endif

@@ -1,9 +1,9 @@
 """Autotuner for the pair kernels' build-time settings.
 
-The settings are the waves (work items) per workgroup, the unroll depth of the
-Born, force and chain loops, the XCD-aware item order, whether each pass's
-j-side accumulators rotate by DPP or through the LDS crossbar (ds_bpermute), and a
-minimum occupancy the force and chain kernels' registers must fit. They are
+The settings are the unroll depth of the Born, force and chain passes' loops
+over an item's rows of patches, the XCD-aware item order, and a minimum
+occupancy the three kernels' registers must fit (0: none for the Born and chain
+passes, the force pass's own choice for it). They are
 compile-time constants of ``csrc/prx_pair_dev.h`` (the pair passes' device
 code, compiled into ``prx_pair.hip``'s kernels); the chosen ones live in
 ``csrc/prx_tuned.h``, which that header includes before its defaults.
@@ -42,19 +42,14 @@ TUNE_DIR = PKG / "lib" / "tune"
 
 # Each setting's values, and its default in prx_pair_dev.h.
 KNOBS = {
-    "PRX_PAIR_WAVES": (2, 4, 8),
-    "PRX_UNROLL_BORN": (4, 8),
-    "PRX_UNROLL_FORCE": (2, 4, 8),
-    "PRX_UNROLL_CHAIN": (4, 8),
+    "PRX_UNROLL_BORN": (1, 2),
+    "PRX_UNROLL_FORCE": (1, 2),
+    "PRX_UNROLL_CHAIN": (1, 2),
     "PRX_XCD_MAP": (0, 1),
-    "PRX_ROT_BPERM_BORN": (0, 1),
-    "PRX_ROT_BPERM_FORCE": (0, 1),
-    "PRX_ROT_BPERM_CHAIN": (0, 1, 2, 3),
     "PRX_MIN_WAVES": (0, 6),
 }
-DEFAULTS = {"PRX_PAIR_WAVES": 4, "PRX_UNROLL_BORN": 8, "PRX_UNROLL_FORCE": 4, "PRX_UNROLL_CHAIN": 8,
-            "PRX_XCD_MAP": 1, "PRX_ROT_BPERM_BORN": 0, "PRX_ROT_BPERM_FORCE": 0,
-            "PRX_ROT_BPERM_CHAIN": 0, "PRX_MIN_WAVES": 0}
+DEFAULTS = {"PRX_UNROLL_BORN": 1, "PRX_UNROLL_FORCE": 1, "PRX_UNROLL_CHAIN": 1, "PRX_XCD_MAP": 1,
+            "PRX_MIN_WAVES": 0}
 NOISE = 0.005
 
 
@@ -72,9 +67,8 @@ def current() -> dict:
 
 
 def name_of(settings: dict) -> str:
-    short = {"PRX_PAIR_WAVES": "w", "PRX_UNROLL_BORN": "ub", "PRX_UNROLL_FORCE": "uf", "PRX_UNROLL_CHAIN": "uc",
-             "PRX_XCD_MAP": "x", "PRX_ROT_BPERM_BORN": "bpb", "PRX_ROT_BPERM_FORCE": "bpf",
-             "PRX_ROT_BPERM_CHAIN": "bpc", "PRX_MIN_WAVES": "mw"}
+    short = {"PRX_UNROLL_BORN": "ub", "PRX_UNROLL_FORCE": "uf", "PRX_UNROLL_CHAIN": "uc", "PRX_XCD_MAP": "x",
+             "PRX_MIN_WAVES": "mw"}
     return "_".join(f"{short[k]}{settings[k]}" for k in KNOBS)
 
 
@@ -97,8 +91,8 @@ def header(settings: dict, note: str = "") -> str:
     lines += [f"// {l}" for l in note.splitlines() if l.strip()]
     lines.append("#pragma once")
     # guarded, so a -D on the compiler line (a tuning candidate) takes precedence
-    for k in KNOBS:
-        lines += [f"#ifndef {k}", f"#define {k} {settings[k]}", "#endif"]
+    for k, value in settings.items():
+        lines += [f"#ifndef {k}", f"#define {k} {value}", "#endif"]
     return "\n".join(lines) + "\n"
 
 
