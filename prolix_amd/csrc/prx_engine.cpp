@@ -359,10 +359,13 @@ struct prx_engine {
   // kFusedAutoAtoms atoms and none uses a neighbour list, else graphs: on
   // MI355X the fused kernel beats graphs only on systems of one tile. us a step,
   // fused / graphs: 64 atoms 32 / 43, 100 atoms 52 / 43, 138 atoms 77 / 44; 192
-  // systems of 64 atoms 34 / 47, of 100 atoms 57 / 54), 1 = captured graphs, 2 = the persistent kernel, 3 = the
-  // fused kernel (one workgroup per system)
+  // systems of 64 atoms 34 / 47, of 100 atoms 57 / 54), 1 = captured graphs,
+  // 2 = the persistent kernel, 3 = the fused kernel (one workgroup per system)
   int32_t step_mode = 0;
   static constexpr int32_t kFusedAutoAtoms = prx::kTile;
+  // Steps recorded into a caller's own graph: no step graph can be captured or
+  // launched there, but the fused kernel can run, and does up to this size.
+  static constexpr int32_t kFusedRecordAtoms = 3 * prx::kTile;
   int32_t max_system_atoms = 0;   // largest live system (rebuild)
   prx::GridBarrier* d_bar = nullptr;
   int persist_blocks = -1;        // co-resident grid of the persistent kernel (0: unavailable)
@@ -1139,8 +1142,13 @@ struct prx_engine {
 
   // The fused kernel: every system in one workgroup of its own. Not for
   // neighbour-list systems (their list build spans workgroups).
-  bool use_fused() const {
-    if (step_mode == 0) return !has_nl && max_system_atoms <= kFusedAutoAtoms;
+  bool use_fused(hipStream_t s) const {
+    if (step_mode == 0) {
+      if (has_nl || max_system_atoms > kFusedRecordAtoms) return false;
+      if (max_system_atoms <= kFusedAutoAtoms) return true;
+      hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+      return s != nullptr && hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusActive;
+    }
     if (step_mode != 3) return false;
     if (has_nl) throw StateError("the fused step kernel does not run neighbour-list systems");
     return true;
@@ -1175,7 +1183,7 @@ struct prx_engine {
         HIPCHECK(hipEventRecord(ev, s));
         HIPCHECK(hipStreamWaitEvent(stream, ev, 0));
       }
-      if (use_fused()) {
+      if (use_fused(s)) {
         for (int left = n_steps; left > 0;) {
           const int k = std::min(left, kPersistChunk);
           prx::launch_fused_steps(v, d_ranges, (int)order.size(), k, stream);
