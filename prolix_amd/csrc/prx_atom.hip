@@ -1,6 +1,7 @@
 // Per-atom kernels: Born-radius finish, chain-rule factors, BAOAB halves,
 // Philox noise, copies and deterministic per-system reductions.
 #include "prx_atom_dev.h"
+#include "prx_lanes_dev.h"
 
 namespace prx {
 // One block per tile: the gathers and finishes of prx_atom_dev.h.
@@ -48,11 +49,14 @@ __device__ double block_sum(double x, double* sh) {
 constexpr int kRangeInts = 14;
 
 // Energy reduction: one 1024-thread block per listed system. Each thread sums
-// its strided share of every term in index order (the work-item loop issues
-// four iterations' loads before their adds: the loop is bound by load
-// latency, not bandwidth), then the lanes of each wave are combined by a
-// fixed butterfly and the 16 waves in wave order, so the result is
-// deterministic.
+// its strided share of every term in index order, then each wave sums its 64
+// lanes' terms and the 16 waves' are added in wave order, so the result is
+// deterministic. Bound by load latency and, in small systems, by the sums over
+// lanes: the first element of every kind is loaded before any is added, later
+// ones four iterations at a time, and the lanes are summed by exchanges in which
+// a lane gives up half the terms it carries (wave_sum_terms; a butterfly per term
+// through LDS took 6 of the 11 us of a 138-atom system, now 3.7 us; 64 systems of
+// up to 5,000 atoms 19 us, now 12.7).
 constexpr int kEnThreads = 1024;
 constexpr int kEnWaves = kEnThreads / 64;
 
@@ -75,19 +79,64 @@ __device__ __forceinline__ void strided4(int b, int e, int t, K kind, E energy, 
   for (; k < e; k += kEnThreads) acc(kind(k), energy(k));
 }
 
-__device__ __forceinline__ double wave_sum_lane0(double x) {
-  for (int off = 32; off > 0; off >>= 1) x += __shfl_xor(x, off);
-  return x;  // lane 0's value is used
+// Sixteen terms summed over the wave: lanes 4 k to 4 k + 3 get term k.
+__device__ __forceinline__ double wave_sum_terms(const double (&v)[16], int lane) {
+  double h[8], g[4], f[2];
+#pragma unroll
+  for (int k = 0; k < 8; ++k) h[k] = add_swap<true>(v[k], v[k + 8]);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) g[k] = add_swap<false>(h[k], h[k + 4]);
+  const bool b3 = (lane & 8) != 0, b2 = (lane & 4) != 0;
+#pragma unroll
+  for (int k = 0; k < 2; ++k) f[k] = (b3 ? g[k + 2] : g[k]) + dpp<kDppRor8>(b3 ? g[k] : g[k + 2]);
+  double e = (b2 ? f[1] : f[0]) + dpp<kDppHalfMirror>(b2 ? f[0] : f[1]);
+  e += dpp<kDppXor2>(e);
+  return e + dpp<kDppXor1>(e);
 }
 
 __global__ __launch_bounds__(kEnThreads) void k_energy_reduce(DeviceView v, const int32_t* ranges,
                                                               double* out) {
   constexpr int kTerms = 12;
-  __shared__ double part[kTerms][kEnWaves];
+  __shared__ double part[16][kEnWaves];
+  __shared__ double sum[16];
   const int32_t* R = ranges + blockIdx.x * kRangeInts;
   const int t = threadIdx.x;
-  double e_gbp = 0, e_cl = 0, e_lj = 0;
-  int i = R[0] + t;
+  // the first element of each kind
+  const auto first = [&](int b, int e, auto load) {
+    if (b < e) load(min(b + t, e - 1));
+  };
+  double i0 = 0, i1 = 0, i2 = 0, s0 = 0, a0 = 0, xb = 0, xa = 0, xt = 0, xm = 0, xe = 0;
+  int zb = 0;
+  float zt = 0.0f;
+  first(R[0], R[1], [&](int k) {
+    i0 = v.e_items[(size_t)k * 3];
+    i1 = v.e_items[(size_t)k * 3 + 1];
+    i2 = v.e_items[(size_t)k * 3 + 2];
+  });
+  first(0, R[3], [&](int k) {
+    s0 = v.e_atom[(size_t)(R[2] + k) * 2];
+    a0 = v.e_atom[(size_t)(R[2] + k) * 2 + 1];
+  });
+  // A system's bonded ranges hold only its own entries (free entries lie
+  // outside every listed range), so no entry is tested for being free; the
+  // kind of a bond (bond / Urey-Bradley) and of a torsion entry (proper /
+  // improper) is read beside its energy.
+  first(R[4], R[5], [&](int k) { zb = v.bonds[k].idx.z; xb = v.e_bond[k]; });
+  first(R[6], R[7], [&](int k) { xa = v.e_angle[k]; });
+  first(R[8], R[9], [&](int k) { zt = v.tors[k].a.w; xt = v.e_tors[k]; });
+  first(R[10], R[11], [&](int k) { xm = v.e_cmap[k]; });
+  first(R[12], R[13], [&](int k) { xe = v.e_exc[k]; });
+
+  const bool in_i = R[0] + t < R[1], in_a = t < R[3], in_b = R[4] + t < R[5], in_t = R[8] + t < R[9];
+  double e_gbp = in_i ? i0 : 0.0, e_cl = in_i ? i1 : 0.0, e_lj = in_i ? i2 : 0.0;
+  double e_self = in_a ? s0 : 0.0, e_ace = in_a ? a0 : 0.0;
+  double e_bond = in_b && zb == 0 ? xb : 0.0, e_ub = in_b && zb != 0 ? xb : 0.0;
+  double e_ang = R[6] + t < R[7] ? xa : 0.0;
+  double e_dih = in_t && zt == 0.0f ? xt : 0.0, e_imp = in_t && zt != 0.0f ? xt : 0.0;
+  double e_cm = R[10] + t < R[11] ? xm : 0.0;
+  double e_ex = R[12] + t < R[13] ? xe : 0.0;
+
+  int i = R[0] + kEnThreads + t;
   for (; i + 3 * kEnThreads < R[1]; i += 4 * kEnThreads) {
     double a[4][3];
 #pragma unroll
@@ -106,45 +155,34 @@ __global__ __launch_bounds__(kEnThreads) void k_energy_reduce(DeviceView v, cons
     e_cl += v.e_items[(size_t)i * 3 + 1];
     e_lj += v.e_items[(size_t)i * 3 + 2];
   }
-  double e_self = 0, e_ace = 0;
-  for (int k = t; k < R[3]; k += kEnThreads) {
+  for (int k = t + kEnThreads; k < R[3]; k += kEnThreads) {
     e_self += v.e_atom[(size_t)(R[2] + k) * 2 + 0];
     e_ace += v.e_atom[(size_t)(R[2] + k) * 2 + 1];
   }
-  // A system's bonded ranges hold only its own entries (free entries lie
-  // outside every listed range), so no entry is tested for being free; the
-  // kind of a bond (bond / Urey-Bradley) and of a torsion entry (proper /
-  // improper) is read beside its energy. Four entries' loads per iteration.
-  double e_bond = 0, e_ub = 0;
-  strided4(R[4], R[5], t, [&](int k) { return v.bonds[k].idx.z; }, [&](int k) { return v.e_bond[k]; },
+  const int t1 = t + kEnThreads;
+  strided4(R[4], R[5], t1, [&](int k) { return v.bonds[k].idx.z; }, [&](int k) { return v.e_bond[k]; },
            [&](int z, double e) { if (z == 0) e_bond += e; else e_ub += e; });
-  double e_ang = 0;
-  strided4(R[6], R[7], t, [&](int) { return 0; }, [&](int k) { return v.e_angle[k]; },
+  strided4(R[6], R[7], t1, [&](int) { return 0; }, [&](int k) { return v.e_angle[k]; },
            [&](int, double e) { e_ang += e; });
-  double e_dih = 0, e_imp = 0;
-  strided4(R[8], R[9], t, [&](int k) { return v.tors[k].a.w == 0.0f ? 0 : 1; }, [&](int k) { return v.e_tors[k]; },
+  strided4(R[8], R[9], t1, [&](int k) { return v.tors[k].a.w == 0.0f ? 0 : 1; }, [&](int k) { return v.e_tors[k]; },
            [&](int z, double e) { if (z == 0) e_dih += e; else e_imp += e; });
-  double e_cm = 0;
-  strided4(R[10], R[11], t, [&](int) { return 0; }, [&](int k) { return v.e_cmap[k]; },
+  strided4(R[10], R[11], t1, [&](int) { return 0; }, [&](int k) { return v.e_cmap[k]; },
            [&](int, double e) { e_cm += e; });
-  double e_ex = 0;
-  strided4(R[12], R[13], t, [&](int) { return 0; }, [&](int k) { return v.e_exc[k]; },
+  strided4(R[12], R[13], t1, [&](int) { return 0; }, [&](int k) { return v.e_exc[k]; },
            [&](int, double e) { e_ex += e; });
-  const double mine[kTerms] = {e_bond, e_ang, e_ub, e_dih, e_imp, e_cm, e_lj, e_ex, e_gbp, e_self, e_cl, e_ace};
+  const double mine[16] = {e_bond, e_ang, e_ub, e_dih, e_imp, e_cm, e_lj, e_ex, e_gbp, e_self, e_cl, e_ace};
   const int lane = t & 63, wave = t >> 6;
+  const double w = wave_sum_terms(mine, lane);
+  if ((lane & 3) == 0) part[lane >> 2][wave] = w;
+  __syncthreads();
+  if (t < kTerms) {
+    double acc = 0.0;
 #pragma unroll
-  for (int k = 0; k < kTerms; ++k) {
-    const double w = wave_sum_lane0(mine[k]);
-    if (lane == 0) part[k][wave] = w;
+    for (int k = 0; k < kEnWaves; ++k) acc += part[t][k];
+    sum[t] = acc;
   }
   __syncthreads();
   if (t != 0) return;
-  double sum[kTerms];
-  for (int k = 0; k < kTerms; ++k) {
-    double acc = 0.0;
-    for (int w = 0; w < kEnWaves; ++w) acc += part[k][w];
-    sum[k] = acc;
-  }
   double terms[PRX_N_ENERGY];
   terms[PRX_E_BOND] = sum[0];
   terms[PRX_E_ANGLE] = sum[1];

@@ -27,6 +27,7 @@
 #pragma once
 
 #include "prx_common.h"
+#include "prx_lanes_dev.h"
 #include "prx_obc_farfield.h"
 
 namespace prx {
@@ -97,15 +98,6 @@ __device__ __forceinline__ float4 pad_pos(int lane) { return make_float4(1e15f +
 // ---------------------------------------------------------------------------
 // Cross-lane sums
 // ---------------------------------------------------------------------------
-template <int CTRL>
-__device__ __forceinline__ float dpp(float x) {
-  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
-}
-constexpr int kDppHalfMirror = 0x141;  // lane p of 8 reads lane 7 - p
-constexpr int kDppXor2 = 0x4E;         // quad_perm [2, 3, 0, 1]
-constexpr int kDppXor1 = 0xB1;         // quad_perm [1, 0, 3, 2]
-constexpr int kDppRor8 = 0x128;        // lane l of 16 reads lane l + 8 mod 16
-
 // Sum over the eight lanes p; every lane gets it.
 __device__ __forceinline__ float sum_p(float x) {
   x += dpp<kDppHalfMirror>(x);
@@ -125,17 +117,6 @@ __device__ __forceinline__ float sum_p4(float c0, float c1, float c2, float c3, 
   const float r = (mid ? r1 : r0) + dpp<kDppXor2>(mid ? r0 : r1);
   return r + dpp<kDppXor1>(r);
 }
-// x and y with their halves (of 64 lanes) or rows of 16 exchanged:
-// swap32: (x.lo, y.lo), (x.hi, y.hi); swap16: the same within each half.
-__device__ __forceinline__ float add_swap32(float x, float y) {
-  const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-__device__ __forceinline__ float add_swap16(float x, float y) {
-  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
-  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
-}
-
 // Sums over the eight lane groups q of the eight columns v[a] of lane p: lane
 // 8 q + p gets the sum of column a = q, which is atom (lane) of the tile.
 __device__ __forceinline__ float sum_q(const float (&v)[kEdge], int lane) {
@@ -822,30 +803,12 @@ struct ForceSum {
 
 // Three doubles summed over the wave, in the lanes of ForceSum::e: each
 // exchange puts two values' sums into the halves of one register.
-template <bool HALF>
-__device__ __forceinline__ double add_swap(double x, double y) {
-  const auto swap = [](unsigned p, unsigned q) {
-    if constexpr (HALF)
-      return __builtin_amdgcn_permlane32_swap(p, q, false, false);
-    else
-      return __builtin_amdgcn_permlane16_swap(p, q, false, false);
-  };
-  const auto lo = swap((unsigned)__double2loint(x), (unsigned)__double2loint(y));
-  const auto hi = swap((unsigned)__double2hiint(x), (unsigned)__double2hiint(y));
-  return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
-}
-template <int CTRL>
-__device__ __forceinline__ double add_dpp(double x) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(x), CTRL, 0xF, 0xF, true);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(x), CTRL, 0xF, 0xF, true);
-  return x + __hiloint2double(hi, lo);
-}
 __device__ __forceinline__ double sum_energies(double gb, double cl, double lj) {
   double e = add_swap<false>(add_swap<true>(gb, cl), add_swap<true>(lj, lj));
-  e = add_dpp<kDppRor8>(e);
-  e = add_dpp<kDppRor8 - 4>(e);
-  e = add_dpp<kDppRor8 - 6>(e);
-  return add_dpp<kDppRor8 - 7>(e);
+  e += dpp<kDppRor8>(e);
+  e += dpp<kDppRor8 - 4>(e);
+  e += dpp<kDppRor8 - 6>(e);
+  return e + dpp<kDppRor8 - 7>(e);
 }
 
 // What the pass takes from its system's constants and its item.
