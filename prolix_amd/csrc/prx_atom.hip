@@ -5,10 +5,10 @@
 
 namespace prx {
 // One block per tile: the gathers and finishes of prx_atom_dev.h.
-__global__ __launch_bounds__(256) void k_born_gather(DeviceView v) {
+__global__ __launch_bounds__(256) void k_born_gather(DeviceView v, float* out) {
   __shared__ GatherLds G;
   if ((int)blockIdx.x >= v.n_tiles) return;
-  born_gather_tile(v, blockIdx.x, G);
+  born_gather_tile(v, blockIdx.x, G, out);
 }
 
 template <bool ENERGY>
@@ -18,10 +18,10 @@ __global__ __launch_bounds__(256) void k_force_gather(DeviceView v) {
   force_gather_tile<ENERGY>(v, blockIdx.x, G);
 }
 
-__global__ __launch_bounds__(256) void k_chain_gather(DeviceView v, int mode) {
+__global__ __launch_bounds__(256) void k_chain_gather(DeviceView v, int mode, float* out) {
   __shared__ GatherLds G;
   if ((int)blockIdx.x >= v.n_tiles) return;
-  chain_gather_tile(v, blockIdx.x, mode, G);
+  chain_gather_tile(v, blockIdx.x, mode, G, out);
 }
 
 __global__ void k_step_begin(DeviceView v) { step_begin_atom(v, blockIdx.x * blockDim.x + threadIdx.x); }
@@ -267,13 +267,6 @@ __global__ __launch_bounds__(kRedThreads) void k_init_momenta(DeviceView v, cons
 }
 
 // map[p] = arena index of packed atom p.
-__global__ void k_copy_in_pos(DeviceView v, const float* src, const int32_t* map, int n) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  const int g = map[p];
-  v.pos[g] = make_float4(src[3 * p], src[3 * p + 1], src[3 * p + 2], 0.0f);
-}
-
 __global__ void k_copy_in_mom(DeviceView v, const float* src, const int32_t* map, int n) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
@@ -292,12 +285,6 @@ __global__ void k_copy_out(DeviceView v, float* pos, float* mom, float* frc, con
   if (frc) { const float4 a = v.force[g]; frc[3 * p] = a.x; frc[3 * p + 1] = a.y; frc[3 * p + 2] = a.z; }
 }
 
-__global__ void k_born_out(DeviceView v, float* out, const int32_t* map, int n) {
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= n) return;
-  out[p] = v.gb4[map[p]].x;
-}
-
 static inline dim3 atom_grid(int n) { return dim3((n + 255) / 256); }
 
 static inline dim3 tile_grid(int n_tiles) { return dim3((n_tiles + 3) / 4); }  // one wave per tile
@@ -313,12 +300,22 @@ __global__ __launch_bounds__(256) void k_tile_boxes(DeviceView v) {
   tile_box_wave(v, t);
 }
 
+// The same, with the positions brought in from the caller's packed array on the
+// way. With the forces and radii written by the gathers that form them and the
+// bonded terms in the Born pass's launch, an evaluation takes 7 launches (8 with
+// energies) instead of 12, which bound the small ones.
+__global__ __launch_bounds__(256) void k_positions_in(DeviceView v, const float* packed) {
+  const int t = gather_wave();
+  if (t >= v.n_tiles) return;
+  tile_box_wave(v, t, packed);
+}
+
 void launch_tile_boxes(const DeviceView& v, hipStream_t s) {
   if (v.n_tiles) hipLaunchKernelGGL(k_tile_boxes, tile_grid(v.n_tiles), dim3(256), 0, s, v);
 }
 
-void launch_born_gather(const DeviceView& v, hipStream_t s) {
-  if (v.n_tiles) hipLaunchKernelGGL(k_born_gather, gather_grid(v.n_tiles), dim3(256), 0, s, v);
+void launch_born_gather(const DeviceView& v, float* packed_radii, hipStream_t s) {
+  if (v.n_tiles) hipLaunchKernelGGL(k_born_gather, gather_grid(v.n_tiles), dim3(256), 0, s, v, packed_radii);
 }
 void launch_force_gather(const DeviceView& v, bool energy, hipStream_t s) {
   if (!v.n_tiles) return;
@@ -327,8 +324,11 @@ void launch_force_gather(const DeviceView& v, bool energy, hipStream_t s) {
   else
     hipLaunchKernelGGL(k_force_gather<false>, gather_grid(v.n_tiles), dim3(256), 0, s, v);
 }
-void launch_chain_gather(const DeviceView& v, int mode, hipStream_t s) {
-  if (v.n_tiles) hipLaunchKernelGGL(k_chain_gather, gather_grid(v.n_tiles), dim3(256), 0, s, v, mode);
+void launch_positions_in(const DeviceView& v, const float* packed, hipStream_t s) {
+  if (v.n_tiles) hipLaunchKernelGGL(k_positions_in, tile_grid(v.n_tiles), dim3(256), 0, s, v, packed);
+}
+void launch_chain_gather(const DeviceView& v, int mode, float* packed_forces, hipStream_t s) {
+  if (v.n_tiles) hipLaunchKernelGGL(k_chain_gather, gather_grid(v.n_tiles), dim3(256), 0, s, v, mode, packed_forces);
 }
 void launch_step_begin(const DeviceView& v, hipStream_t s) {
   if (v.atom_hw) hipLaunchKernelGGL(k_step_begin, atom_grid(v.atom_hw), dim3(256), 0, s, v);
@@ -357,10 +357,6 @@ void launch_recenter_com(const DeviceView& v, const int32_t* ranges, int n_slots
 void launch_init_momenta(const DeviceView& v, const int32_t* slot_list, int n, hipStream_t s) {
   if (n) hipLaunchKernelGGL(k_init_momenta, dim3(n), dim3(kRedThreads), 0, s, v, slot_list);
 }
-void launch_copy_in_positions(const DeviceView& v, const float* src, const int32_t* map, int n,
-                              hipStream_t s) {
-  if (n) hipLaunchKernelGGL(k_copy_in_pos, atom_grid(n), dim3(256), 0, s, v, src, map, n);
-}
 __global__ void k_fill_u32(uint32_t* dst, uint32_t value, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) dst[i] = value;
@@ -376,9 +372,6 @@ void launch_copy_in_momenta(const DeviceView& v, const float* src, const int32_t
 void launch_copy_out(const DeviceView& v, float* pos, float* mom, float* frc, const int32_t* map, int n,
                      hipStream_t s) {
   if (n) hipLaunchKernelGGL(k_copy_out, atom_grid(n), dim3(256), 0, s, v, pos, mom, frc, map, n);
-}
-void launch_born_out(const DeviceView& v, float* out, const int32_t* map, int n, hipStream_t s) {
-  if (n) hipLaunchKernelGGL(k_born_out, atom_grid(n), dim3(256), 0, s, v, out, map, n);
 }
 
 }  // namespace prx

@@ -302,9 +302,15 @@ __device__ __forceinline__ bool tile_done(const DeviceView& v, int t) {
   return S.step_limit != 0u && slot_done(S, v.atom_step[tl.x]);
 }
 
+// Packed index of a tile's atom (c.lane) in its caller's arrays.
+__device__ __forceinline__ size_t packed_index(const DeviceView& v, const TileCtx& c) {
+  const SlotConst& S = v.slots[c.slot];
+  return (size_t)(S.pack0 + (c.g - S.a0));
+}
+
 // B_i from I_i in FP64 (generalized_born.py:81-93); dB/dI for the chain rule.
 // Neighbour-list GB systems floor 1/B at 1e-4 (generalized_born.py:333-337).
-__device__ __forceinline__ void born_gather_tile(const DeviceView& v, int t, GatherLds& G) {
+__device__ __forceinline__ void born_gather_tile(const DeviceView& v, int t, GatherLds& G, float* out = nullptr) {
   if (tile_done(v, t)) return;
   const TileCtx c = tile_ctx(v, t);
   const double I = combine1(gather1(v, c), c, G);
@@ -319,6 +325,7 @@ __device__ __forceinline__ void born_gather_tile(const DeviceView& v, int t, Gat
   const double B = 1.0 / inv_b;
   const double dBdI = floored ? 0.0 : B * B * (1.0 - th * th) * (1.0 + psi * (-1.6 + 14.55 * psi)) * f.x / f.y;
   v.gb4[c.g] = make_float4((float)B, (float)(0.6005612043932249 / B), (float)dBdI, 0.0f);  // sqrt(log2(e)/4)/B
+  if (out) out[packed_index(v, c)] = (float)B;
 }
 
 // Pair force and dE/dB; c_i = dE/dB_i * dB_i/dI_i with the GB self term and ACE (FP64).
@@ -418,7 +425,7 @@ __device__ __forceinline__ float4 begin_step(const DeviceView& v, const SlotCons
 // then mode -1: store it; 2: B(F) and count the step; 1: B(F), then B A O A.
 // Returns the atom's position after the call.
 __device__ __forceinline__ float4 finish_atom(const DeviceView& v, const TileCtx& c, const double4& a,
-                                              const float4 (*shb)[kTile], int mode) {
+                                              const float4 (*shb)[kTile], int mode, float* out) {
   float3 fb = make_float3(0.f, 0.f, 0.f);
 #pragma unroll
   for (int k = 0; k < kGW; ++k) {
@@ -440,7 +447,12 @@ __device__ __forceinline__ float4 finish_atom(const DeviceView& v, const TileCtx
       if (mode >= 0) atomicAdd(&v.warn[c.slot * kWarnStride + kWarnForceCap], 1u);
     }
   }
-  v.force[c.g] = make_float4(f.x, f.y, f.z, 0.0f);
+  if (out) {
+    float* o = out + 3 * packed_index(v, c);
+    o[0] = f.x; o[1] = f.y; o[2] = f.z;
+  } else {
+    v.force[c.g] = make_float4(f.x, f.y, f.z, 0.0f);
+  }
   if (mode < 0 || !S.active) return v.pos[c.g];
   const uint32_t prev = v.atom_step[c.g];  // each lane owns its atom's counter
   if (slot_done(S, prev)) return v.pos[c.g];
@@ -462,8 +474,9 @@ __device__ __forceinline__ float4 finish_atom(const DeviceView& v, const TileCtx
 // finish each atom's force (finish_atom). In mode 1 the tile's atoms have
 // moved to the next step's positions, and wave 0 also writes the tile's box
 // for that step (what k_tile_boxes computes), so the step graph needs no box
-// kernel after its first step.
-__device__ __forceinline__ void chain_gather_tile(const DeviceView& v, int t, int mode, GatherLds& G) {
+// kernel after its first step. out: the forces go there, packed, instead of v.force.
+__device__ __forceinline__ void chain_gather_tile(const DeviceView& v, int t, int mode, GatherLds& G,
+                                                  float* out = nullptr) {
   if (tile_done(v, t)) return;
   const TileCtx c = tile_ctx(v, t);
   double4 part = gather3(v, c);
@@ -473,7 +486,7 @@ __device__ __forceinline__ void chain_gather_tile(const DeviceView& v, int t, in
   const double4 a = combine4(part, c, G);
   if (c.q != 0) return;
   float4 x = make_float4(0.f, 0.f, 0.f, 0.f);
-  if (c.valid) x = finish_atom(v, c, a, G.shb, mode);
+  if (c.valid) x = finish_atom(v, c, a, G.shb, mode, out);
   if (mode != 1 || !v.slots[c.slot].active) return;  // uniform over the tile
   const int last = v.tiles[t].y - 1;
   const float xl = __shfl(x.x, last), yl = __shfl(x.y, last), zl = __shfl(x.z, last);
@@ -508,12 +521,21 @@ __device__ __forceinline__ void step_begin_atom(const DeviceView& v, int g) {
 }
 
 // Bounding box of tile t's atoms at the current positions, with the tile's
-// largest offset radius rho and descreening radius s; one wave.
-__device__ __forceinline__ void tile_box_wave(const DeviceView& v, int t) {
+// largest offset radius rho and descreening radius s; one wave. packed: the
+// positions come from there and are stored in v.pos.
+__device__ __forceinline__ void tile_box_wave(const DeviceView& v, int t, const float* packed = nullptr) {
   const int4 tl = v.tiles[t];
   const int lane = threadIdx.x & 63;
-  const int g = tl.x + min(lane, tl.y - 1);
-  const float4 p = v.pos[g], b = v.born4[g];
+  const int l = min(lane, tl.y - 1), g = tl.x + l;
+  const float4 b = v.born4[g];
+  float4 p;
+  if (packed) {
+    const float* x = packed + 3 * (size_t)(v.slots[tl.z].pack0 + tl.w * kTile + l);
+    p = make_float4(x[0], x[1], x[2], 0.0f);
+    if (lane == l) v.pos[g] = p;
+  } else {
+    p = v.pos[g];
+  }
   float lx = p.x, ly = p.y, lz = p.z, hx = p.x, hy = p.y, hz = p.z, mr = b.x, ms = b.y;
   for (int off = 32; off > 0; off >>= 1) {
     lx = fminf(lx, __shfl_xor(lx, off));

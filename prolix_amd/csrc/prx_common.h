@@ -104,6 +104,7 @@ struct SlotConst {
   int32_t tile0;        // global index of the system's first tile
   uint64_t seed;
   int32_t unit0, n_units;  // the system's units
+  int32_t pack0;        // packed index of the system's first atom
   // neighbour-list systems (gb_cut with a cutoff): list build and reuse
   int32_t nl;           // 1: pair work from the list (chunk items), 0: all tile pairs
   int32_t tp_base;      // global index of the system's first tile pair (I < J) record
@@ -250,6 +251,8 @@ struct GridBarrier {
 
 // Launchers (defined in the .hip translation units).
 void launch_tile_boxes(const DeviceView& v, hipStream_t s);                // -> tbox (every evaluation)
+// Packed positions -> pos, and launch_tile_boxes.
+void launch_positions_in(const DeviceView& v, const float* packed, hipStream_t s);
 // Neighbour-list build of the gb_cut systems (after the tile boxes): with
 // force, every list is rebuilt; otherwise those whose atoms moved more than
 // skin / 2 since their last build (every list, when skin = 0).
@@ -258,20 +261,18 @@ void launch_nl_build(const DeviceView& v, const int32_t* slot_ranges, int n_slot
 void launch_dense_list(const float* pos, int n, float radius, int capacity, int32_t* idx, int32_t* counts,
                        float4* boxes, hipStream_t s);
 void launch_born_pairs(const DeviceView& v, hipStream_t s);                // also -> item_cls
-void launch_born_pairs_bonded(const DeviceView& v, hipStream_t s);         // the same, and launch_bonded (forces only)
-void launch_born_gather(const DeviceView& v, hipStream_t s);               // -> B, dB/dI
+void launch_born_pairs_bonded(const DeviceView& v, bool energy, hipStream_t s);  // the same, and launch_bonded
+void launch_born_gather(const DeviceView& v, float* packed_radii, hipStream_t s);  // -> B, dB/dI (radii out or nullptr)
 void launch_force_pairs(const DeviceView& v, bool energy, hipStream_t s);
 void launch_force_gather(const DeviceView& v, bool energy, hipStream_t s);  // -> chain factors, pair force
 void launch_chain_pairs(const DeviceView& v, hipStream_t s);
 void launch_bonded(const DeviceView& v, bool energy, hipStream_t s);
 // Sum chain partials + pair force + bonded records into the force, then
 //   mode -1: store the force only; 2: B(F), count the step; 1: B(F) then B A O A.
-void launch_chain_gather(const DeviceView& v, int mode, hipStream_t s);
+void launch_chain_gather(const DeviceView& v, int mode, float* packed_forces, hipStream_t s);  // nullptr: -> force
 void launch_step_begin(const DeviceView& v, hipStream_t s);  // B A O A from the stored force
 void launch_energy_reduce(const DeviceView& v, const int32_t* slot_ranges, int n_slots, double* out,
                           hipStream_t s);
-void launch_copy_in_positions(const DeviceView& v, const float* packed, const int32_t* map, int n,
-                              hipStream_t s);
 void launch_copy_out(const DeviceView& v, float* pos, float* mom, float* frc, const int32_t* map, int n,
                      hipStream_t s);
 void launch_copy_in_momenta(const DeviceView& v, const float* packed, const int32_t* map, int n,
@@ -291,6 +292,5 @@ int persist_max_blocks();
 void launch_fused_steps(const DeviceView& v, const int32_t* slot_ranges, int n_slots, int n_steps, hipStream_t s);
 hipError_t launch_persist_steps(const DeviceView& v, const int32_t* slot_ranges, int n_slots, int n_steps,
                                 bool has_nl, GridBarrier* bar, int n_blocks, hipStream_t s);
-void launch_born_out(const DeviceView& v, float* out, const int32_t* map, int n, hipStream_t s);
 
 }  // namespace prx

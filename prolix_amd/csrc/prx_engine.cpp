@@ -308,6 +308,16 @@ struct CmapCache {
 };
 CmapCache g_cmap_cache;
 
+namespace {
+// Packed arrays of the caller: positions to evaluate at (nullptr: those in
+// vv), forces (nullptr: left in vv) and Born radii out (nullptr: none).
+struct Packed {
+  const float* positions = nullptr;
+  float* forces = nullptr;
+  float* radii = nullptr;
+};
+}  // namespace
+
 // Pinned host memory from which a pool's admissions are copied to the device
 // asynchronously on the pool's stream. Reset only once those copies are done
 // (a synchronised stream).
@@ -936,6 +946,7 @@ struct prx_engine {
       const int nT = (s.n + prx::kTile - 1) / prx::kTile;
       const int32_t n_it = (int32_t)s.items.size();
       s.c.unit0 = (int32_t)units.size();
+      s.c.pack0 = offsets.back();
       all_cut = prx::append_units(s.items, ib, units) && all_cut;
       s.c.n_units = (int32_t)units.size() - s.c.unit0;
       push_const(sid, s.c);
@@ -1071,40 +1082,35 @@ struct prx_engine {
   // branch).
   // boxes = false when the previous chain gather (mode 1) already wrote the
   // tile boxes of the current positions.
-  void force_passes(const prx::DeviceView& vv, bool energy, hipStream_t s, bool boxes = true) {
+  void force_passes(const prx::DeviceView& vv, bool energy, hipStream_t s, bool boxes = true,
+                    const Packed& io = Packed()) {
     const bool fork = fork_bonded();
+    if (io.positions) prx::launch_positions_in(vv, io.positions, s);
     if (fork) {
       HIPCHECK(hipEventRecord(ev_fork, s));
       HIPCHECK(hipStreamWaitEvent(side, ev_fork, 0));
       prx::launch_bonded(vv, energy, side);
       HIPCHECK(hipEventRecord(ev_join, side));
     }
-    if (boxes) prx::launch_tile_boxes(vv, s);
+    if (boxes && !io.positions) prx::launch_tile_boxes(vv, s);
     // every list is rebuilt where the boxes are (eager evaluations, the first
     // step of a graph launch); later steps rebuild by the skin rule
     if (has_nl) prx::launch_nl_build(vv, d_ranges, (int)order.size(), boxes, s);
-    // in line, the bonded forces ride in the Born pass's launch (one graph
-    // node less per step); energy evaluations run the bonded kernel
-    const bool merged = !fork && !energy;
-    if (merged)
-      prx::launch_born_pairs_bonded(vv, s);
-    else
+    // in line, the bonded forces ride in the Born pass's launch
+    if (fork)
       prx::launch_born_pairs(vv, s);
-    prx::launch_born_gather(vv, s);
+    else
+      prx::launch_born_pairs_bonded(vv, energy, s);
+    prx::launch_born_gather(vv, io.radii, s);
     prx::launch_force_pairs(vv, energy, s);
     prx::launch_force_gather(vv, energy, s);
-    if (fork) {
-      prx::launch_chain_pairs(vv, s);
-      HIPCHECK(hipStreamWaitEvent(s, ev_join, 0));
-    } else {
-      if (!merged) prx::launch_bonded(vv, energy, s);
-      prx::launch_chain_pairs(vv, s);
-    }
+    prx::launch_chain_pairs(vv, s);
+    if (fork) HIPCHECK(hipStreamWaitEvent(s, ev_join, 0));
   }
 
-  void evaluate(const prx::DeviceView& vv, bool energy, hipStream_t s) {
-    force_passes(vv, energy, s);
-    prx::launch_chain_gather(vv, -1, s);
+  void evaluate(const prx::DeviceView& vv, bool energy, hipStream_t s, const Packed& io = Packed()) {
+    force_passes(vv, energy, s, true, io);
+    prx::launch_chain_gather(vv, -1, io.forces, s);
   }
   void evaluate(bool energy, hipStream_t s) { evaluate(v, energy, s); }
 
@@ -1125,7 +1131,7 @@ struct prx_engine {
       for (int k = 0; k < n_steps; ++k) {
         // after the first step, the previous chain gather wrote the boxes
         force_passes(sv, false, stream, k == 0);
-        prx::launch_chain_gather(sv, k + 1 == n_steps ? 2 : 1, stream);
+        prx::launch_chain_gather(sv, k + 1 == n_steps ? 2 : 1, nullptr, stream);
       }
       HIPCHECK(hipGetLastError());
     } catch (...) {
@@ -1393,14 +1399,10 @@ int prx_energy_forces(prx_engine* eng, const float* positions, float* forces, do
     need(eng && positions, "prx_energy_forces: bad arguments");
     eng->rebuild();
     hipStream_t s = eng->pick(stream);
-    const int n = eng->total_atoms();
     const prx::DeviceView ev = eng->eval_view();
-    prx::launch_copy_in_positions(ev, positions, eng->d_map, n, s);
-    eng->evaluate(ev, energies != nullptr, s);
+    eng->evaluate(ev, energies != nullptr, s, {positions, forces, born_radii});
     if (energies)
       prx::launch_energy_reduce(ev, eng->d_ranges, (int)eng->order.size(), energies, s);
-    if (forces) prx::launch_copy_out(ev, nullptr, nullptr, forces, eng->d_map, n, s);
-    if (born_radii) prx::launch_born_out(ev, born_radii, eng->d_map, n, s);
     HIPCHECK(hipGetLastError());
   });
 }
@@ -1453,13 +1455,9 @@ int prx_energy_forces_noalloc(const prx_system_desc* desc, const float* position
       eng.alloc_device(n_items, nT);  // CapacityError if the system does not fit
       eng.admit(d);
       eng.rebuild();
-      const int n = eng.total_atoms();
       const prx::DeviceView ev = eng.eval_view();
-      prx::launch_copy_in_positions(ev, positions, eng.d_map, n, s);
-      eng.evaluate(ev, energies != nullptr, s);
+      eng.evaluate(ev, energies != nullptr, s, {positions, forces, born_radii});
       if (energies) prx::launch_energy_reduce(ev, eng.d_ranges, 1, energies, s);
-      if (forces) prx::launch_copy_out(ev, nullptr, nullptr, forces, eng.d_map, n, s);
-      if (born_radii) prx::launch_born_out(ev, born_radii, eng.d_map, n, s);
       HIPCHECK(hipGetLastError());
       HIPCHECK(hipStreamSynchronize(s));
     } catch (...) {
@@ -1481,7 +1479,6 @@ int prx_integrator_init(prx_engine* eng, const float* positions, const float* mo
     HIPCHECK(hipStreamSynchronize(eng->stream));
     HIPCHECK(hipStreamSynchronize(s));
     eng->set_params(params);
-    prx::launch_copy_in_positions(eng->v, positions, eng->d_map, n, s);
     if (momenta) {
       prx::launch_copy_in_momenta(eng->v, momenta, eng->d_map, n, s);
       HIPCHECK(hipMemsetAsync(eng->v.atom_step, 0, eng->cap_atoms * sizeof(uint32_t), s));
@@ -1490,7 +1487,7 @@ int prx_integrator_init(prx_engine* eng, const float* positions, const float* mo
                               hipMemcpyHostToDevice, s));
       prx::launch_init_momenta(eng->v, eng->d_slot_list, (int)eng->order.size(), s);
     }
-    eng->evaluate(false, s);
+    eng->evaluate(eng->v, false, s, {positions, nullptr, nullptr});
     HIPCHECK(hipGetLastError());
     eng->initialized = true;
   });
@@ -1807,12 +1804,12 @@ int prx_profile_passes(prx_engine* eng, int32_t n_reps, double* ms) {
     prx::launch_tile_boxes(eng->v, s);
     if (eng->has_nl) prx::launch_nl_build(eng->v, eng->d_ranges, (int)eng->order.size(), true, s);
     timed(0, [&] { prx::launch_born_pairs(eng->v, s); });
-    timed(1, [&] { prx::launch_born_gather(eng->v, s); });
+    timed(1, [&] { prx::launch_born_gather(eng->v, nullptr, s); });
     timed(2, [&] { prx::launch_force_pairs(eng->v, false, s); });
     timed(3, [&] { prx::launch_force_gather(eng->v, false, s); });
     timed(4, [&] { prx::launch_chain_pairs(eng->v, s); });
     timed(5, [&] { prx::launch_bonded(eng->v, false, s); });
-    timed(6, [&] { prx::launch_chain_gather(eng->v, -1, s); });
+    timed(6, [&] { prx::launch_chain_gather(eng->v, -1, nullptr, s); });
     for (int k = 0; k < n_pass; ++k) {
       ms[k] /= n_reps;
       hipEventDestroy(ev[k][0]);
@@ -1869,13 +1866,13 @@ int prx_profile_steps(prx_engine* eng, int32_t n_steps, double* ms) {
           if (k == 0) prx::launch_tile_boxes(v, s);
           if (eng->has_nl) prx::launch_nl_build(v, eng->d_ranges, (int)eng->order.size(), k == 0, s);
           timed(0, s, [&] { prx::launch_born_pairs(v, s); });
-          timed(1, s, [&] { prx::launch_born_gather(v, s); });
+          timed(1, s, [&] { prx::launch_born_gather(v, nullptr, s); });
           timed(2, s, [&] { prx::launch_force_pairs(v, false, s); });
           timed(3, s, [&] { prx::launch_force_gather(v, false, s); });
           if (!fork) timed(5, s, [&] { prx::launch_bonded(v, false, s); });
           timed(4, s, [&] { prx::launch_chain_pairs(v, s); });
           if (fork) HIPCHECK(hipStreamWaitEvent(s, eng->ev_join, 0));
-          timed(6, s, [&] { prx::launch_chain_gather(v, k + 1 == n_steps ? 2 : 1, s); });
+          timed(6, s, [&] { prx::launch_chain_gather(v, k + 1 == n_steps ? 2 : 1, nullptr, s); });
         }
         HIPCHECK(hipGetLastError());
       } catch (...) {

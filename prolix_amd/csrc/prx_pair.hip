@@ -64,7 +64,7 @@ __global__ __launch_bounds__(kThreads<WAVES>) PRX_OCCUPANCY void k_chain_pairs(D
 // bonded records are read by the chain gather, so the merged launch saves the
 // bonded kernel's graph node where that kernel would run in line; results are
 // bit for bit those of the two kernels.
-template <int WAVES>
+template <int WAVES, bool ENERGY>
 __global__ __launch_bounds__(kThreads<WAVES>) PRX_OCCUPANCY void k_born_pairs_bonded(DeviceView v, int n_pair) {
   const int b = (int)blockIdx.x;
   if (b < n_pair) {
@@ -72,20 +72,28 @@ __global__ __launch_bounds__(kThreads<WAVES>) PRX_OCCUPANCY void k_born_pairs_bo
     return;
   }
   const int e = (b - n_pair) * kThreads<WAVES> + (int)threadIdx.x;
-  if (e < bonded_entries(v)) bonded_entry<false>(v, e);
+  if (e < bonded_entries(v)) bonded_entry<ENERGY>(v, e);
 }
 
 static inline bool by_wave(const DeviceView& v) { return v.n_items >= kWaveItems; }
 static inline int pair_blocks(const DeviceView& v) { return by_wave(v) ? v.n_items : v.n_units; }
 
-void launch_born_pairs_bonded(const DeviceView& v, hipStream_t s) {
+template <bool ENERGY>
+static void born_pairs_bonded(const DeviceView& v, hipStream_t s) {
   const int np = pair_blocks(v), nt = by_wave(v) ? kThreads<1> : kThreads<kUnitWaves>;
   const int nb = np + (bonded_entries(v) + nt - 1) / nt;
   if (nb == 0) return;
   if (by_wave(v))
-    hipLaunchKernelGGL(k_born_pairs_bonded<1>, dim3(nb), dim3(nt), 0, s, v, np);
+    hipLaunchKernelGGL((k_born_pairs_bonded<1, ENERGY>), dim3(nb), dim3(nt), 0, s, v, np);
   else
-    hipLaunchKernelGGL(k_born_pairs_bonded<kUnitWaves>, dim3(nb), dim3(nt), 0, s, v, np);
+    hipLaunchKernelGGL((k_born_pairs_bonded<kUnitWaves, ENERGY>), dim3(nb), dim3(nt), 0, s, v, np);
+}
+
+void launch_born_pairs_bonded(const DeviceView& v, bool energy, hipStream_t s) {
+  if (energy)
+    born_pairs_bonded<true>(v, s);
+  else
+    born_pairs_bonded<false>(v, s);
 }
 
 void launch_born_pairs(const DeviceView& v, hipStream_t s) {
