@@ -29,7 +29,7 @@ struct PairItem {
   int32_t meta;  // ni (bits 0-6), nj (bits 7-13), flags (bits 14-15), slot (bits 16-31)
   int32_t excl;  // exclusion-mask tile index, or -1
   int32_t ti, tj;  // global indices of the two tiles (a chunk item's ti is its row's; tj unused)
-  int32_t nsub;    // shares of the item (1, 2 or kUnitWaves, prx_pair_dev.h)
+  int32_t nsub;    // shares of the item (1, 2 or 4, prx_pair_dev.h)
   int32_t pad;
 };
 // Unit of the pair passes, the work of a group of kUnitWaves waves: the items
@@ -182,6 +182,7 @@ struct DeviceView {
   int32_t n_items;
   const PairUnit* units;  // nullptr: unit = item, every item cut
   int32_t n_units;
+  int32_t shares;  // of every item, or 0 where systems differ
   float4* part;        // partial sums, 2 * 64 float4 per item (part1 / part3 / part4 below)
   const int4* tiles;   // per tile: (first atom, atoms in tile, slot, tile index T)
   int32_t n_tiles;

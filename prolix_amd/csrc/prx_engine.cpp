@@ -935,7 +935,7 @@ struct prx_engine {
     std::vector<int2> nl_col;
     std::vector<int32_t> nl_colitems;
     offsets.assign(1, 0);
-    bool all_cut = true;
+    int32_t shares = -1;  // of every item so far, 0 where systems differ
     max_system_atoms = 0;
     has_nl = false;
     for (int32_t sid : order) {
@@ -947,7 +947,8 @@ struct prx_engine {
       const int32_t n_it = (int32_t)s.items.size();
       s.c.unit0 = (int32_t)units.size();
       s.c.pack0 = offsets.back();
-      all_cut = prx::append_units(s.items, ib, units) && all_cut;
+      const int32_t sh = prx::append_units(s.items, ib, units);
+      shares = shares < 0 || shares == sh ? sh : 0;
       s.c.n_units = (int32_t)units.size() - s.c.unit0;
       push_const(sid, s.c);
       for (int T = 0; T < nT; ++T) {
@@ -1029,7 +1030,8 @@ struct prx_engine {
     if (!map.empty()) HIPCHECK(hipMemcpy(d_map, map.data(), map.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     v.items = d_items;
     v.n_items = (int32_t)items.size();
-    v.units = all_cut ? nullptr : d_units;
+    v.units = shares == prx::kUnitWaves ? nullptr : d_units;
+    v.shares = std::max(shares, 0);
     v.n_units = (int32_t)units.size();
     v.e_items = d_e_items;
     v.part = d_part;

@@ -281,12 +281,12 @@ void build_items(int n_atoms, int a0, int slot, const ExclPlan& plan, int excl_b
     }
 }
 
-bool append_units(const std::vector<PairItem>& items, int base, std::vector<PairUnit>& out) {
-  if (items.empty()) return true;
+int append_units(const std::vector<PairItem>& items, int base, std::vector<PairUnit>& out) {
+  if (items.empty()) return 0;
   const int shares = items[0].nsub, per = kUnitWaves / shares, n = (int)items.size();
   for (int k = 0; k < n; k += per)
     out.push_back({base + k, (int16_t)std::min(per, n - k), (int16_t)shares});
-  return shares == kUnitWaves;
+  return shares;
 }
 
 namespace {

@@ -23,12 +23,15 @@
 // and the gathers). Far items skip LJ and Coulomb, and with the neighbour-list
 // GB form (generalized_born.py:266-415, gb_cut) skip every pass; straddling
 // items test r^2 < cutoff^2 per pair.
+#include <type_traits>
+
 #include "prx_bonded_dev.h"
 #include "prx_pair_dev.h"
 
 namespace prx {
 
-// Blocks of WAVES waves: 1 (an item each) or kUnitWaves (a unit each).
+// Blocks of WAVES waves: 1 (an item each), 2 (an item in two shares each) or
+// kUnitWaves (a unit each).
 template <int WAVES>
 constexpr int kThreads = 64 * WAVES;
 
@@ -38,8 +41,8 @@ __device__ __forceinline__ void pair_block(const DeviceView& v, int b, int nb) {
     __shared__ float4 mem[Pass::kLds];
     pair_wave<Pass>(v, unit_id(v, b, nb), mem);
   } else {
-    __shared__ UnitLds<Pass::kLds> mem;
-    pair_unit<false, Pass>(v, unit_id(v, b, nb), unit_wave(), mem);
+    __shared__ UnitLds<Pass::kLds, WAVES> mem;
+    pair_unit<false, Pass>(v, unit_id(v, b, nb), unit_wave<WAVES>(), mem);
   }
 }
 
@@ -75,18 +78,32 @@ __global__ __launch_bounds__(kThreads<WAVES>) PRX_OCCUPANCY void k_born_pairs_bo
   if (e < bonded_entries(v)) bonded_entry<ENERGY>(v, e);
 }
 
-static inline bool by_wave(const DeviceView& v) { return v.n_items >= kWaveItems; }
-static inline int pair_blocks(const DeviceView& v) { return by_wave(v) ? v.n_items : v.n_units; }
+// Waves per block: an item per wave in a long list or where every item is
+// whole, two per item where every item is in two shares, else units. Two-wave
+// blocks free their slots as soon as one item is done, and read no unit list:
+// 8,000 atoms 144 us an evaluation, 148 with units of two items.
+static inline int block_waves(const DeviceView& v) {
+  return v.n_items >= kWaveItems ? 1 : (v.shares > 0 ? v.shares : kUnitWaves);
+}
+static inline int pair_blocks(const DeviceView& v, int waves) { return waves < kUnitWaves ? v.n_items : v.n_units; }
+
+// launch(std::integral_constant<int, WAVES>) with the list's block_waves.
+template <class F>
+static void by_waves(const DeviceView& v, F&& launch) {
+  switch (block_waves(v)) {
+    case 1: return launch(std::integral_constant<int, 1>());
+    case 2: return launch(std::integral_constant<int, 2>());
+    default: return launch(std::integral_constant<int, kUnitWaves>());
+  }
+}
 
 template <bool ENERGY>
 static void born_pairs_bonded(const DeviceView& v, hipStream_t s) {
-  const int np = pair_blocks(v), nt = by_wave(v) ? kThreads<1> : kThreads<kUnitWaves>;
-  const int nb = np + (bonded_entries(v) + nt - 1) / nt;
-  if (nb == 0) return;
-  if (by_wave(v))
-    hipLaunchKernelGGL((k_born_pairs_bonded<1, ENERGY>), dim3(nb), dim3(nt), 0, s, v, np);
-  else
-    hipLaunchKernelGGL((k_born_pairs_bonded<kUnitWaves, ENERGY>), dim3(nb), dim3(nt), 0, s, v, np);
+  by_waves(v, [&](auto w) {
+    constexpr int W = decltype(w)::value, nt = kThreads<W>;
+    const int np = pair_blocks(v, W), nb = np + (bonded_entries(v) + nt - 1) / nt;
+    if (nb > 0) hipLaunchKernelGGL((k_born_pairs_bonded<W, ENERGY>), dim3(nb), dim3(nt), 0, s, v, np);
+  });
 }
 
 void launch_born_pairs_bonded(const DeviceView& v, bool energy, hipStream_t s) {
@@ -98,18 +115,18 @@ void launch_born_pairs_bonded(const DeviceView& v, bool energy, hipStream_t s) {
 
 void launch_born_pairs(const DeviceView& v, hipStream_t s) {
   if (v.n_items == 0) return;
-  if (by_wave(v))
-    hipLaunchKernelGGL(k_born_pairs<1>, dim3(pair_blocks(v)), dim3(kThreads<1>), 0, s, v);
-  else
-    hipLaunchKernelGGL(k_born_pairs<kUnitWaves>, dim3(pair_blocks(v)), dim3(kThreads<kUnitWaves>), 0, s, v);
+  by_waves(v, [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    hipLaunchKernelGGL(k_born_pairs<W>, dim3(pair_blocks(v, W)), dim3(kThreads<W>), 0, s, v);
+  });
 }
 
 template <bool ENERGY>
 static void force_pairs(const DeviceView& v, hipStream_t s) {
-  if (by_wave(v))
-    hipLaunchKernelGGL((k_force_pairs<1, ENERGY>), dim3(pair_blocks(v)), dim3(kThreads<1>), 0, s, v);
-  else
-    hipLaunchKernelGGL((k_force_pairs<kUnitWaves, ENERGY>), dim3(pair_blocks(v)), dim3(kThreads<kUnitWaves>), 0, s, v);
+  by_waves(v, [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    hipLaunchKernelGGL((k_force_pairs<W, ENERGY>), dim3(pair_blocks(v, W)), dim3(kThreads<W>), 0, s, v);
+  });
 }
 
 void launch_force_pairs(const DeviceView& v, bool energy, hipStream_t s) {
@@ -122,10 +139,10 @@ void launch_force_pairs(const DeviceView& v, bool energy, hipStream_t s) {
 
 void launch_chain_pairs(const DeviceView& v, hipStream_t s) {
   if (v.n_items == 0) return;
-  if (by_wave(v))
-    hipLaunchKernelGGL(k_chain_pairs<1>, dim3(pair_blocks(v)), dim3(kThreads<1>), 0, s, v);
-  else
-    hipLaunchKernelGGL(k_chain_pairs<kUnitWaves>, dim3(pair_blocks(v)), dim3(kThreads<kUnitWaves>), 0, s, v);
+  by_waves(v, [&](auto w) {
+    constexpr int W = decltype(w)::value;
+    hipLaunchKernelGGL(k_chain_pairs<W>, dim3(pair_blocks(v, W)), dim3(kThreads<W>), 0, s, v);
+  });
 }
 
 }  // namespace prx

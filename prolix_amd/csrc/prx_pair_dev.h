@@ -1259,17 +1259,20 @@ __device__ __forceinline__ void pair_wave(const DeviceView& v, int w, float4* L)
 
 // Workgroup memory of one group: per wave two tiles (used by the first wave of
 // each item) and the wave's scratch, which takes its column sums at the end.
-template <int N>
+template <int N, int WAVES = kUnitWaves>
 struct UnitLds {
-  float4 wave[kUnitWaves][N];
+  static constexpr int kWaves = WAVES;
+  float4 wave[WAVES][N];
 };
 
-// k: the wave's index in the group.
+// k: the wave's index in the group. Groups of kUnitWaves take the units of the
+// list, smaller ones the item of the unit's index, in as many shares.
 template <bool SYNC, class Pass, class Lds>
 __device__ __forceinline__ void pair_unit(const DeviceView& v, int unit, int k, Lds& L) {
-  const PairUnit u = v.units != nullptr ? v.units[unit] : PairUnit{unit, 1, kUnitWaves};
+  constexpr int W = Lds::kWaves;
+  const PairUnit u = W == kUnitWaves && v.units != nullptr ? v.units[unit] : PairUnit{unit, 1, W};
   const int sh = u.shares;
-  const int m = sh == kUnitWaves ? 0 : (sh == 1 ? k : k / 2), sub = k - m * sh;
+  const int m = sh == W ? 0 : (sh == 1 ? k : k / 2), sub = k - m * sh;
   const int w = u.first + m;
   float4* const tiles = L.wave[m * sh];
   float4* const own = L.wave[k] + 4 * kTile;
@@ -1322,9 +1325,10 @@ __device__ __forceinline__ int unit_id(const DeviceView& v, int b, int nb) {
   return b;
 }
 
-// Wave of this thread within its group of kUnitWaves (wave-uniform).
+// Wave of this thread within its group (wave-uniform).
+template <int WAVES = kUnitWaves>
 __device__ __forceinline__ int unit_wave() {
-  return __builtin_amdgcn_readfirstlane((int)((threadIdx.x >> 6) & (kUnitWaves - 1)));
+  return __builtin_amdgcn_readfirstlane((int)((threadIdx.x >> 6) & (WAVES - 1)));
 }
 
 }  // namespace prx
