@@ -52,7 +52,7 @@ __global__ __launch_bounds__(kThreads<WAVES>) PRX_OCCUPANCY void k_born_pairs(De
 }
 
 template <int WAVES, bool ENERGY>
-__global__ __launch_bounds__(kThreads<WAVES>) PRX_FORCE_OCCUPANCY(ENERGY) void k_force_pairs(DeviceView v) {
+__global__ __launch_bounds__(kThreads<WAVES>) PRX_FORCE_OCCUPANCY(WAVES, ENERGY) void k_force_pairs(DeviceView v) {
   pair_block<WAVES, ForcePass<ENERGY>>(v, blockIdx.x, gridDim.x);
 }
 

@@ -69,12 +69,14 @@ __device__ __forceinline__ void wave_lds_sync() {
 #endif
 #if PRX_MIN_WAVES > 0
 #define PRX_OCCUPANCY __attribute__((amdgpu_waves_per_eu(PRX_MIN_WAVES)))
-#define PRX_FORCE_OCCUPANCY(ENERGY) PRX_OCCUPANCY
+#define PRX_FORCE_OCCUPANCY(WAVES, ENERGY) PRX_OCCUPANCY
 #else
 #define PRX_OCCUPANCY
-// The force pass takes 96 VGPRs, 128 with energies, without a spill (its free
-// choice is 144: 64 systems of up to 5,000 atoms 526 us an evaluation, 519 with 128).
-#define PRX_FORCE_OCCUPANCY(ENERGY) __attribute__((amdgpu_waves_per_eu(ENERGY ? 4 : 5)))
+// The force pass: four waves per SIMD where a wave takes an item, five where
+// work lists are short (256 systems of 300 to 5,000 atoms 613 and 628 us, one of
+// 8,000 atoms 49.5 and 48.0), without a spill. With energies four (128 VGPRs; its
+// free choice is 144: 64 systems of up to 5,000 atoms 526 us an evaluation, 519).
+#define PRX_FORCE_OCCUPANCY(WAVES, ENERGY) __attribute__((amdgpu_waves_per_eu(ENERGY || WAVES == 1 ? 4 : 5)))
 #endif
 #define PRX_PRAGMA(x) _Pragma(#x)
 #define PRX_UNROLL(n) PRX_PRAGMA(unroll n)
