@@ -257,7 +257,8 @@ void launch_positions_in(const DeviceView& v, const float* packed, hipStream_t s
 // Neighbour-list build of the gb_cut systems (after the tile boxes): with
 // force, every list is rebuilt; otherwise those whose atoms moved more than
 // skin / 2 since their last build (every list, when skin = 0).
-void launch_nl_build(const DeviceView& v, const int32_t* slot_ranges, int n_slots, bool force, hipStream_t s);
+void launch_nl_build(const DeviceView& v, const int32_t* slot_ranges, int n_slots, bool force, bool skins,
+                     hipStream_t s);  // skins: a listed system has one
 // Dense per-atom neighbour lists of raw (n, 3) positions (prx_neighbor_list_dense).
 void launch_dense_list(const float* pos, int n, float radius, int capacity, int32_t* idx, int32_t* counts,
                        float4* boxes, hipStream_t s);

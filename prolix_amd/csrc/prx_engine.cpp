@@ -365,6 +365,7 @@ struct prx_engine {
   int32_t* d_nl_colitems = nullptr;
   int64_t cap_colitems = 0;
   bool has_nl = false;            // a live system uses its neighbour list
+  bool has_skin = false;          // and one of these has a skin
   // step path: 0 = auto (the fused kernel when every system fits in
   // kFusedAutoAtoms atoms and none uses a neighbour list, else graphs: on
   // MI355X the fused kernel beats graphs only on systems of one tile. us a step,
@@ -937,7 +938,7 @@ struct prx_engine {
     offsets.assign(1, 0);
     int32_t shares = -1;  // of every item so far, 0 where systems differ
     max_system_atoms = 0;
-    has_nl = false;
+    has_nl = has_skin = false;
     for (int32_t sid : order) {
       Slot& s = slots[sid];
       const int32_t ib = (int32_t)items.size();
@@ -964,6 +965,7 @@ struct prx_engine {
         }
       }
       has_nl = has_nl || s.nl;
+      has_skin = has_skin || (s.nl && s.c.skin_half2 > 0.0f);
       items.insert(items.end(), s.items.begin(), s.items.end());
       for (size_t k = items.size() - s.items.size(); k < items.size(); ++k) {
         items[k].ti += s.c.tile0;
@@ -1097,7 +1099,7 @@ struct prx_engine {
     if (boxes && !io.positions) prx::launch_tile_boxes(vv, s);
     // every list is rebuilt where the boxes are (eager evaluations, the first
     // step of a graph launch); later steps rebuild by the skin rule
-    if (has_nl) prx::launch_nl_build(vv, d_ranges, (int)order.size(), boxes, s);
+    if (has_nl) prx::launch_nl_build(vv, d_ranges, (int)order.size(), boxes, has_skin, s);
     // in line, the bonded forces ride in the Born pass's launch
     if (fork)
       prx::launch_born_pairs(vv, s);
@@ -1625,6 +1627,9 @@ int prx_engine_set_nl_skin(prx_engine* eng, double skin) {
       sl.c.nl_cut2 = (float)(rl * rl * 1.00001);
       sl.c.skin_half2 = (float)(0.25 * skin * skin);
       eng->push_const(sid, sl.c);
+      const bool has = sl.c.skin_half2 > 0.0f;  // the same for every list system
+      if (has != eng->has_skin) eng->drop_graphs();
+      eng->has_skin = has;
     }
   });
 }
@@ -1804,7 +1809,7 @@ int prx_profile_passes(prx_engine* eng, int32_t n_reps, double* ms) {
       ms[k] = t;
     };
     prx::launch_tile_boxes(eng->v, s);
-    if (eng->has_nl) prx::launch_nl_build(eng->v, eng->d_ranges, (int)eng->order.size(), true, s);
+    if (eng->has_nl) prx::launch_nl_build(eng->v, eng->d_ranges, (int)eng->order.size(), true, eng->has_skin, s);
     timed(0, [&] { prx::launch_born_pairs(eng->v, s); });
     timed(1, [&] { prx::launch_born_gather(eng->v, nullptr, s); });
     timed(2, [&] { prx::launch_force_pairs(eng->v, false, s); });
@@ -1866,7 +1871,7 @@ int prx_profile_steps(prx_engine* eng, int32_t n_steps, double* ms) {
             HIPCHECK(hipEventRecord(eng->ev_join, eng->side));
           }
           if (k == 0) prx::launch_tile_boxes(v, s);
-          if (eng->has_nl) prx::launch_nl_build(v, eng->d_ranges, (int)eng->order.size(), k == 0, s);
+          if (eng->has_nl) prx::launch_nl_build(v, eng->d_ranges, (int)eng->order.size(), k == 0, eng->has_skin, s);
           timed(0, s, [&] { prx::launch_born_pairs(v, s); });
           timed(1, s, [&] { prx::launch_born_gather(v, nullptr, s); });
           timed(2, s, [&] { prx::launch_force_pairs(v, false, s); });

@@ -1,5 +1,5 @@
-// Device code of the neighbour-list build, shared by prx_nl.hip (three
-// kernels) and prx_persist.hip. See prx_nl.hip for the algorithm.
+// Device code of the neighbour-list build, shared by prx_nl.hip
+// and prx_persist.hip. See prx_nl.hip for the algorithm.
 #pragma once
 
 #include "prx_common.h"
@@ -15,18 +15,14 @@ __device__ __forceinline__ unsigned long long nl_below(int lane) {
 }
 
 // Listed system k, by one block of kNlThreads threads.
-__device__ __forceinline__ void nl_check_block(const DeviceView& v, const int32_t* ranges, int k, int force) {
+__device__ __forceinline__ void nl_check_block(const DeviceView& v, const int32_t* ranges, int k) {
   __shared__ float sh[kNlThreads];
   const int32_t* R = ranges + k * kRangeInts;
   const int a0 = R[2], n = R[3];
   if (n <= 0) return;
   const int slot = v.slot_of[a0];
   const SlotConst& S = v.slots[slot];
-  if (!S.nl) return;
-  if (force || S.skin_half2 <= 0.0f) {
-    if (threadIdx.x == 0) v.nl_flag[slot] = 1;
-    return;
-  }
+  if (!S.nl || S.skin_half2 <= 0.0f) return;  // without a skin the list is built every time
   float m = 0.0f;
   auto take = [&](const float4& x, const float4& r) {
     const float dx = x.x - r.x, dy = x.y - r.y, dz = x.z - r.z;
@@ -55,83 +51,100 @@ __device__ __forceinline__ void nl_check_block(const DeviceView& v, const int32_
   if (threadIdx.x == 0) v.nl_flag[slot] = sh[0] > S.skin_half2 ? 1 : 0;
 }
 
-// Tile-pair record w, by one wave.
-__device__ __forceinline__ void nl_mask_wave(const DeviceView& v, int w) {
-  const TilePairInfo tp = v.nl_tp[w];
-  if (tp.ij < 0) return;  // a free record
-  const bool excl = tp.slot < 0;
-  const int slot = excl ? ~tp.slot : tp.slot;
-  if (!v.nl_flag[slot]) return;
-  const int lane = threadIdx.x & 63;
-  if (excl) {  // an ordinary item covers this tile pair
-    if (lane == 0) v.nl_mask[w] = 0ull;
-    return;
-  }
-  const SlotConst& S = v.slots[slot];
-  const int I = tp.ij & 0xFFFF, J = tp.ij >> 16;
-  const int tI = S.tile0 + I, tJ = S.tile0 + J;
-  const float4 li = v.tbox[2 * tI], hi = v.tbox[2 * tI + 1];
-  const float4 lj = v.tbox[2 * tJ], hj = v.tbox[2 * tJ + 1];
-  const float bx = fmaxf(0.0f, fmaxf(lj.x - hi.x, li.x - hj.x));
-  const float by = fmaxf(0.0f, fmaxf(lj.y - hi.y, li.y - hj.y));
-  const float bz = fmaxf(0.0f, fmaxf(lj.z - hi.z, li.z - hj.z));
-  if (bx * bx + by * by + bz * bz >= S.nl_cut2) {  // wave-uniform: no atom of J is in range
-    if (lane == 0) v.nl_mask[w] = 0ull;
-    return;
-  }
-  const int nJ = min(kTile, S.n - J * kTile);
-  const float4 p = v.pos[S.a0 + J * kTile + min(lane, nJ - 1)];
-  const float gx = fmaxf(0.0f, fmaxf(li.x - p.x, p.x - hi.x));
-  const float gy = fmaxf(0.0f, fmaxf(li.y - p.y, p.y - hi.y));
-  const float gz = fmaxf(0.0f, fmaxf(li.z - p.z, p.z - hi.z));
-  const bool in = lane < nJ && gx * gx + gy * gy + gz * gz < S.nl_cut2;
-  const unsigned long long m = __ballot(in);
-  if (lane == 0) v.nl_mask[w] = m;
-}
-
-// Tile t's row, by one wave: the exclusive prefix of the entry counts of its
-// tile pairs (I, J > I) in J order, the row's total, and for a list with a
-// skin the reference positions of the tile's atoms.
-__device__ __forceinline__ void nl_rows_wave(const DeviceView& v, int t) {
+// Tile t's list, by one block: the masks of its tile pairs (I, J > I), their
+// prefix counts, the row's total, the entries, and with a skin the reference
+// positions of the tile's atoms. THREADS tile pairs a round: a thread each for
+// the box test, the pairs in range then dealt to the waves, four loads in flight,
+// and their entries written from the masks in LDS.
+template <int THREADS>
+__device__ __forceinline__ void nl_row_block(const DeviceView& v, int t, int force) {
+  __shared__ unsigned long long masks[THREADS];
+  __shared__ int prefs[THREADS];
+  __shared__ int near[THREADS];
+  __shared__ int totals[THREADS / 64];
+  __shared__ int n_near;
+  constexpr int kWaves = THREADS / 64, kBatch = 4;
   const int4 tl = v.tiles[t];
   const int slot = tl.z;
   const SlotConst& S = v.slots[slot];
-  if (!S.nl || !v.nl_flag[slot]) return;
-  const int lane = threadIdx.x & 63;
+  if (!S.nl || !(force || S.skin_half2 <= 0.0f || v.nl_flag[slot])) return;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int I = tl.w;
   const int nT = (S.n + kTile - 1) / kTile;
   const int tp0 = S.tp_base + I * (nT - 1) - (I * (I - 1)) / 2;  // record of (I, I + 1)
+  const int entry0 = v.nl_row[t].y;
+  const float4 li = v.tbox[2 * t], hi = v.tbox[2 * t + 1];
+  if (S.skin_half2 > 0.0f && tid < tl.y) v.nl_xref[tl.x + tid] = v.pos[tl.x + tid];
   int running = 0;
-  for (int J0 = I + 1; J0 < nT; J0 += 64) {
-    const int J = J0 + lane;
-    const bool valid = J < nT;
-    const int c = valid ? __popcll(v.nl_mask[tp0 + (J - I - 1)]) : 0;
+  for (int J0 = I + 1; J0 < nT; J0 += THREADS) {
+    const int n = min(THREADS, nT - J0), tp = tp0 + (J0 - I - 1) + tid;
+    if (tid == 0) n_near = 0;
+    __syncthreads();  // and the last round's entries are written
+    masks[tid] = 0ull;
+    bool in = false;
+    if (tid < n && v.nl_tp[tp].slot >= 0) {  // else an ordinary item covers this tile pair
+      const int tJ = S.tile0 + J0 + tid;
+      const float4 lj = v.tbox[2 * tJ], hj = v.tbox[2 * tJ + 1];
+      const float bx = fmaxf(0.0f, fmaxf(lj.x - hi.x, li.x - hj.x));
+      const float by = fmaxf(0.0f, fmaxf(lj.y - hi.y, li.y - hj.y));
+      const float bz = fmaxf(0.0f, fmaxf(lj.z - hi.z, li.z - hj.z));
+      in = !(bx * bx + by * by + bz * bz >= S.nl_cut2);
+    }
+    const unsigned long long some = __ballot(in);
+    int base = 0;
+    if (lane == 0 && some != 0ull) base = atomicAdd(&n_near, __popcll(some));
+    base = __builtin_amdgcn_readfirstlane(base);
+    if (in) near[base + __popcll(some & nl_below(lane))] = tid;
+    __syncthreads();
+    for (int k = wave; k < n_near; k += kBatch * kWaves) {
+      int e[kBatch], nJ[kBatch];
+      float4 p[kBatch];
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        e[u] = near[min(k + u * kWaves, n_near - 1)];
+        const int a = (J0 + e[u]) * kTile;
+        nJ[u] = min(kTile, S.n - a);
+        p[u] = v.pos[S.a0 + a + min(lane, nJ[u] - 1)];
+      }
+#pragma unroll
+      for (int u = 0; u < kBatch; ++u) {
+        const float gx = fmaxf(0.0f, fmaxf(li.x - p[u].x, p[u].x - hi.x));
+        const float gy = fmaxf(0.0f, fmaxf(li.y - p[u].y, p[u].y - hi.y));
+        const float gz = fmaxf(0.0f, fmaxf(li.z - p[u].z, p[u].z - hi.z));
+        const unsigned long long m = __ballot(lane < nJ[u] && gx * gx + gy * gy + gz * gz < S.nl_cut2);
+        if (lane == 0) masks[e[u]] = m;
+      }
+    }
+    __syncthreads();
+    const unsigned long long mine = masks[tid];
+    const int c = __popcll(mine);
     int incl = c;  // inclusive prefix over the lanes, in lane order
     for (int off = 1; off < 64; off <<= 1) {
       const int y = __shfl_up(incl, off);
       if (lane >= off) incl += y;
     }
-    if (valid) v.nl_pref[tp0 + (J - I - 1)] = running + incl - c;
-    running += __builtin_amdgcn_readlane(incl, 63);
+    if (lane == 63) totals[wave] = incl;
+    __syncthreads();
+    int before = running;
+    for (int k = 0; k < kWaves; ++k) {
+      if (k < wave) before += totals[k];
+      running += totals[k];
+    }
+    prefs[tid] = before + incl - c;
+    if (tid < n) {
+      v.nl_mask[tp] = mine;
+      v.nl_pref[tp] = before + incl - c;
+    }
+    __syncthreads();
+    for (int k = wave; k < n_near; k += kWaves) {
+      const int e = near[k];
+      const unsigned long long m = masks[e];
+      if ((m >> lane) & 1ull)
+        v.nl_entries[entry0 + prefs[e] + __popcll(m & nl_below(lane))] = S.a0 + (J0 + e) * kTile + lane;
+    }
+    __syncthreads();
   }
-  if (lane == 0) v.nl_count[t] = running;
-  if (S.skin_half2 > 0.0f && lane < tl.y) v.nl_xref[tl.x + lane] = v.pos[tl.x + lane];
-}
-
-// Tile-pair record w, by one wave: the atoms of J in I's list, written at
-// I's entry base + the pair's prefix, in lane order -- so each row's entries
-// run in increasing atom index.
-__device__ __forceinline__ void nl_fill_wave(const DeviceView& v, int w) {
-  const TilePairInfo tp = v.nl_tp[w];
-  if (tp.ij < 0 || tp.slot < 0) return;  // a free record, or one an ordinary item covers
-  if (!v.nl_flag[tp.slot]) return;
-  const unsigned long long m = v.nl_mask[w];
-  if (m == 0ull) return;
-  const SlotConst& S = v.slots[tp.slot];
-  const int lane = threadIdx.x & 63;
-  const int I = tp.ij & 0xFFFF, J = tp.ij >> 16;
-  const int E = v.nl_row[S.tile0 + I].y + v.nl_pref[w];
-  if ((m >> lane) & 1ull) v.nl_entries[E + __popcll(m & nl_below(lane))] = S.a0 + J * kTile + lane;
+  if (tid == 0) v.nl_count[t] = running;
 }
 
 }  // namespace prx

@@ -86,16 +86,17 @@ __global__ __launch_bounds__(kPersistThreads) void k_persist_steps(DeviceView v,
 
   for (int k = 0; k < n_steps; ++k) {
     if (has_nl) {  // the list build (forced at the first step, as in a graph launch)
-      for (int s = blockIdx.x; s < n_slots; s += gridDim.x) {
-        nl_check_block(v, ranges, s, k == 0);
+      if (k != 0) {
+        for (int s = blockIdx.x; s < n_slots; s += gridDim.x) {
+          nl_check_block(v, ranges, s);
+          __syncthreads();
+        }
+        if (!grid_sync(bar, gen)) return;
+      }
+      for (int t = blockIdx.x; t < v.n_tiles; t += gridDim.x) {
+        nl_row_block<kPersistThreads>(v, t, k == 0);
         __syncthreads();
       }
-      if (!grid_sync(bar, gen)) return;
-      for (int w = wave; w < v.nl_tp_hw; w += n_waves) nl_mask_wave(v, w);
-      if (!grid_sync(bar, gen)) return;
-      for (int t = wave; t < v.n_tiles; t += n_waves) nl_rows_wave(v, t);
-      if (!grid_sync(bar, gen)) return;
-      for (int w = wave; w < v.nl_tp_hw; w += n_waves) nl_fill_wave(v, w);
       if (!grid_sync(bar, gen)) return;
     }
     for (int u = blockIdx.x; u < v.n_units; u += gridDim.x) {
