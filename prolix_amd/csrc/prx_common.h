@@ -263,6 +263,9 @@ void launch_nl_build(const DeviceView& v, const int32_t* slot_ranges, int n_slot
 void launch_dense_list(const float* pos, int n, float radius, int capacity, int32_t* idx, int32_t* counts,
                        float4* boxes, hipStream_t s);
 void launch_born_pairs(const DeviceView& v, hipStream_t s);                // also -> item_cls
+// launch_chain_pairs and launch_energy_reduce in one launch; false (and nothing
+// launched) where they take two.
+bool launch_chain_pairs_energies(const DeviceView& v, const int32_t* ranges, int n_slots, double* out, hipStream_t s);
 void launch_born_pairs_bonded(const DeviceView& v, bool energy, hipStream_t s);  // the same, and launch_bonded
 void launch_born_gather(const DeviceView& v, float* packed_radii, hipStream_t s);  // -> B, dB/dI (radii out or nullptr)
 void launch_force_pairs(const DeviceView& v, bool energy, hipStream_t s);

@@ -310,11 +310,13 @@ CmapCache g_cmap_cache;
 
 namespace {
 // Packed arrays of the caller: positions to evaluate at (nullptr: those in
-// vv), forces (nullptr: left in vv) and Born radii out (nullptr: none).
+// vv), forces (nullptr: left in vv) and Born radii out (nullptr: none); energies
+// of the listed systems out.
 struct Packed {
   const float* positions = nullptr;
   float* forces = nullptr;
   float* radii = nullptr;
+  double* energies = nullptr;
 };
 }  // namespace
 
@@ -1108,8 +1110,12 @@ struct prx_engine {
     prx::launch_born_gather(vv, io.radii, s);
     prx::launch_force_pairs(vv, energy, s);
     prx::launch_force_gather(vv, energy, s);
-    prx::launch_chain_pairs(vv, s);
+    // in line, every energy is there before the chain pass
+    const int n = (int)order.size();
+    const bool reduced = io.energies && !fork && prx::launch_chain_pairs_energies(vv, d_ranges, n, io.energies, s);
+    if (!reduced) prx::launch_chain_pairs(vv, s);
     if (fork) HIPCHECK(hipStreamWaitEvent(s, ev_join, 0));
+    if (io.energies && !reduced) prx::launch_energy_reduce(vv, d_ranges, n, io.energies, s);
   }
 
   void evaluate(const prx::DeviceView& vv, bool energy, hipStream_t s, const Packed& io = Packed()) {
@@ -1404,9 +1410,7 @@ int prx_energy_forces(prx_engine* eng, const float* positions, float* forces, do
     eng->rebuild();
     hipStream_t s = eng->pick(stream);
     const prx::DeviceView ev = eng->eval_view();
-    eng->evaluate(ev, energies != nullptr, s, {positions, forces, born_radii});
-    if (energies)
-      prx::launch_energy_reduce(ev, eng->d_ranges, (int)eng->order.size(), energies, s);
+    eng->evaluate(ev, energies != nullptr, s, {positions, forces, born_radii, energies});
     HIPCHECK(hipGetLastError());
   });
 }
@@ -1460,8 +1464,7 @@ int prx_energy_forces_noalloc(const prx_system_desc* desc, const float* position
       eng.admit(d);
       eng.rebuild();
       const prx::DeviceView ev = eng.eval_view();
-      eng.evaluate(ev, energies != nullptr, s, {positions, forces, born_radii});
-      if (energies) prx::launch_energy_reduce(ev, eng.d_ranges, 1, energies, s);
+      eng.evaluate(ev, energies != nullptr, s, {positions, forces, born_radii, energies});
       HIPCHECK(hipGetLastError());
       HIPCHECK(hipStreamSynchronize(s));
     } catch (...) {
@@ -1491,7 +1494,7 @@ int prx_integrator_init(prx_engine* eng, const float* positions, const float* mo
                               hipMemcpyHostToDevice, s));
       prx::launch_init_momenta(eng->v, eng->d_slot_list, (int)eng->order.size(), s);
     }
-    eng->evaluate(eng->v, false, s, {positions, nullptr, nullptr});
+    eng->evaluate(eng->v, false, s, {positions, nullptr, nullptr, nullptr});
     HIPCHECK(hipGetLastError());
     eng->initialized = true;
   });
@@ -1771,8 +1774,7 @@ int prx_pool_energy(prx_engine* pool, int32_t slot, double* energies_host, void*
     // integrator's stored forces stay those of its own force-only passes
     const prx::DeviceView ev = pool->eval_view();
     HIPCHECK(hipMemcpyAsync(ev.pos, pool->v.pos, (size_t)pool->v.atom_hw * sizeof(float4), hipMemcpyDeviceToDevice, s));
-    pool->evaluate(ev, true, s);
-    prx::launch_energy_reduce(ev, pool->d_ranges, (int)pool->order.size(), pool->d_energy_tmp, s);
+    pool->evaluate(ev, true, s, {nullptr, nullptr, nullptr, pool->d_energy_tmp});
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(s));
     const auto it = std::find(pool->order.begin(), pool->order.end(), slot);

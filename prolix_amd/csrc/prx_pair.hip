@@ -26,6 +26,7 @@
 #include <type_traits>
 
 #include "prx_bonded_dev.h"
+#include "prx_energy_dev.h"
 #include "prx_pair_dev.h"
 
 namespace prx {
@@ -59,6 +60,18 @@ __global__ __launch_bounds__(kThreads<WAVES>) PRX_FORCE_OCCUPANCY(WAVES, ENERGY)
 template <int WAVES>
 __global__ __launch_bounds__(kThreads<WAVES>) PRX_OCCUPANCY void k_chain_pairs(DeviceView v) {
   pair_block<WAVES, ChainPass>(v, blockIdx.x, gridDim.x);
+}
+
+// The chain pass with the energy reduction in the same launch: blocks below
+// n_slots take a system's energies each, which are complete before the pass, the
+// rest the pass's units.
+__global__ __launch_bounds__(kThreads<kUnitWaves>) void k_chain_pairs_energies(DeviceView v, const int32_t* ranges,
+                                                                               int n_slots, double* out) {
+  const int b = (int)blockIdx.x;
+  if (b < n_slots)
+    energy_reduce_block<kThreads<kUnitWaves>>(v, ranges, b, out);
+  else
+    pair_block<kUnitWaves, ChainPass>(v, b - n_slots, (int)gridDim.x - n_slots);
 }
 
 // The Born pass with the bonded terms in the same launch: blocks below
@@ -143,6 +156,17 @@ void launch_chain_pairs(const DeviceView& v, hipStream_t s) {
     constexpr int W = decltype(w)::value;
     hipLaunchKernelGGL(k_chain_pairs<W>, dim3(pair_blocks(v, W)), dim3(kThreads<W>), 0, s, v);
   });
+}
+
+// Lists of four-wave units are short, and the reduction hides behind them (138
+// atoms 68.3 us an evaluation with a launch of its own, 66.0 in this one, 1,237
+// atoms 75.7 and 71.5); with the large systems of the other lists 64 or 128
+// threads would outlast the pass.
+bool launch_chain_pairs_energies(const DeviceView& v, const int32_t* ranges, int n_slots, double* out, hipStream_t s) {
+  if (v.n_items == 0 || block_waves(v) != kUnitWaves) return false;
+  hipLaunchKernelGGL(k_chain_pairs_energies, dim3(n_slots + v.n_units), dim3(kThreads<kUnitWaves>), 0, s, v, ranges,
+                     n_slots, out);
+  return true;
 }
 
 }  // namespace prx
