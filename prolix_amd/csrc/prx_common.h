@@ -60,6 +60,8 @@ constexpr int kHalfTiles = 128;
 // 35, 54, 52 us a pass with waves, 33, 50, 44 with units; 142,848 items: 319,
 // 609, 445 us with waves, 470, 686, 540 with units.
 constexpr int kWaveItems = 10000;
+// The persistent kernel runs units up to this many, else an item per wave.
+constexpr int kPersistUnits = 64;
 
 constexpr int kFlagDiag = 1;
 constexpr int kFlagExcl = 2;
@@ -249,6 +251,8 @@ struct GridBarrier {
   int error;            // 1: a wait timed out; every block leaves the launch
   int pad;
 };
+
+inline __host__ __device__ bool persist_by_unit(const DeviceView& v) { return v.n_units <= kPersistUnits; }
 
 // Launchers (defined in the .hip translation units).
 void launch_tile_boxes(const DeviceView& v, hipStream_t s);                // -> tbox (every evaluation)

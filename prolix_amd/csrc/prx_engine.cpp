@@ -376,9 +376,11 @@ struct prx_engine {
   // 2 = the persistent kernel, 3 = the fused kernel (one workgroup per system)
   int32_t step_mode = 0;
   static constexpr int32_t kFusedAutoAtoms = prx::kTile;
-  // Steps recorded into a caller's own graph: no step graph can be captured or
-  // launched there, but the fused kernel can run, and does up to this size.
-  static constexpr int32_t kFusedRecordAtoms = 3 * prx::kTile;
+  // Steps recorded into a caller's own graph, in which no step graph can be
+  // captured or launched: systems up to this size, as the passes themselves (138
+  // atoms 44 us a step, 78 fused), or fused in calls of more than kGraphSteps.
+  static constexpr int32_t kRecordAtoms = 3 * prx::kTile;
+  static constexpr int kGraphSteps = 50;  // steps per step graph
   int32_t max_system_atoms = 0;   // largest live system (rebuild)
   prx::GridBarrier* d_bar = nullptr;
   int persist_blocks = -1;        // co-resident grid of the persistent kernel (0: unavailable)
@@ -1136,14 +1138,7 @@ struct prx_engine {
     hipGraph_t g = nullptr;
     HIPCHECK(hipStreamBeginCapture(stream, hipStreamCaptureModeRelaxed));
     try {
-      prx::launch_step_begin(v, stream);
-      const prx::DeviceView sv = step_view();
-      for (int k = 0; k < n_steps; ++k) {
-        // after the first step, the previous chain gather wrote the boxes
-        force_passes(sv, false, stream, k == 0);
-        prx::launch_chain_gather(sv, k + 1 == n_steps ? 2 : 1, nullptr, stream);
-      }
-      HIPCHECK(hipGetLastError());
+      launch_steps(n_steps, stream);
     } catch (...) {
       // leave the stream out of capture mode before reporting the failure
       if (hipStreamEndCapture(stream, &g) == hipSuccess && g) hipGraphDestroy(g);
@@ -1185,24 +1180,39 @@ struct prx_engine {
     return true;
   }
 
+  // The caller's stream is recording a graph of the caller's own.
+  static bool recording(hipStream_t s) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return s != nullptr && hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusActive;
+  }
+
+  // n_steps steps as single launches on s.
+  void launch_steps(int n_steps, hipStream_t s) {
+    prx::launch_step_begin(v, s);
+    const prx::DeviceView sv = step_view();
+    for (int k = 0; k < n_steps; ++k) {
+      // after the first step, the previous chain gather wrote the boxes
+      force_passes(sv, false, s, k == 0);
+      prx::launch_chain_gather(sv, k + 1 == n_steps ? 2 : 1, nullptr, s);
+    }
+    HIPCHECK(hipGetLastError());
+  }
+
   // The fused kernel: every system in one workgroup of its own. Not for
   // neighbour-list systems (their list build spans workgroups).
-  bool use_fused(hipStream_t s) const {
-    if (step_mode == 0) {
-      if (has_nl || max_system_atoms > kFusedRecordAtoms) return false;
-      if (max_system_atoms <= kFusedAutoAtoms) return true;
-      hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-      return s != nullptr && hipStreamIsCapturing(s, &st) == hipSuccess && st == hipStreamCaptureStatusActive;
-    }
+  bool use_fused(bool recorded) const {
+    if (step_mode == 0) return !has_nl && max_system_atoms <= (recorded ? kRecordAtoms : kFusedAutoAtoms);
     if (step_mode != 3) return false;
     if (has_nl) throw StateError("the fused step kernel does not run neighbour-list systems");
     return true;
   }
 
-  // The persistent kernel: at most one unit and one tile per block in each
-  // pass, within the co-resident grid.
+  // The persistent kernel: at most one unit, or one item per wave, and one tile
+  // per block in each pass, within the co-resident grid.
   void steps_persistent(int n_steps, hipStream_t s) {
-    const int64_t want = std::max<int64_t>({(int64_t)v.n_tiles, (int64_t)v.n_units, 1});
+    const int64_t pair_blocks =
+        prx::persist_by_unit(v) ? v.n_units : ((int64_t)v.n_items + prx::kUnitWaves - 1) / prx::kUnitWaves;
+    const int64_t want = std::max<int64_t>({(int64_t)v.n_tiles, pair_blocks, 1});
     const int blocks = (int)std::min<int64_t>(want, persist_blocks);
     for (int left = n_steps; left > 0;) {
       const int k = std::min(left, kPersistChunk);
@@ -1220,6 +1230,11 @@ struct prx_engine {
     flush_pending(s);
     rebuild();
     if (order.empty() || n_steps <= 0) return;
+    const bool recorded = step_mode == 0 && recording(s);
+    if (recorded && n_steps <= kGraphSteps && use_fused(true) && !use_fused(false) && !fork_bonded()) {
+      launch_steps(n_steps, s);
+      return;
+    }
     // the steps run on the engine stream, ordered after the caller's
     hipEvent_t ev;
     HIPCHECK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
@@ -1228,7 +1243,7 @@ struct prx_engine {
         HIPCHECK(hipEventRecord(ev, s));
         HIPCHECK(hipStreamWaitEvent(stream, ev, 0));
       }
-      if (use_fused(s)) {
+      if (use_fused(recorded)) {
         for (int left = n_steps; left > 0;) {
           const int k = std::min(left, kPersistChunk);
           prx::launch_fused_steps(v, d_ranges, (int)order.size(), k, stream);
@@ -1238,7 +1253,7 @@ struct prx_engine {
       } else if (use_persistent()) {
         steps_persistent(n_steps, stream);
       } else {
-        const int chunk = std::min(n_steps, 50);
+        const int chunk = std::min(n_steps, kGraphSteps);
         for (int left = n_steps; left > 0;) {
           const int k = std::min(chunk, left);
           HIPCHECK(hipGraphLaunch(capture(k), stream));

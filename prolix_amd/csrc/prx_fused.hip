@@ -60,6 +60,25 @@ __device__ __forceinline__ void group_round(int t, int t1, int grp, F&& work) {
   __syncthreads();
 }
 
+// One pair pass of a system, items i0 to i1 - 1 (R[0], R[1]): up to kFusedUnits
+// items in shares, a unit per group, more of them an item per wave, without barriers
+// in between. us a step with units and with waves: 138 atoms (6 items) 78 and 91,
+// 256 (10) 136 and 151, 500 (36) 387 and 293, 2,500 (820) 5,446 and 3,698.
+constexpr int kFusedUnits = 10;
+
+template <class Pass>
+__device__ __forceinline__ void pair_pass(const DeviceView& v, const SlotConst& S, int i0, int i1, int wave, int grp,
+                                          int uw, UnitLds<kPairLds>& L) {
+  if (i1 - i0 <= kFusedUnits) {
+    const int u1 = S.unit0 + S.n_units;
+    for (int u = S.unit0; u < u1; u += kFusedGroups)
+      group_round<2>(u, u1, grp, [&](int uu) { pair_unit<true, Pass>(v, uu, uw, L); });
+  } else {
+    for (int w = i0 + wave; w < i1; w += kFusedWaves) pair_wave<Pass>(v, w, L.wave[uw]);
+    __syncthreads();
+  }
+}
+
 // Block b: the b-th listed system, ranges row b (item_b, item_e, a0, n, then
 // the bonded ranges).
 __global__ __launch_bounds__(kFusedThreads) void k_fused_steps(DeviceView v, const int32_t* ranges, int n_steps) {
@@ -69,7 +88,6 @@ __global__ __launch_bounds__(kFusedThreads) void k_fused_steps(DeviceView v, con
   const int a0 = R[2], n = R[3];
   if (n <= 0) return;
   const SlotConst& S = v.slots[v.slot_of[a0]];
-  const int u0 = S.unit0, u1 = u0 + S.n_units;
   const int t0 = S.tile0;
   const int t1 = t0 + (n + kTile - 1) / kTile;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
@@ -86,16 +104,13 @@ __global__ __launch_bounds__(kFusedThreads) void k_fused_steps(DeviceView v, con
 
   for (int k = 0; k < n_steps; ++k) {
     bonded_slot(v, R);
-    for (int u = u0; u < u1; u += kFusedGroups)
-      group_round<2>(u, u1, grp, [&](int uu) { pair_unit<true, BornPass>(v, uu, uw, L); });
+    pair_pass<BornPass>(v, S, R[0], R[1], wave, grp, uw, L);
     for (int t = t0; t < t1; t += kFusedGroups)
       group_round<1>(t, t1, grp, [&](int tt) { born_gather_tile(v, tt, G); });
-    for (int u = u0; u < u1; u += kFusedGroups)
-      group_round<2>(u, u1, grp, [&](int uu) { pair_unit<true, ForcePass<false>>(v, uu, uw, L); });
+    pair_pass<ForcePass<false>>(v, S, R[0], R[1], wave, grp, uw, L);
     for (int t = t0; t < t1; t += kFusedGroups)
       group_round<1>(t, t1, grp, [&](int tt) { force_gather_tile<false>(v, tt, G); });
-    for (int u = u0; u < u1; u += kFusedGroups)
-      group_round<2>(u, u1, grp, [&](int uu) { pair_unit<true, ChainPass>(v, uu, uw, L); });
+    pair_pass<ChainPass>(v, S, R[0], R[1], wave, grp, uw, L);
     const int mode = k + 1 == n_steps ? 2 : 1;  // the last step stops after B(F)
     for (int t = t0; t < t1; t += kFusedGroups)
       group_round<1>(t, t1, grp, [&](int tt) { chain_gather_tile(v, tt, mode, G); });

@@ -66,6 +66,22 @@ __device__ __forceinline__ bool grid_sync(GridBarrier* bar, unsigned& gen) {
   return s_ok != 0;
 }
 
+// One pair pass over the grid: short lists a unit per block (138 atoms 48 us a
+// step, 72 with an item per wave), longer ones an item per wave, with a quarter of
+// the blocks, whose number the grid barriers' time grows with (2,500 atoms 201 us
+// a step, 480 with units).
+template <class Pass>
+__device__ __forceinline__ void pair_pass(const DeviceView& v, int wave, int n_waves, int uw, UnitLds<kPairLds>& L) {
+  if (persist_by_unit(v)) {
+    for (int u = blockIdx.x; u < v.n_units; u += gridDim.x) {
+      pair_unit<true, Pass>(v, u, uw, L);
+      __syncthreads();
+    }
+  } else {
+    for (int w = wave; w < v.n_items; w += n_waves) pair_wave<Pass>(v, w, L.wave[uw]);
+  }
+}
+
 __global__ __launch_bounds__(kPersistThreads) void k_persist_steps(DeviceView v, const int32_t* ranges, int n_slots,
                                                                     int n_steps, int has_nl, GridBarrier* bar) {
   __shared__ UnitLds<kPairLds> L;
@@ -99,10 +115,7 @@ __global__ __launch_bounds__(kPersistThreads) void k_persist_steps(DeviceView v,
       }
       if (!grid_sync(bar, gen)) return;
     }
-    for (int u = blockIdx.x; u < v.n_units; u += gridDim.x) {
-      pair_unit<true, BornPass>(v, u, uw, L);
-      __syncthreads();
-    }
+    pair_pass<BornPass>(v, wave, n_waves, uw, L);
     for (int e = tid; e < n_bonded; e += n_threads) bonded_entry<false>(v, e);
     if (!grid_sync(bar, gen)) return;
     for (int t = blockIdx.x; t < v.n_tiles; t += gridDim.x) {
@@ -110,20 +123,14 @@ __global__ __launch_bounds__(kPersistThreads) void k_persist_steps(DeviceView v,
       __syncthreads();
     }
     if (!grid_sync(bar, gen)) return;
-    for (int u = blockIdx.x; u < v.n_units; u += gridDim.x) {
-      pair_unit<true, ForcePass<false>>(v, u, uw, L);
-      __syncthreads();
-    }
+    pair_pass<ForcePass<false>>(v, wave, n_waves, uw, L);
     if (!grid_sync(bar, gen)) return;
     for (int t = blockIdx.x; t < v.n_tiles; t += gridDim.x) {
       force_gather_tile<false>(v, t, G);
       __syncthreads();
     }
     if (!grid_sync(bar, gen)) return;
-    for (int u = blockIdx.x; u < v.n_units; u += gridDim.x) {
-      pair_unit<true, ChainPass>(v, u, uw, L);
-      __syncthreads();
-    }
+    pair_pass<ChainPass>(v, wave, n_waves, uw, L);
     if (!grid_sync(bar, gen)) return;
     const int mode = k + 1 == n_steps ? 2 : 1;  // the last step stops after B(F)
     for (int t = blockIdx.x; t < v.n_tiles; t += gridDim.x) {

@@ -1,5 +1,6 @@
-"""Steps recorded into a caller's own graph (small systems: the fused kernel)
-and replayed equal the same steps run directly, bit for bit."""
+"""Steps recorded into a caller's own graph (systems up to 192 atoms: the passes
+themselves, the fused kernel for one tile and in long calls) and replayed equal
+the same steps run directly, bit for bit."""
 
 from __future__ import annotations
 
@@ -11,8 +12,8 @@ from tests.helpers import protein
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [64, 65, 192])
-def test_recorded_steps_equal_direct_ones(n):
+@pytest.mark.parametrize("n,steps", [(64, 5), (65, 5), (192, 5), (100, 50), (100, 51)])
+def test_recorded_steps_equal_direct_ones(n, steps):
     import torch
 
     from prolix_amd.engine import GBEngine, Langevin
@@ -26,12 +27,12 @@ def test_recorded_steps_equal_direct_ones(n):
         if record:
             g = torch.cuda.CUDAGraph()
             with torch.cuda.graph(g):
-                eng.steps(5)
+                eng.steps(steps)
         for _ in range(3):
             if record:
                 g.replay()
             else:
-                eng.steps(5)
+                eng.steps(steps)
             torch.cuda.synchronize()
             out.append([a.cpu().numpy() for a in eng.state()])
         eng.close()
