@@ -45,7 +45,7 @@ FLOPS_PER_PAIR = {"born_pairs": 56, "force_pairs": 73, "chain_pairs": 62}  # alg
 FLOPS_TOTAL = 191
 PEAK_FP32 = 157.3  # TFLOP/s, MI355X FP32 vector peak (packed FP32)
 PEAK_FP32_UNPACKED = 78.6  # TFLOP/s, one FP32 FMA per lane per clock (the kernels issue above it: plain
-#                            v_fma_f32 measured at 1.36 wave64 instructions per clock per CU)
+#                            FP32 measured at about 1.8 wave64 instructions per clock per CU)
 DT_FS = 1.0
 
 
