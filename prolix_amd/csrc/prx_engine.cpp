@@ -446,6 +446,14 @@ struct prx_engine {
     return reinterpret_cast<T*>(arena + off);
   }
 
+  // The items and, behind them, the units (each holds an item at least).
+  void alloc_items() {
+    const size_t n = std::max<size_t>((size_t)cap_items, 1);
+    char* p = dalloc<char>(n * (sizeof(prx::PairItem) + sizeof(prx::PairUnit)));
+    d_items = reinterpret_cast<prx::PairItem*>(p);
+    d_units = reinterpret_cast<prx::PairUnit*>(p + n * sizeof(prx::PairItem));
+  }
+
   // In arena mode the work list's buffers are sized now, exactly (the engine
   // holds one fixed set of systems); otherwise rebuild() sizes them.
   void alloc_work(int64_t n_items, int64_t n_tiles) {
@@ -454,8 +462,7 @@ struct prx_engine {
       d_units = reinterpret_cast<prx::PairUnit*>(get<float4>(cap_items));
       d_items = reinterpret_cast<prx::PairItem*>(arena + arena_cap);
     } else {
-      d_items = get<prx::PairItem>(cap_items);
-      d_units = get<prx::PairUnit>(cap_items);
+      alloc_items();
     }
     d_e_items = get<double>(cap_items * 3);
     d_part = get<float4>(cap_items * 2 * prx::kTile);
@@ -569,7 +576,7 @@ struct prx_engine {
     void* ptrs[] = {v.pos, v.mom, v.force, v.born4, v.nb4, v.fin4, v.sqrt_m, v.slot_of, v.gb4, v.fpair, d_part, d_tiles,
                     v.e_atom, v.atom_step, v.bonds, v.angles, v.tors, v.cmaps, v.excs, v.e_bond, v.e_angle,
                     v.e_tors, v.e_cmap, v.e_exc, d_coeff, d_excl, v.slots, d_ranges, d_slot_list,
-                    d_energy_tmp, d_map, d_items, d_units, d_e_items, v.rec, v.atom_rec, d_rec_list, v.warn,
+                    d_energy_tmp, d_map, d_items, d_e_items, v.rec, v.atom_rec, d_rec_list, v.warn,
                     d_tbox, d_item_cls, d_eval_pos, d_eval_force, d_nl_tp, d_nl_mask, d_nl_pref,
                     d_nl_entries, d_nl_xref, d_nl_flag, d_nl_row, d_nl_count, d_nl_col, d_nl_colitems, d_bar};
     for (void* p : ptrs)
@@ -991,9 +998,7 @@ struct prx_engine {
       if (d_part) HIPCHECK(hipFree(d_part));
       cap_items = std::max<int64_t>((int64_t)items.size(), cap_items * 3 / 2);
       if (d_item_cls) HIPCHECK(hipFree(d_item_cls));
-      if (d_units) HIPCHECK(hipFree(d_units));
-      d_items = dalloc<prx::PairItem>(cap_items);
-      d_units = dalloc<prx::PairUnit>(cap_items);  // a unit holds an item at least
+      alloc_items();
       d_e_items = dalloc<double>(cap_items * 3);
       d_part = dalloc<float4>(cap_items * 2 * prx::kTile);
       d_item_cls = dalloc<int32_t>(cap_items);
@@ -1029,7 +1034,7 @@ struct prx_engine {
       HIPCHECK(hipMemcpy(d_tiles, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice));
     if (!items.empty())
       HIPCHECK(hipMemcpy(d_items, items.data(), items.size() * sizeof(prx::PairItem), hipMemcpyHostToDevice));
-    if (!units.empty())
+    if (!units.empty() && shares != prx::kUnitWaves)  // else unit k is item k, and no list is read
       HIPCHECK(hipMemcpy(d_units, units.data(), units.size() * sizeof(prx::PairUnit), hipMemcpyHostToDevice));
     if (!ranges.empty())
       HIPCHECK(hipMemcpy(d_ranges, ranges.data(), ranges.size() * sizeof(int32_t), hipMemcpyHostToDevice));
