@@ -55,11 +55,12 @@ struct PairUnit {
 // and above kHalfTiles, where one system fills the chip, items stay whole.
 constexpr int kQuarterTiles = 40;
 constexpr int kHalfTiles = 128;
-// Work lists of at least this many items (9 or more per SIMD) run one wave per
-// item, shorter ones a group of waves per unit. 16,110 items of four systems:
-// 35, 54, 52 us a pass with waves, 33, 50, 44 with units; 142,848 items: 319,
-// 609, 445 us with waves, 470, 686, 540 with units.
-constexpr int kWaveItems = 10000;
+// Work lists of at least this many items run one wave per item, shorter ones with
+// shares a group of waves per unit. us a pass (Born, force, chain) with units and
+// with waves: 8,064 items of four systems 33, 52, 45 and 41, 58, 56; 50,560 of 16
+// systems 109, 207, 153 and 110, 217, 163; 78,720 of 96 systems 230, 363, 286 and
+// 203, 362, 288; 142,848 of 256 systems 355, 617, 465 and 324, 604, 458.
+constexpr int kWaveItems = 64000;
 // The persistent kernel runs units up to this many, else an item per wave.
 constexpr int kPersistUnits = 64;
 

@@ -43,11 +43,12 @@ def test_edges_match_the_oracle(n, cutoff):
 @pytest.mark.parametrize("cutoff,gb_cutoff", [(0.0, False), (12.0, True)])
 def test_waves_and_units_agree(cutoff, gb_cutoff):
     """Systems of four, two and one share per item, alone (units) and in a pack of
-    more than 10,000 items (a wave each)."""
+    more than 64,000 items (a wave each)."""
     systems = [protein(n, 30 + n % 7) for n in (130, 2300, 2600, 8300, 130)]
+    systems += [systems[3]] * 7
     e, f, f0 = _evaluate(systems, cutoff=cutoff, gb_cutoff=gb_cutoff)
     at = 0
-    for k, s in enumerate(systems):
+    for k, s in enumerate(systems[:5]):
         n = len(s["charges"])
         e1, f1, f01 = _evaluate([s], cutoff=cutoff, gb_cutoff=gb_cutoff)
         assert np.array_equal(e[k], e1[0]), n
