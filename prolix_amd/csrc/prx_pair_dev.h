@@ -987,8 +987,9 @@ struct ForcePass {
     if (rows) { pi = v.pos[gi]; ci = v.nb4[gi]; bi = v.gb4[gi]; }
     if (cols) { pj = v.pos[gj]; cj = v.nb4[gj]; bj = v.gb4[gj]; }
     Tile4* t = reinterpret_cast<Tile4*>(L);
-    // past the end of a ragged tile: no charge, no well depth, B = 1 and an exponent of 0
-    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f), one = make_float4(1.f, 0.f, 0.f, 0.f);
+    // past the end of a ragged tile: no charge, no well depth, B = 1 and next to no
+    // exponent (0 times the r^2 of an atom at infinity would not be a number)
+    const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f), one = make_float4(1.f, 1e-30f, 0.f, 0.f);
     if (rows) {
       if (!full && lane >= ni) { pi = pad_pos(lane); ci = zero; bi = one; }
       t[0][lane] = make_float4(pi.x, pi.y, pi.z, ci.x);
