@@ -240,14 +240,14 @@ template <int CLS>
 struct BornW {
   static constexpr int N = (CLS == kFar2 ? kObcH2Deg : CLS == kFar3 ? kObcH3Deg : CLS == kFar4 ? kObcH4Deg : kObcHDeg) + 1;
   __device__ static constexpr float c(int k) {
-    return k == 0 ? 1.0f : 1.5f * (CLS == kFar2 ? kObcH2[k] : CLS == kFar3 ? kObcH3[k] : CLS == kFar4 ? kObcH4[k] : kObcH[k]);
+    return (float)(1.5 * (CLS == kFar2 ? kObcH2[k] : CLS == kFar3 ? kObcH3[k] : CLS == kFar4 ? kObcH4[k] : kObcH[k]));
   }
 };
 template <int CLS>
 struct ChainW {
   static constexpr int N = (CLS == kFar2 ? kObcK2Deg : CLS == kFar3 ? kObcK3Deg : CLS == kFar4 ? kObcK4Deg : kObcKDeg) + 1;
   __device__ static constexpr float c(int k) {
-    return k == 0 ? -4.0f : -3.0f * (CLS == kFar2 ? kObcK2[k] : CLS == kFar3 ? kObcK3[k] : CLS == kFar4 ? kObcK4[k] : kObcK[k]);
+    return (float)(-3.0 * (CLS == kFar2 ? kObcK2[k] : CLS == kFar3 ? kObcK3[k] : CLS == kFar4 ? kObcK4[k] : kObcK[k]));
   }
 };
 
