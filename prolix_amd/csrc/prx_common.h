@@ -40,6 +40,8 @@ struct PairUnit {
   int32_t first;
   int16_t n, shares;
 };
+// the serving loop's footprint of an item counts these
+static_assert(sizeof(PairItem) == 32 && sizeof(PairUnit) == 8, "serving.hbm_bytes");
 // Shares of the items of a system by its size (item_shares). A wave alone on
 // its SIMD issues at half rate and no other hides its loads, and a system of a few
 // thousand atoms has fewer items than the chip has SIMDs (2,500 atoms: 820 of

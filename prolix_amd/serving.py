@@ -30,9 +30,9 @@ TILE = 64
 def hbm_bytes(n_atoms: int, n_bonded: int = 0) -> int:
     """Device footprint of one system: per-atom arrays (~330 B), bonded entries
     with force records and energy slots (~120 B each) and the pair work list
-    with its 2 x 64 float4 partial slots and energies (~2.1 KB per 64x64 tile pair)."""
+    with its 2 x 64 float4 partial slots, unit, energies and class (2,116 B per 64x64 tile pair)."""
     nt = (n_atoms + TILE - 1) // TILE
-    return 330 * n_atoms + 120 * n_bonded + 2100 * nt * (nt + 1) // 2
+    return 330 * n_atoms + 120 * n_bonded + 2116 * nt * (nt + 1) // 2
 
 
 @dataclass
