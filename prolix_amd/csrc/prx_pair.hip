@@ -158,10 +158,12 @@ void launch_chain_pairs(const DeviceView& v, hipStream_t s) {
   });
 }
 
-// Lists of four-wave units are short, and the reduction hides behind them (138
-// atoms 68.3 us an evaluation with a launch of its own, 66.0 in this one, 1,237
-// atoms 75.7 and 71.5); with the large systems of the other lists 64 or 128
-// threads would outlast the pass.
+// In lists of four-wave units the reduction hides behind the pass (138 atoms 68.3 us
+// an evaluation with a launch of its own, 66.0 in this one, 1,237 atoms 75.7 and
+// 71.5), also that of a large system which a smaller one brings into such a list
+// (energies add 10 us to the forces of 130 + 8,300 atoms, 17 to those of 130 + 12,000). The
+// other lists' blocks of 64 or 128 threads would take two or four times as long
+// over a system.
 bool launch_chain_pairs_energies(const DeviceView& v, const int32_t* ranges, int n_slots, double* out, hipStream_t s) {
   if (v.n_items == 0 || block_waves(v) != kUnitWaves) return false;
   hipLaunchKernelGGL(k_chain_pairs_energies, dim3(n_slots + v.n_units), dim3(kThreads<kUnitWaves>), 0, s, v, ranges,
