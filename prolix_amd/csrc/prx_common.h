@@ -17,7 +17,7 @@
 
 namespace prx {
 
-constexpr int kTile = 64;               // wave64: one i atom per lane, 64 j atoms rotate
+constexpr int kTile = 64;               // wave64: atoms of a tile, one per lane when staged
 constexpr int kMaxExclClasses = 3;      // distinct non-unit (vdw, elec) scale pairs
 constexpr float kLog2E = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
@@ -29,12 +29,11 @@ struct PairItem {
   int32_t meta;  // ni (bits 0-6), nj (bits 7-13), flags (bits 14-15), slot (bits 16-31)
   int32_t excl;  // exclusion-mask tile index, or -1
   int32_t ti, tj;  // global indices of the two tiles (a chunk item's ti is its row's; tj unused)
-  int32_t nsub;    // shares of the item (1, 2 or 4, prx_pair_dev.h)
+  int32_t nsub;    // shares of the item's rows (1 or 2, prx_pair_dev.h)
   int32_t pad;
 };
 // Unit of the pair passes, the work of a group of kUnitWaves waves: the items
-// first .. first + n - 1, each cut into the same number of shares, a share per
-// wave (n * shares <= kUnitWaves).
+// first .. first + n - 1, each on `shares` waves (n * shares <= kUnitWaves).
 constexpr int kUnitWaves = 4;
 struct PairUnit {
   int32_t first;
@@ -42,27 +41,20 @@ struct PairUnit {
 };
 // the serving loop's footprint of an item counts these
 static_assert(sizeof(PairItem) == 32 && sizeof(PairUnit) == 8, "serving.hbm_bytes");
-// Shares of the items of a system by its size (item_shares). A wave alone on
-// its SIMD issues at half rate and no other hides its loads, and a system of a few
-// thousand atoms has fewer items than the chip has SIMDs (2,500 atoms: 820 of
-// 1,024), so that a pass takes the time of one item on one wave. Alone, whole
-// items / 2 shares / 4 shares, us a pass (Born, force, chain):
-//     3,000 atoms   24.4 23.4 31.1 / 17.6 16.6 20.2 / 16.0 13.8 17.4
-//     5,000 atoms   27.4 31.9 33.7 / 21.0 25.9 26.5 / 21.2 24.4 25.2
-//     8,000 atoms   40.2 52.5 49.9 / 34.3 47.8 43.3 / 32.3 49.0 40.2
-// In a pack that fills the chip each share more costs 3 to 4% of a pass
-// (the column sums of a share are summed over its lanes; 256 systems of 300 to 5,000
-// atoms: 322, 624, 457 us with these lines, 344, 673, 497 with 4 shares for
-// all), so systems above kQuarterTiles, where most of a pack's items are, take 2,
-// and above kHalfTiles, where one system fills the chip, items stay whole.
-constexpr int kQuarterTiles = 40;
+// The rows of an item are two shares in systems up to kHalfTiles tiles, else one
+// (item_shares): a wave alone on its SIMD issues at half rate and no other hides its
+// loads, and one such system has too few items to fill the chip. us a pass (Born,
+// force, chain) with whole items and with two shares: one system of 8,000 atoms 31.4,
+// 42.9, 42.9 and 27.6, 43.3, 37.5; of 15,000 atoms 64.6, 117, 92 and 62.8, 119, 88;
+// nine of 8,300 155, 309, 222 and 162, 318, 226.
 constexpr int kHalfTiles = 128;
-// Work lists of at least this many items run one wave per item, shorter ones with
-// shares a group of waves per unit. us a pass (Born, force, chain) with units and
-// with waves: 8,064 items of four systems 33, 52, 45 and 41, 58, 56; 50,560 of 16
-// systems 109, 207, 153 and 110, 217, 163; 78,720 of 96 systems 230, 363, 286 and
-// 203, 362, 288; 142,848 of 256 systems 355, 617, 465 and 324, 604, 458.
-constexpr int kWaveItems = 64000;
+// Two shares run on two waves, in work lists shorter than kQuarterItems on four (a half of
+// the columns each). us a step on four and on two: one system of 3,000 atoms 58 and
+// 67, of 5,000 (3,160 items) 83 and 86; of 1,250 atoms 19 systems (3,990 items) 102 and
+// 103, 28 (5,880) 129 and 127, 61 (12,810) 227 and 204. An item per wave is no
+// faster in the longest lists: 303 systems of 700 atoms (20,000 items) 361 and 338
+// with two, 31 of 5,000 (97,960) 1,113 and 1,064.
+constexpr int kQuarterItems = 5000;
 // The persistent kernel runs units up to this many, else an item per wave.
 constexpr int kPersistUnits = 64;
 

@@ -947,7 +947,9 @@ struct prx_engine {
     std::vector<int2> nl_col;
     std::vector<int32_t> nl_colitems;
     offsets.assign(1, 0);
-    int32_t shares = -1;  // of every item so far, 0 where systems differ
+    int32_t shares = -1;  // waves per item so far, 0 where systems differ
+    size_t n_list = 0;
+    for (int32_t sid : order) n_list += slots[sid].items.size();
     max_system_atoms = 0;
     has_nl = has_skin = false;
     for (int32_t sid : order) {
@@ -956,10 +958,9 @@ struct prx_engine {
       s.c.item_base = ib;
       s.c.tile0 = (int32_t)tiles.size();
       const int nT = (s.n + prx::kTile - 1) / prx::kTile;
-      const int32_t n_it = (int32_t)s.items.size();
       s.c.unit0 = (int32_t)units.size();
       s.c.pack0 = offsets.back();
-      const int32_t sh = prx::append_units(s.items, ib, units);
+      const int32_t sh = prx::append_units(s.items, nT, n_list, ib, units);
       shares = shares < 0 || shares == sh ? sh : 0;
       s.c.n_units = (int32_t)units.size() - s.c.unit0;
       push_const(sid, s.c);

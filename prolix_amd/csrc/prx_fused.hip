@@ -46,17 +46,15 @@ __device__ __forceinline__ void bonded_slot(const DeviceView& v, const int32_t* 
   for (int e = R[12] + (int)threadIdx.x; e < R[13]; e += kFusedThreads) do_exception<false>(v, e);
 }
 
-// One round of units or tile gathers: group g of four waves takes unit or tile
-// t + g, or, past the last one, the barriers that it would have held (two a
-// unit, one a gather). Then the round's barrier, before the workgroup memory is
-// used again.
-template <int BARRIERS, class F>
-__device__ __forceinline__ void group_round(int t, int t1, int grp, F&& work) {
-  if (t + grp < t1) {
-    work(t + grp);
-  } else {
-    for (int k = 0; k < BARRIERS; ++k) __syncthreads();
-  }
+// One round of tile gathers: group g of four waves gathers tile t + g, or,
+// past the last tile, takes the one barrier that gather would have held.
+// Then the round's barrier, before the workgroup memory is used again.
+template <class F>
+__device__ __forceinline__ void gather_round(int t, int t1, int grp, F&& gather) {
+  if (t + grp < t1)
+    gather(t + grp);
+  else
+    __syncthreads();
   __syncthreads();
 }
 
@@ -68,21 +66,26 @@ constexpr int kFusedUnits = 10;
 
 template <class Pass>
 __device__ __forceinline__ void pair_pass(const DeviceView& v, const SlotConst& S, int i0, int i1, int wave, int grp,
-                                          int uw, UnitLds<kPairLds>& L) {
-  if (i1 - i0 <= kFusedUnits) {
-    const int u1 = S.unit0 + S.n_units;
-    for (int u = S.unit0; u < u1; u += kFusedGroups)
-      group_round<2>(u, u1, grp, [&](int uu) { pair_unit<true, Pass>(v, uu, uw, L); });
-  } else {
-    for (int w = i0 + wave; w < i1; w += kFusedWaves) pair_wave<Pass>(v, w, L.wave[uw]);
-    __syncthreads();
+                                          int uw, float4* L) {
+  const bool units = i1 - i0 <= kFusedUnits;
+  const int end = units ? S.unit0 + S.n_units : i1, step = units ? kFusedGroups : kFusedWaves;
+  for (int k = units ? S.unit0 : i0 + wave; k < end; k += step) {
+    if (units && k + grp >= end) {  // the barriers that the unit would have held
+      __syncthreads();
+      __syncthreads();
+    } else {
+      const PairUnit u = units ? unit_of(v, k + grp) : PairUnit{k, 1, 1};
+      pair_unit<Pass, kUnitWaves, true>(v, u, units ? uw : 0, units, units ? L : L + uw * kAnyWaveLds);
+    }
+    if (units) __syncthreads();
   }
+  if (!units) __syncthreads();
 }
 
 // Block b: the b-th listed system, ranges row b (item_b, item_e, a0, n, then
 // the bonded ranges).
 __global__ __launch_bounds__(kFusedThreads) void k_fused_steps(DeviceView v, const int32_t* ranges, int n_steps) {
-  __shared__ UnitLds<kPairLds> ulds[kFusedGroups];
+  __shared__ float4 ulds[kFusedGroups][kAnyGroupLds];
   __shared__ GatherLds glds[kFusedGroups];
   const int32_t* R = ranges + (size_t)blockIdx.x * kRangeInts;
   const int a0 = R[2], n = R[3];
@@ -93,7 +96,7 @@ __global__ __launch_bounds__(kFusedThreads) void k_fused_steps(DeviceView v, con
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int grp = wave / kGW;
   const int uw = unit_wave();
-  UnitLds<kPairLds>& L = ulds[grp];
+  float4* const L = ulds[grp];
   GatherLds& G = glds[grp];
 
   // B A O A of the first step from the stored force, then the tile boxes
@@ -106,14 +109,14 @@ __global__ __launch_bounds__(kFusedThreads) void k_fused_steps(DeviceView v, con
     bonded_slot(v, R);
     pair_pass<BornPass>(v, S, R[0], R[1], wave, grp, uw, L);
     for (int t = t0; t < t1; t += kFusedGroups)
-      group_round<1>(t, t1, grp, [&](int tt) { born_gather_tile(v, tt, G); });
+      gather_round(t, t1, grp, [&](int tt) { born_gather_tile(v, tt, G); });
     pair_pass<ForcePass<false>>(v, S, R[0], R[1], wave, grp, uw, L);
     for (int t = t0; t < t1; t += kFusedGroups)
-      group_round<1>(t, t1, grp, [&](int tt) { force_gather_tile<false>(v, tt, G); });
+      gather_round(t, t1, grp, [&](int tt) { force_gather_tile<false>(v, tt, G); });
     pair_pass<ChainPass>(v, S, R[0], R[1], wave, grp, uw, L);
     const int mode = k + 1 == n_steps ? 2 : 1;  // the last step stops after B(F)
     for (int t = t0; t < t1; t += kFusedGroups)
-      group_round<1>(t, t1, grp, [&](int tt) { chain_gather_tile(v, tt, mode, G); });
+      gather_round(t, t1, grp, [&](int tt) { chain_gather_tile(v, tt, mode, G); });
   }
 }
 

@@ -249,8 +249,8 @@ void build_exclusions(const prx_system_desc& d, ExclPlan& plan) {
   }
 }
 
-// Shares of every item of a system of nT tiles.
-static int item_shares(int nT) { return nT <= kQuarterTiles ? kUnitWaves : (nT <= kHalfTiles ? 2 : 1); }
+// Row shares of every item of a system of nT tiles.
+static int item_shares(int nT) { return nT <= kHalfTiles ? 2 : 1; }
 
 void build_items(int n_atoms, int a0, int slot, const ExclPlan& plan, int excl_base,
                  std::vector<PairItem>& out) {
@@ -281,12 +281,12 @@ void build_items(int n_atoms, int a0, int slot, const ExclPlan& plan, int excl_b
     }
 }
 
-int append_units(const std::vector<PairItem>& items, int base, std::vector<PairUnit>& out) {
-  if (items.empty()) return 0;
-  const int shares = items[0].nsub, per = kUnitWaves / shares, n = (int)items.size();
+int append_units(const std::vector<PairItem>& items, int nT, size_t list, int base, std::vector<PairUnit>& out) {
+  const int waves = nT > kHalfTiles ? 1 : (list >= kQuarterItems ? 2 : kUnitWaves);
+  const int per = kUnitWaves / waves, n = (int)items.size();
   for (int k = 0; k < n; k += per)
-    out.push_back({base + k, (int16_t)std::min(per, n - k), (int16_t)shares});
-  return shares;
+    out.push_back({base + k, (int16_t)std::min(per, n - k), (int16_t)waves});
+  return waves;
 }
 
 namespace {

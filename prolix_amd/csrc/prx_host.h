@@ -23,9 +23,9 @@ void build_exclusions(const prx_system_desc& d, ExclPlan& plan);
 void build_items(int n_atoms, int a0, int slot, const ExclPlan& plan, int excl_base,
                  std::vector<PairItem>& out);
 
-// Appends the units of one system's items, whose first has index base. Returns
-// the shares of each (0: no items).
-int append_units(const std::vector<PairItem>& items, int base, std::vector<PairUnit>& out);
+// Appends the units of the items of a system of nT tiles, whose first has index
+// base in a work list of `list` items. Returns the waves per item.
+int append_units(const std::vector<PairItem>& items, int nT, size_t list, int base, std::vector<PairUnit>& out);
 
 // Work layout of a neighbour-list system (relative to the system: item
 // indices from its first item, entries from its entry base, tiles local).

@@ -31,47 +31,58 @@
 
 namespace prx {
 
-// Blocks of WAVES waves: 1 (an item each), 2 (an item in two shares each) or
-// kUnitWaves (a unit each).
-template <int WAVES>
-constexpr int kThreads = 64 * WAVES;
+// Blocks of the pair kernels: one, two or four waves that take an item each, or
+// four waves that take a unit of the list (items of systems that differ in waves
+// per item).
+enum { kWaveBlocks = 1, kPairBlocks = 2, kQuadBlocks = 4, kUnitBlocks = 0 };
+template <int BLOCKS>
+constexpr int kThreads = 64 * (BLOCKS == kUnitBlocks ? kUnitWaves : BLOCKS);
 
-template <int WAVES, class Pass>
+template <int BLOCKS, class Pass>
 __device__ __forceinline__ void pair_block(const DeviceView& v, int b, int nb) {
-  if constexpr (WAVES == 1) {
-    __shared__ float4 mem[Pass::kLds];
-    pair_wave<Pass>(v, unit_id(v, b, nb), mem);
+  const int i = unit_id(v, b, nb);
+  if constexpr (BLOCKS == kWaveBlocks) {
+    __shared__ float4 mem[kWaveLds<Pass>];
+    pair_wave<Pass>(v, i, mem);
+  } else if constexpr (BLOCKS == kPairBlocks) {
+    __shared__ float4 mem[2 * kWaveLds<Pass>];
+    pair_unit<Pass, 2, false>(v, PairUnit{i, 1, 2}, unit_wave<2>(), true, mem);
+  } else if constexpr (BLOCKS == kQuadBlocks) {
+    __shared__ float4 mem[Pass::Quarter::kSize];
+    pair_unit<Pass, kUnitWaves, false, true>(v, PairUnit{i, 1, kUnitWaves}, unit_wave(), true, mem);
   } else {
-    __shared__ UnitLds<Pass::kLds, WAVES> mem;
-    pair_unit<false, Pass>(v, unit_id(v, b, nb), unit_wave<WAVES>(), mem);
+    __shared__ float4 mem[kGroupLds<Pass>];
+    const PairUnit u = v.units[i];
+    pair_unit<Pass, kUnitWaves, false>(v, u, unit_wave(), u.shares > 1, mem);
   }
 }
 
-template <int WAVES>
-__global__ __launch_bounds__(kThreads<WAVES>) PRX_OCCUPANCY void k_born_pairs(DeviceView v) {
-  pair_block<WAVES, BornPass>(v, blockIdx.x, gridDim.x);
+template <int BLOCKS>
+__global__ __launch_bounds__(kThreads<BLOCKS>) PRX_OCCUPANCY void k_born_pairs(DeviceView v) {
+  pair_block<BLOCKS, BornPass>(v, blockIdx.x, gridDim.x);
 }
 
-template <int WAVES, bool ENERGY>
-__global__ __launch_bounds__(kThreads<WAVES>) PRX_FORCE_OCCUPANCY(WAVES, ENERGY) void k_force_pairs(DeviceView v) {
-  pair_block<WAVES, ForcePass<ENERGY>>(v, blockIdx.x, gridDim.x);
+template <int BLOCKS, bool ENERGY>
+__global__ __launch_bounds__(kThreads<BLOCKS>) PRX_FORCE_OCCUPANCY(BLOCKS, ENERGY) void k_force_pairs(DeviceView v) {
+  pair_block<BLOCKS, ForcePass<ENERGY>>(v, blockIdx.x, gridDim.x);
 }
 
-template <int WAVES>
-__global__ __launch_bounds__(kThreads<WAVES>) PRX_OCCUPANCY void k_chain_pairs(DeviceView v) {
-  pair_block<WAVES, ChainPass>(v, blockIdx.x, gridDim.x);
+template <int BLOCKS>
+__global__ __launch_bounds__(kThreads<BLOCKS>) PRX_OCCUPANCY void k_chain_pairs(DeviceView v) {
+  pair_block<BLOCKS, ChainPass>(v, blockIdx.x, gridDim.x);
 }
 
 // The chain pass with the energy reduction in the same launch: blocks below
 // n_slots take a system's energies each, which are complete before the pass, the
-// rest the pass's units.
-__global__ __launch_bounds__(kThreads<kUnitWaves>) void k_chain_pairs_energies(DeviceView v, const int32_t* ranges,
-                                                                               int n_slots, double* out) {
+// rest the pass's items or units.
+template <int BLOCKS>
+__global__ __launch_bounds__(kThreads<BLOCKS>) void k_chain_pairs_energies(DeviceView v, const int32_t* ranges,
+                                                                           int n_slots, double* out) {
   const int b = (int)blockIdx.x;
   if (b < n_slots)
-    energy_reduce_block<kThreads<kUnitWaves>>(v, ranges, b, out);
+    energy_reduce_block<kThreads<BLOCKS>>(v, ranges, b, out);
   else
-    pair_block<kUnitWaves, ChainPass>(v, b - n_slots, (int)gridDim.x - n_slots);
+    pair_block<BLOCKS, ChainPass>(v, b - n_slots, (int)gridDim.x - n_slots);
 }
 
 // The Born pass with the bonded terms in the same launch: blocks below
@@ -80,42 +91,42 @@ __global__ __launch_bounds__(kThreads<kUnitWaves>) void k_chain_pairs_energies(D
 // bonded records are read by the chain gather, so the merged launch saves the
 // bonded kernel's graph node where that kernel would run in line; results are
 // bit for bit those of the two kernels.
-template <int WAVES, bool ENERGY>
-__global__ __launch_bounds__(kThreads<WAVES>) PRX_OCCUPANCY void k_born_pairs_bonded(DeviceView v, int n_pair) {
+template <int BLOCKS, bool ENERGY>
+__global__ __launch_bounds__(kThreads<BLOCKS>) PRX_OCCUPANCY void k_born_pairs_bonded(DeviceView v, int n_pair) {
   const int b = (int)blockIdx.x;
   if (b < n_pair) {
-    pair_block<WAVES, BornPass>(v, b, n_pair);
+    pair_block<BLOCKS, BornPass>(v, b, n_pair);
     return;
   }
-  const int e = (b - n_pair) * kThreads<WAVES> + (int)threadIdx.x;
+  const int e = (b - n_pair) * kThreads<BLOCKS> + (int)threadIdx.x;
   if (e < bonded_entries(v)) bonded_entry<ENERGY>(v, e);
 }
 
-// Waves per block: an item per wave in a long list or where every item is
-// whole, two per item where every item is in two shares, else units. Two-wave
-// blocks free their slots as soon as one item is done, and read no unit list:
+// Blocks of a list: an item per wave in a long list or where every item is
+// whole, two or four waves per item where every item takes as many, else units.
+// Two-wave blocks free their slots as soon as one item is done, and read no unit list:
 // 8,000 atoms 144 us an evaluation, 148 with units of two items.
-static inline int block_waves(const DeviceView& v) {
-  return v.n_items >= kWaveItems ? 1 : (v.shares > 0 ? v.shares : kUnitWaves);
-}
-static inline int pair_blocks(const DeviceView& v, int waves) { return waves < kUnitWaves ? v.n_items : v.n_units; }
+static inline int list_blocks(const DeviceView& v) { return v.shares; }
+static inline int pair_blocks(const DeviceView& v, int blocks) { return blocks == kUnitBlocks ? v.n_units : v.n_items; }
 
-// launch(std::integral_constant<int, WAVES>) with the list's block_waves.
+// launch(std::integral_constant<int, BLOCKS>) with the list's blocks.
 template <class F>
-static void by_waves(const DeviceView& v, F&& launch) {
-  switch (block_waves(v)) {
-    case 1: return launch(std::integral_constant<int, 1>());
-    case 2: return launch(std::integral_constant<int, 2>());
-    default: return launch(std::integral_constant<int, kUnitWaves>());
+static void by_blocks(const DeviceView& v, F&& launch) {
+  static_assert(kQuadBlocks == kUnitWaves, "shares name the blocks");
+  switch (list_blocks(v)) {
+    case kWaveBlocks: return launch(std::integral_constant<int, kWaveBlocks>());
+    case kPairBlocks: return launch(std::integral_constant<int, kPairBlocks>());
+    case kQuadBlocks: return launch(std::integral_constant<int, kQuadBlocks>());
+    default: return launch(std::integral_constant<int, kUnitBlocks>());
   }
 }
 
 template <bool ENERGY>
 static void born_pairs_bonded(const DeviceView& v, hipStream_t s) {
-  by_waves(v, [&](auto w) {
-    constexpr int W = decltype(w)::value, nt = kThreads<W>;
-    const int np = pair_blocks(v, W), nb = np + (bonded_entries(v) + nt - 1) / nt;
-    if (nb > 0) hipLaunchKernelGGL((k_born_pairs_bonded<W, ENERGY>), dim3(nb), dim3(nt), 0, s, v, np);
+  by_blocks(v, [&](auto b) {
+    constexpr int B = decltype(b)::value, nt = kThreads<B>;
+    const int np = pair_blocks(v, B), nb = np + (bonded_entries(v) + nt - 1) / nt;
+    if (nb > 0) hipLaunchKernelGGL((k_born_pairs_bonded<B, ENERGY>), dim3(nb), dim3(nt), 0, s, v, np);
   });
 }
 
@@ -128,17 +139,17 @@ void launch_born_pairs_bonded(const DeviceView& v, bool energy, hipStream_t s) {
 
 void launch_born_pairs(const DeviceView& v, hipStream_t s) {
   if (v.n_items == 0) return;
-  by_waves(v, [&](auto w) {
-    constexpr int W = decltype(w)::value;
-    hipLaunchKernelGGL(k_born_pairs<W>, dim3(pair_blocks(v, W)), dim3(kThreads<W>), 0, s, v);
+  by_blocks(v, [&](auto b) {
+    constexpr int B = decltype(b)::value;
+    hipLaunchKernelGGL(k_born_pairs<B>, dim3(pair_blocks(v, B)), dim3(kThreads<B>), 0, s, v);
   });
 }
 
 template <bool ENERGY>
 static void force_pairs(const DeviceView& v, hipStream_t s) {
-  by_waves(v, [&](auto w) {
-    constexpr int W = decltype(w)::value;
-    hipLaunchKernelGGL((k_force_pairs<W, ENERGY>), dim3(pair_blocks(v, W)), dim3(kThreads<W>), 0, s, v);
+  by_blocks(v, [&](auto b) {
+    constexpr int B = decltype(b)::value;
+    hipLaunchKernelGGL((k_force_pairs<B, ENERGY>), dim3(pair_blocks(v, B)), dim3(kThreads<B>), 0, s, v);
   });
 }
 
@@ -152,9 +163,9 @@ void launch_force_pairs(const DeviceView& v, bool energy, hipStream_t s) {
 
 void launch_chain_pairs(const DeviceView& v, hipStream_t s) {
   if (v.n_items == 0) return;
-  by_waves(v, [&](auto w) {
-    constexpr int W = decltype(w)::value;
-    hipLaunchKernelGGL(k_chain_pairs<W>, dim3(pair_blocks(v, W)), dim3(kThreads<W>), 0, s, v);
+  by_blocks(v, [&](auto b) {
+    constexpr int B = decltype(b)::value;
+    hipLaunchKernelGGL(k_chain_pairs<B>, dim3(pair_blocks(v, B)), dim3(kThreads<B>), 0, s, v);
   });
 }
 
@@ -165,9 +176,16 @@ void launch_chain_pairs(const DeviceView& v, hipStream_t s) {
 // other lists' blocks of 64 or 128 threads would take two or four times as long
 // over a system.
 bool launch_chain_pairs_energies(const DeviceView& v, const int32_t* ranges, int n_slots, double* out, hipStream_t s) {
-  if (v.n_items == 0 || block_waves(v) != kUnitWaves) return false;
-  hipLaunchKernelGGL(k_chain_pairs_energies, dim3(n_slots + v.n_units), dim3(kThreads<kUnitWaves>), 0, s, v, ranges,
-                     n_slots, out);
+  if (v.n_items == 0) return false;
+  const int blocks = list_blocks(v);
+  if (blocks == kQuadBlocks)
+    hipLaunchKernelGGL(k_chain_pairs_energies<kQuadBlocks>, dim3(n_slots + v.n_items), dim3(kThreads<kQuadBlocks>), 0, s,
+                       v, ranges, n_slots, out);
+  else if (blocks == kUnitBlocks)
+    hipLaunchKernelGGL(k_chain_pairs_energies<kUnitBlocks>, dim3(n_slots + v.n_units), dim3(kThreads<kUnitBlocks>), 0, s,
+                       v, ranges, n_slots, out);
+  else
+    return false;
   return true;
 }
 

@@ -20,15 +20,22 @@
 // per lane and iteration (64 rotations of the j sums through DPP or
 // ds_bpermute, 1-2 LDS reads an iteration) bound the force pass by LDS: 40 of
 // its 40 cycles per CU and iteration. A patch takes 26 (Born, average of its
-// classes), 48 (force) and 37 (chain) VALU instructions, where an iteration
-// took 40 to 50. 256 systems of 300 to 5,000 atoms, us a pass (Born, force,
-// chain): 376, 609, 486 then, 322, 624, 457 now; one system of 2,500 atoms: 23.3,
-// 23.2, 32.7 then, 14.1, 11.8, 15.3 now.
+// classes), 46 (force) and 37 (chain) VALU instructions, where an iteration
+// took 40 to 50. 256 compact systems of 300 to 5,000 atoms, us a pass (Born, force,
+// chain): 424, 655, 533 then, 373, 643, 501 now; one system of 2,500 atoms: 23.0,
+// 18.9, 32.1 then, 10.4, 10.7, 12.6 now.
 #pragma once
+
+#include <type_traits>
 
 #include "prx_common.h"
 #include "prx_lanes_dev.h"
 #include "prx_obc_farfield.h"
+
+// Multiply-adds are fused only where the code says so: the sums of an item are the same
+// on one, two and four waves only if each of their instances rounds alike, and left to
+// itself the compiler fuses either product of a b + c d.
+#pragma clang fp contract(off)
 
 namespace prx {
 
@@ -69,27 +76,43 @@ __device__ __forceinline__ void wave_lds_sync() {
 #endif
 #if PRX_MIN_WAVES > 0
 #define PRX_OCCUPANCY __attribute__((amdgpu_waves_per_eu(PRX_MIN_WAVES)))
-#define PRX_FORCE_OCCUPANCY(WAVES, ENERGY) PRX_OCCUPANCY
+#define PRX_FORCE_OCCUPANCY(BLOCKS, ENERGY) PRX_OCCUPANCY
 #else
 #define PRX_OCCUPANCY
-// The force pass: four waves per SIMD where a wave takes an item, five where
-// work lists are short (256 systems of 300 to 5,000 atoms 613 and 628 us, one of
-// 8,000 atoms 49.5 and 48.0), without a spill. With energies four (128 VGPRs; its
-// free choice is 144: 64 systems of up to 5,000 atoms 526 us an evaluation, 519).
-#define PRX_FORCE_OCCUPANCY(WAVES, ENERGY) __attribute__((amdgpu_waves_per_eu(ENERGY || WAVES == 1 ? 4 : 5)))
+// The force pass: five waves per SIMD, without a spill (one system of 8,000 atoms 49.5
+// us with four, 48.0); four with energies (five spill 15 registers: 256 systems of 300 to
+// 5,000 atoms 1,950 us an evaluation, 2,065) and where a wave takes an item or a unit of any
+// kind.
+#define PRX_FORCE_OCCUPANCY(BLOCKS, ENERGY) \
+  __attribute__((amdgpu_waves_per_eu(ENERGY || BLOCKS == 1 || BLOCKS == 0 ? 4 : 5)))
 #endif
 #define PRX_PRAGMA(x) _Pragma(#x)
 #define PRX_UNROLL(n) PRX_PRAGMA(unroll n)
 
-constexpr int kEdge = 8;  // edge of a patch
+constexpr int kEdge = 8;          // edge of a patch
+// Half h of an item's columns: the columns of patches a = h, h + 2, ... (neighbours in the
+// sequence are near in a corner of the item, which left and right halves would give
+// to one of them).
+constexpr int kHalf = kEdge / 2;
+// Half of column k of COLS (all, or those of one half).
+template <int COLS>
+__device__ constexpr int half_of(int k) { return COLS == kHalf ? 0 : k & 1; }
 
-// Index x, hidden from the optimiser and ready only once y is: the columns are
-// read from LDS at such an index, so that column a is read while column a - 1
+typedef float4 Tile4[kTile];
+constexpr int kByte = sizeof(float4);
+
+// Byte offset x, hidden from the optimiser and ready only once y is: the columns
+// are read from LDS at such an offset, so that column a is read while column a - 1
 // is evaluated. Left alone, the compiler reads all eight ahead of the row loop
-// and keeps them, 8 x 8 to 12 registers that cost half the waves.
+// and keeps them, 8 x 8 to 12 registers that cost half the waves. (Of an index
+// each read would shift a new one.)
 __device__ __forceinline__ int after(int x, float y) {
   asm volatile("" : "+v"(x) : "v"(y));
   return x;
+}
+// Element at byte offset x of plane k of a staged tile.
+__device__ __forceinline__ const float4& at_byte(const Tile4* t, int k, int x) {
+  return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(t[k]) + x);
 }
 
 // Position of the lanes past the end of a ragged tile: so far away that every
@@ -130,6 +153,15 @@ __device__ __forceinline__ float sum_q(const float (&v)[kEdge], int lane) {
   const bool odd = (lane & 8) != 0;
   return (odd ? g[1] : g[0]) + dpp<kDppRor8>(odd ? g[0] : g[1]);
 }
+// The same for the four columns of a half, in the same order of additions: lane l
+// gets column l / 16 of them, atom half_col(l) of the half's 32.
+__device__ __forceinline__ float sum_q(const float (&v)[kHalf], int) {
+  const float g = add_swap16(add_swap32(v[0], v[2]), add_swap32(v[1], v[3]));
+  return g + dpp<kDppRor8>(g);
+}
+__device__ __forceinline__ int half_col(int lane) { return kEdge * (lane >> 4) + (lane & 7); }
+// Tile's atom i of the 32 of half h.
+__device__ __forceinline__ int half_atom(int h, int i) { return 2 * (i & ~7) + kEdge * h + (i & 7); }
 
 // The j atoms of an item: a tile (gj = j0 + lane), or for a chunk item of a
 // neighbour list up to 64 listed atoms (gj = the lane's entry). nj = 0: an
@@ -203,10 +235,11 @@ __device__ __forceinline__ float born_dr(float r, float rs, float rho, float s, 
   const float iL = Uc * inv, iU = Lc * inv;
   const float lg = flog2(Lc * iU) * kLn2;
   const float iL2 = iL * iL, iU2 = iU * iU;
-  const float d1 = 0.5f * (Up * iU2 - Lp * iL2);
-  const float d2 = 0.25f * rs * ((Lp * iL - Up * iU) - lg * rp * rs);
+  // Lp and Up are 0 or 1 in size, so these products are exact
+  const float d1 = 0.5f * fmaf(Up, iU2, -(Lp * iL2));
+  const float d2 = 0.25f * rs * fmaf(-(lg * rp), rs, fmaf(Lp, iL, -(Up * iU)));
   const float d3 = 0.125f * fmaf(s2 * rp, rs * rs, 1.0f) * (iU2 - iL2);
-  const float d4 = 0.25f * fmaf(-s2, rs, r) * (Lp * iL2 * iL - Up * iU2 * iU);
+  const float d4 = 0.25f * fmaf(-s2, rs, r) * fmaf(Lp * iL2, iL, -(Up * iU2 * iU));
   // Every intermediate is finite (Lc, Uc >= 1e-4), so a 0/1 factor is exact
   // and keeps the wave free of a divergent branch.
   const float on = (U > rho) ? 1.0f : 0.0f;
@@ -283,12 +316,29 @@ __device__ __forceinline__ float horner(const float (&w)[N], float u) {
 // Pass 1: Born sums
 // ---------------------------------------------------------------------------
 
-// One wave's LDS in float4: the rows (tile I) and columns (tile J) of its item,
-// two per atom, and a scratch list of 64 for the near pairs and the column sums
-// (force: with the energies). 5 KB let eight waves of a SIMD run.
-constexpr int kBornLds = 5 * kTile, kForceLds = 5 * kTile + 2, kChainLds = 5 * kTile;
-constexpr int kPairLds = kForceLds;  // of any pass
-typedef float4 Tile4[kTile];
+// LDS in float4: the rows (tile I) and columns (tile J) of an item, two per atom,
+// and per wave a scratch list: 64 for the near pairs, later the sums that go to
+// another wave ("Items to waves" below).
+constexpr int kTilesLds = 4 * kTile;
+
+// Scratch of a wave in float4: 64 for the list, later C sums of 64 rows (or, of a
+// diagonal item, atoms) and of 32 columns.
+template <int C>
+constexpr int kObcScratch = C * (kTile + kTile / 2) / 4 > kTile ? C * (kTile + kTile / 2) / 4 : kTile;
+// Memory of four waves that share an item: its tiles, per wave the lanes' sums of
+// its four rows of patches (C sums each), per wave its scratch.
+template <int C, int SCRATCH = kObcScratch<C>>
+struct QuarterLds {
+  static constexpr int kRowsLds = C * kHalf * 64 / 4;
+  static constexpr int kSize = kTilesLds + 4 * (kRowsLds + SCRATCH);
+  __device__ static __forceinline__ float* rows(float4* M, int k) {
+    return reinterpret_cast<float*>(M + kTilesLds + k * kRowsLds);
+  }
+  __device__ static __forceinline__ float4* scratch(float4* M, int k) {
+    return M + kTilesLds + 4 * kRowsLds + k * SCRATCH;
+  }
+};
+
 
 // An atom of the Born pass. Short: the tiers of at most five coefficients,
 // (x, y, z, w0), (w1, w2, w3, w4). The others keep (x, y, z, s^2), (s^3/3, rho,
@@ -314,17 +364,17 @@ struct BornAtom {
     }
   }
   // row: with its weights
-  __device__ __forceinline__ void read(const Tile4* t, int e, bool row) {
-    const float4 a = t[0][e];
+  __device__ __forceinline__ void read(const Tile4* t, int byte, bool row) {
+    const float4 a = at_byte(t, 0, byte);
     x = a.x; y = a.y; z = a.z;
     if constexpr (kShort) {
-      const float4 b = t[1][e];
+      const float4 b = at_byte(t, 1, byte);
       w[0] = a.w; w[1] = b.x; w[2] = b.y;
       if constexpr (N > 3) w[3] = b.z;
       if constexpr (N > 4) w[4] = b.w;
     } else {
       s2 = a.w;
-      s33 = t[1][e].x;
+      s33 = at_byte(t, 1, byte).x;
       if (row) obc_weights<BornW<CLS>>(s2, s33, w);
     }
   }
@@ -342,23 +392,29 @@ __device__ __forceinline__ float prev_below(float x) { return __int_as_float(__f
 // near (bit 8 b + a).
 //
 // Off the diagonal they are few (on proteins a tenth of the patches hold one,
-// and three lanes of 64 in those: 20 to 40 pairs an item). They are listed
-// first and then evaluated 64 at a time, a pair per lane, by eval(row, col),
-// which returns the pair's terms; then every lane adds, in list order, the terms
-// of its row 8 p + q and of its column (lane) by row(terms, mine) and col(terms,
-// mine), factors of 1 or 0. Terms that are not finite (two atoms at one point), which
-// a factor of 0 would hand to every row and column, are added by selects behind
-// their batch instead (selects for every term: 1.4% of the chain pass of 256
-// systems of 300 to 5,000 atoms).
-template <class Eval, class Row, class Col>
+// and three lanes of 64 in those: 20 to 40 pairs an item). They are listed first and
+// evaluated 64 at a time, a pair per lane, by eval(row, col); then every lane adds,
+// in list order, the terms of its row 8 p + q and of its column my_col by
+// add_row(half, terms, mine) and add_col(terms, mine), factors of 1 or 0. Terms that are
+// not finite (two atoms at one point), which a factor of 0 would hand to every row and
+// column, are added by selects behind their batch instead (selects for every term:
+// 1.4% of the chain pass of 256 systems of 300 to 5,000 atoms).
+// HALVES: near holds patches of both halves, whose row sums are kept apart: those of
+// half 1 are listed from the other end of the scratch and evaluated in the lanes
+// behind the first's, from a multiple of kBatch on, so that the loops that add
+// need no test (a branch per entry on its half: 1.5 us of 9.3 of the Born pass of 138
+// atoms, whose waves wait for the scalar unit).
+template <bool HALVES, class Eval, class Row, class Col>
 __device__ __forceinline__ void near_list(const Tile4* ti, const Tile4* tj, unsigned long long near, int lane,
-                                          bool cut, float lim2, float4* scratch, Eval&& eval, Row&& add_row,
-                                          Col&& add_col) {
+                                          int my_col, bool cut, float lim2, float4* scratch, Eval&& eval,
+                                          Row&& add_row, Col&& add_col) {
+  constexpr int kBatch = 4;  // entries read before any is added
+  constexpr int kList = 128;
   const int p = lane & 7, q = lane >> 3, my_row = kEdge * p + q;
   unsigned short* const list = reinterpret_cast<unsigned short*>(scratch);
-  int count = 0;
-  while (near != 0 || count > 0) {
-    while (near != 0 && count < 64) {
+  int count[2] = {0, 0};
+  for (;;) {
+    while (near != 0 && count[0] + count[1] < 64) {
       const int k = __builtin_ctzll(near), row = (k & 56) + q, col = kEdge * (k & 7) + p;
       near &= near - 1;
       const float4 a = ti[0][row], b = tj[0][col];
@@ -366,56 +422,77 @@ __device__ __forceinline__ void near_list(const Tile4* ti, const Tile4* tj, unsi
       const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
       const bool on = cut ? r2 <= lim2 : !(r2 > lim2);
       const unsigned long long m = __ballot(on);
-      const int at = count + (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32),
-                                                            __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+      const bool back = HALVES && (k & 1);
+      int at = (int)__builtin_amdgcn_mbcnt_hi((unsigned)(m >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)m, 0u));
+      at = back ? kList - 1 - count[1] - at : count[0] + at;
       if (on) list[at] = (unsigned short)(row << 6 | col);
-      count += __popcll(m);
+      count[0] += back ? 0 : __popcll(m);
+      count[1] += back ? __popcll(m) : 0;
     }
-    if (count == 0) break;
+    if (count[0] + count[1] == 0) break;
     wave_lds_sync();
-    const int n = min(count, 64);
-    const int e = list[min(lane, n - 1)], rest = list[64 + lane];
+    const int n0 = min(count[0], 64), b1 = (n0 + kBatch - 1) & -kBatch;  // lanes of half 0, first lane of half 1
+    const int n1 = HALVES ? min(count[1], 64 - b1) : 0;
+    const bool on = lane < n0 || (HALVES && lane >= b1 && lane < b1 + n1);
+    int e = list[HALVES && lane >= b1 ? kList - 1 - (lane - b1) : min(lane, max(n0 - 1, 0))];
+    int rest0 = 0, rest1 = 0;
+    if (HALVES) {
+      rest0 = list[min(64 + lane, kList - 1)];
+      rest1 = list[max(kList - 1 - n1 - lane, 0)];
+      e = on ? e : 0;
+    } else {
+      rest0 = list[64 + lane];
+    }
     wave_lds_sync();
     const float3 t = eval(e >> 6, e & 63);
-    const bool on = lane < n, sound = fabsf(t.x) + fabsf(t.y) + fabsf(t.z) < INFINITY;
+    const bool sound = fabsf(t.x) + fabsf(t.y) + fabsf(t.z) < INFINITY;
     scratch[lane] = make_float4(sound ? t.x : 0.0f, sound ? t.y : 0.0f, sound ? t.z : 0.0f,
                                 __int_as_float(on ? e : -1));
     wave_lds_sync();
-    constexpr int kBatch = 4;  // entries read before any is added
-    for (int k = 0; k < n; k += kBatch) {
-      float4 c[kBatch];
+    const auto add = [&](int from, int to, auto half) {
+      for (int k = from; k < to; k += kBatch) {
+        float4 c[kBatch];
 #pragma unroll
-      for (int m = 0; m < kBatch; ++m) c[m] = scratch[k + m];
+        for (int m = 0; m < kBatch; ++m) c[m] = scratch[k + m];
 #pragma unroll
-      for (int m = 0; m < kBatch; ++m) {
-        const int ce = __float_as_int(c[m].w);
-        add_row(c[m], (ce >> 6) == my_row ? 1.0f : 0.0f);
-        add_col(c[m], ce >= 0 && (ce & 63) == lane ? 1.0f : 0.0f);
+        for (int m = 0; m < kBatch; ++m) {
+          const int ce = __float_as_int(c[m].w);
+          add_row(half, c[m], (ce >> 6) == my_row ? 1.0f : 0.0f);
+          add_col(c[m], ce >= 0 && (ce & 63) == my_col ? 1.0f : 0.0f);
+        }
       }
-    }
+    };
+    add(0, n0, std::integral_constant<int, 0>());
+    if (HALVES) add(b1, b1 + n1, std::integral_constant<int, 1>());
     for (unsigned long long m = __ballot(on && !sound); m != 0; m &= m - 1) {
       const int k = __builtin_ctzll(m), ce = __builtin_amdgcn_readlane(e, k);
       const float4 c = make_float4(__shfl(t.x, k), __shfl(t.y, k), __shfl(t.z, k), 0.0f);
       const float4 zero = make_float4(0.f, 0.f, 0.f, 0.f);
-      add_row((ce >> 6) == my_row ? c : zero, 1.0f);
-      add_col((ce & 63) == lane ? c : zero, 1.0f);
+      add_row(std::integral_constant<int, 0>(), (ce >> 6) == my_row ? c : zero, 1.0f);
+      add_col((ce & 63) == my_col ? c : zero, 1.0f);
     }
     wave_lds_sync();
-    count -= n;
-    if (lane < count) list[lane] = (unsigned short)rest;
+    count[0] -= n0;
+    count[1] -= n1;
+    if (lane < count[0]) list[lane] = (unsigned short)rest0;
+    if (HALVES && lane < count[1]) list[kList - 1 - lane] = (unsigned short)rest1;
   }
 }
 
-// On the diagonal a fifth of the pairs are near (14 to 20 per atom): each lane
-// walks the near atoms of its own atom (lane), on both sides of the diagonal,
-// so nothing is summed across lanes; eval(atoms, on) adds to the lane's sums. Of a
-// unit's waves, sub = 0 .. nsub - 1, each takes the atoms 8 b + q' of its rows.
-template <class Eval>
-__device__ __forceinline__ void near_diag(const Tile4* t, int lane, int ni, int sub, int nsub, bool cut, float lim2,
-                                          Eval&& eval) {
-  const float4 me = t[0][lane];
+// On the diagonal a fifth of the pairs are near (14 to 20 per atom): a lane walks
+// those of its own atom with the rows of share s, on both sides of the diagonal, so
+// nothing is summed across lanes. The even and the odd ones of them are summed
+// apart, by add(atom, near, on, sum, sum) two at a time (one is a chain of dependent
+// steps), so that an atom can have a lane of its own (atom = lane) or with SPLIT two: lanes
+// l and l + 32 take the even and the odd near atoms of atom l of half h and get its sum.
+template <bool SPLIT, int C, class Add>
+__device__ __forceinline__ void near_diag(const Tile4* t, int lane, int ni, int s, int nsub, int h, bool cut,
+                                          float lim2, Add&& add, float (&sum)[C]) {
+  const int second = SPLIT ? lane >> 5 : 0, atom = SPLIT ? half_atom(h, lane & 31) : lane;
+  const float4 me = t[0][atom];
   unsigned long long near = 0;
-  for (int b = sub; kEdge * b < ni; b += nsub) {
+  // two lanes test every other row of patches each
+  for (int b = s + nsub * second; kEdge * b < ni; b += SPLIT ? 2 * nsub : nsub) {
     unsigned bits = 0;
 #pragma unroll
     for (int k = 0; k < kEdge; ++k) {
@@ -423,23 +500,34 @@ __device__ __forceinline__ void near_diag(const Tile4* t, int lane, int ni, int 
       // the sign of the difference as in the pair loop: later atom minus earlier
       const float dx = o.x - me.x, dy = o.y - me.y, dz = o.z - me.z;
       const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-      const bool on = (cut ? r2 <= lim2 : !(r2 > lim2)) && kEdge * b + k != lane && kEdge * b + k < ni;
+      const bool on = (cut ? r2 <= lim2 : !(r2 > lim2)) && kEdge * b + k != atom && kEdge * b + k < ni;
       bits |= on ? 1u << k : 0u;
     }
     near |= (unsigned long long)bits << (kEdge * b);
   }
-  if (lane >= ni) near = 0;
-  while (__any(near != 0)) {  // two atoms at a time: one is a chain of dependent steps
+  if (SPLIT) {
+    const unsigned x = (unsigned)near, y = (unsigned)(near >> 32);
+    const auto lo = __builtin_amdgcn_permlane32_swap(x, x, false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap(y, y, false, false);
+    near = (unsigned long long)(hi[0] | hi[1]) << 32 | (lo[0] | lo[1]);
+    if (second) near &= near - 1;
+  }
+  if (atom >= ni) near = 0;
+  float even[C] = {}, odd[C] = {};
+  while (__any(near != 0)) {
     int o[2];
     bool on[2];
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
       on[k] = near != 0;
-      o[k] = on[k] ? __builtin_ctzll(near) : lane;
+      o[k] = on[k] ? __builtin_ctzll(near) : atom;
       near &= near - 1;
+      if (SPLIT) near &= near - 1;  // the other lane's
     }
-    eval(o, on);
+    add(atom, o, on, even, SPLIT ? even : odd);
   }
+#pragma unroll
+  for (int c = 0; c < C; ++c) sum[c] += SPLIT ? add_swap32(even[c], even[c]) : even[c] + odd[c];
 }
 
 // I(r; rho_i, s_j) alone, for a near or a far pair.
@@ -454,42 +542,34 @@ __device__ __forceinline__ float born_one(float r2, float rho_i, float s_j, floa
   return obc_far(r, rho_i, s_j) ? (u * u) * (s33_j * obc_poly<BornW<kMixed>>(s2_j * u)) : (U > rho_i ? I : 0.0f);
 }
 
-__device__ __forceinline__ void born_near(float4* L, float4* scratch, unsigned long long near, int lane, int ni, bool diag, bool cut,
-                                          float lim2, int sub, int nsub, float& rows, float& cols) {
-  Tile4* ti = reinterpret_cast<Tile4*>(L);
-  Tile4* tj = ti + 2;
-  if (diag) {
-    const float4 me = ti[0][lane];
-    const float rhoi = ti[1][lane].y;
-    near_diag(ti, lane, ni, sub, nsub, cut, lim2, [&](const int (&o)[2], const bool (&on)[2]) {
-      float I[2];
+// Near pairs of two atoms o of a diagonal item (near_diag).
+__device__ __forceinline__ void born_near_diag(const Tile4* t, int atom, const int (&o)[2], const bool (&on)[2],
+                                               float (&even)[1], float (&odd)[1]) {
+  const float4 me = t[0][atom];
+  const float rhoi = t[1][atom].y;
+  float I[2];
 #pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const float4 a = ti[0][o[k]], b = ti[1][o[k]];
-        const float dx = a.x - me.x, dy = a.y - me.y, dz = a.z - me.z;
-        I[k] = born_one(fmaf(dx, dx, fmaf(dy, dy, dz * dz)), rhoi, b.z, a.w, b.x);
-      }
-#pragma unroll
-      for (int k = 0; k < 2; ++k) cols += on[k] ? I[k] : 0.0f;
-    });
-    return;
+  for (int k = 0; k < 2; ++k) {
+    const float4 a = t[0][o[k]], b = t[1][o[k]];
+    const float dx = a.x - me.x, dy = a.y - me.y, dz = a.z - me.z;
+    I[k] = born_one(fmaf(dx, dx, fmaf(dy, dy, dz * dz)), rhoi, b.z, a.w, b.x);
   }
-  near_list(
-      ti, tj, near, lane, cut, lim2, scratch,
-      [&](int row, int col) {
-        const float4 ai = ti[0][row], bi = ti[1][row], aj = tj[0][col], bj = tj[1][col];
-        const float rhoi = bi.y, si = bi.z, rhoj = bj.y, sj = bj.z;
-        const float dx = aj.x - ai.x, dy = aj.y - ai.y, dz = aj.z - ai.z;
-        const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
-        const float rinv = frsq(r2);
-        const float u = rinv * rinv, u2 = u * u, r = r2 * rinv;
-        const BornPair bp = born_pair(r, rinv, rhoi, si, ai.w, rhoj, sj, aj.w);
-        const float I1 = obc_far(r, rhoi, sj) ? u2 * (bj.x * obc_poly<BornW<kMixed>>(aj.w * u)) : bp.I1;
-        const float I2 = obc_far(r, rhoj, si) ? u2 * (bi.x * obc_poly<BornW<kMixed>>(ai.w * u)) : bp.I2;
-        return make_float3(I1, I2, 0.0f);
-      },
-      [&](const float4& c, float mine) { rows = fmaf(mine, c.x, rows); },
-      [&](const float4& c, float mine) { cols = fmaf(mine, c.y, cols); });
+  even[0] += on[0] ? I[0] : 0.0f;
+  odd[0] += on[1] ? I[1] : 0.0f;
+}
+
+// Terms of a near pair off the diagonal: x to the row, y to the column.
+__device__ __forceinline__ float3 born_near_pair(const Tile4* ti, const Tile4* tj, int row, int col) {
+  const float4 ai = ti[0][row], bi = ti[1][row], aj = tj[0][col], bj = tj[1][col];
+  const float rhoi = bi.y, si = bi.z, rhoj = bj.y, sj = bj.z;
+  const float dx = aj.x - ai.x, dy = aj.y - ai.y, dz = aj.z - ai.z;
+  const float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
+  const float rinv = frsq(r2);
+  const float u = rinv * rinv, u2 = u * u, r = r2 * rinv;
+  const BornPair bp = born_pair(r, rinv, rhoi, si, ai.w, rhoj, sj, aj.w);
+  const float I1 = obc_far(r, rhoi, sj) ? u2 * (bj.x * obc_poly<BornW<kMixed>>(aj.w * u)) : bp.I1;
+  const float I2 = obc_far(r, rhoj, si) ? u2 * (bi.x * obc_poly<BornW<kMixed>>(ai.w * u)) : bp.I2;
+  return make_float3(I1, I2, 0.0f);
 }
 
 // The atoms of an item's tiles (or of one of them), loaded together: lane = atom.
@@ -520,34 +600,47 @@ __device__ __forceinline__ void pad_atoms(ItemAtoms& t, int lane, int ni, int nj
   if (lane >= nj) { t.pj = pad_pos(lane); t.bj = zero; t.cj = 0.0f; }
 }
 
-// The far pairs of rows b = sub, sub + nsub, ... of an item. rows: lane 8 q + p
-// gets the sum of row 8 p + q; cols: lane l that of column l over these rows.
+// The far pairs of the rows b = sub, sub + nsub, ... of an item with COLS columns
+// of patches: all eight (rows: lane 8 q + p gets the sum of row 8 p + q) or those of
+// half h (the lanes' row sums go to t, [row of the share][lane]). A row's sum is that
+// of its half 0 plus that of its half 1, lane by lane, so both ways give the same. cols: the columns' sums over these rows, as sum_q leaves them.
 // CUT: pairs with r^2 >= cut2 add nothing. FULL: both tiles hold 64 atoms.
 // thr2: above it every pair of the item is in the far field; a mixed item
 // adds only the pairs above it here and marks the patches of the others in
 // near, so that the loop has no branch and the registers of the far field alone.
-template <int CLS, bool DIAG, bool CUT, bool FULL>
+template <int CLS, bool DIAG, bool CUT, bool FULL, int COLS>
 __device__ __forceinline__ void born_tile(const float4* L, int ni, int nj, int lane, float cut2, float thr2, int sub,
-                                          int nsub, float& rows, float& cols, unsigned long long& near) {
+                                          int nsub, int h, float* t, float (&rows)[1], float (&cols)[1],
+                                          unsigned long long& near) {
   const Tile4* ti = reinterpret_cast<const Tile4*>(L);
   const Tile4* tj = ti + 2;
   const int p = lane & 7, q = lane >> 3;
-  float accj[kEdge] = {};
+  float accj[COLS] = {};
+  BornAtom<CLS> half_cols[kHalf];  // of half h, kept over the rows
+  if (COLS == kHalf)
+#pragma unroll
+    for (int k = 0; k < kHalf; ++k) half_cols[k].read(tj, kByte * (p + kEdge * (2 * k + h)), false);
   const int nb = FULL ? kEdge : (ni + kEdge - 1) / kEdge, na = FULL ? kEdge : (nj + kEdge - 1) / kEdge;
   PRX_UNROLL(PRX_UNROLL_BORN)
   for (int b = sub; b < nb; b += nsub) {
     BornAtom<CLS> i;
-    float acci = 0.0f;
-    i.read(ti, kEdge * b + q, true);
+    float half[2] = {};
+    i.read(ti, kByte * (kEdge * b + q), true);
     unsigned marks = 0;
-    int col = p;
+    int col = kByte * p;
 #pragma unroll
-    for (int a = 0; a < kEdge; ++a) {
-      if (!FULL && a >= na) break;
+    for (int k = 0; k < COLS; ++k) {
+      const int a = COLS == kHalf ? 2 * k + h : k;
+      if (!FULL && a >= na) continue;
       if (DIAG && a < b) continue;
+      float& acci = half[half_of<COLS>(k)];
       BornAtom<CLS> j;
-      col = after(col, a < 2 ? acci : accj[a - 2]);
-      j.read(tj, col + kEdge * a, false);
+      if constexpr (COLS == kHalf) {
+        j = half_cols[k];
+      } else {
+        col = after(col, k < 2 ? acci : accj[k - 2]);
+        j.read(tj, col + kByte * kEdge * k, false);
+      }
       const float dx = j.x - i.x, dy = j.y - i.y, dz = j.z - i.z;
       float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
       if (DIAG && a == b) r2 = p > q ? r2 : 1e30f;  // each unordered pair once: no term at 1e15 A
@@ -562,13 +655,17 @@ __device__ __forceinline__ void born_tile(const float4* L, int ni, int nj, int l
       if (CUT || CLS == kMixed) u = on ? u : 0.0f;
       const float u2 = u * u;
       acci = fmaf(u2, j.sum(u, false), acci);
-      accj[a] = fmaf(u2, i.sum(u, true), accj[a]);
+      accj[k] = fmaf(u2, i.sum(u, true), accj[k]);
     }
-    const float r = sum_p(acci);
-    rows = p == b ? r : rows;
+    if constexpr (COLS == kHalf) {
+      t[(b >> 1) * 64 + lane] = half[0];
+    } else {
+      const float r = sum_p(half[0] + half[1]);
+      rows[0] = p == b ? r : rows[0];
+    }
     if (CLS == kMixed && !DIAG) near |= (unsigned long long)marks << (kEdge * b);
   }
-  cols = sum_q(accj, lane);
+  cols[0] = sum_q(accj, lane);
 }
 
 // Class bits of an item from its tiles' bounding boxes (wave-uniform). The
@@ -701,38 +798,216 @@ struct StageRun {
   }
 };
 
+template <int COLS>
 struct BornRun {
   const float4* L;
   int ni, nj, lane;
   float cut2, thr2;
-  int sub, nsub;
-  float rows, cols;
+  int sub, nsub, h;
+  float* t;
+  float rows[1], cols[1];
   unsigned long long near;
   template <int CLS, bool DIAG, bool CUT, bool FULL>
   __device__ __forceinline__ void run() {
-    born_tile<CLS, DIAG, CUT, FULL>(L, ni, nj, lane, cut2, thr2, sub, nsub, rows, cols, near);
+    born_tile<CLS, DIAG, CUT, FULL, COLS>(L, ni, nj, lane, cut2, thr2, sub, nsub, h, t, rows, cols, near);
   }
 };
 
-// Column sums of a share of a Born item (lane = column), added share by share.
-struct BornSum {
-  float c = 0.0f;
-  __device__ __forceinline__ void add(const BornSum& o) { c += o.c; }
-  __device__ __forceinline__ void store(const DeviceView& v, int w, int lane) const { part1(v, w, 1)[lane] = c; }
-  __device__ __forceinline__ void to_lds(float4* at, int lane) const { reinterpret_cast<float*>(at)[lane] = c; }
-  __device__ __forceinline__ void from_lds(const float4* at, int lane) { c = reinterpret_cast<const float*>(at)[lane]; }
+// C sums per row and per column of one item: Born (C = 1) and chain (C = 3).
+template <int C>
+__device__ __forceinline__ void put_sums(float* at, int stride, int lane, const float (&v)[C]) {
+#pragma unroll
+  for (int c = 0; c < C; ++c) at[c * stride + lane] = v[c];
+}
+template <int C>
+__device__ __forceinline__ void add_sums(float (&v)[C], const float (&o)[C]) {
+#pragma unroll
+  for (int c = 0; c < C; ++c) v[c] += o[c];
+}
+template <int C>
+struct ObcSum {
+  float v[C] = {};
+  __device__ __forceinline__ void add(const ObcSum& o) { add_sums(v, o.v); }
+  __device__ __forceinline__ void to_lds(float4* at, int lane) const {
+    put_sums(reinterpret_cast<float*>(at), kTile, lane, v);
+  }
+  __device__ __forceinline__ void from_lds(const float4* at, int lane) {
+#pragma unroll
+    for (int c = 0; c < C; ++c) v[c] = reinterpret_cast<const float*>(at)[c * kTile + lane];
+  }
 };
 
-// The Born pass over one item. stage() prepares it (rows and/or cols: which of
-// its tiles this wave brings into LDS at L); false: the item has no work, and no
-// partials. run() evaluates share sub of its rows: stores their sums and
-// returns the columns'. scratch: 64 float4 of this wave's own.
-struct BornPass {
-  typedef BornSum Sum;
-  static constexpr int kLds = kBornLds;
+// The Born and the chain pass over one item; Self has stage(), which prepares it
+// (rows and/or cols: which of its tiles this wave brings into LDS; false: the item has
+// no work, and no partials), the pass's run, near-pair functions and partials.
+template <class Self, int C>
+struct ObcPass {
+  typedef ObcSum<C> Sum;
+  typedef QuarterLds<C> Quarter;
+  static constexpr int kLaneEnergies = 0;
   int w, lane, ni, nj, tier, nsub;
   float cut2, thr2, lim2;
   bool diag, full, cut;
+
+  // Near pairs of a diagonal item: sums of its atoms.
+  template <bool SPLIT>
+  __device__ __forceinline__ void near_atoms(const float4* L, int s, int h, float (&sum)[C]) const {
+    const Tile4* t = reinterpret_cast<const Tile4*>(L);
+    near_diag<SPLIT>(
+        t, lane, ni, s, nsub, h, cut, lim2,
+        [&](int atom, const int (&o)[2], const bool (&on)[2], float (&even)[C], float (&odd)[C]) {
+          Self::near_two(t, atom, o, on, even, odd);
+        },
+        sum);
+  }
+
+  // Near pairs off the diagonal of one share: added to its rows' and its columns' sums.
+  template <bool HALVES>
+  __device__ __forceinline__ void near_pairs(const float4* L, float4* scratch, unsigned long long near, int my_col,
+                                             float (&rows)[C], float (&cols)[C]) const {
+    const Tile4* ti = reinterpret_cast<const Tile4*>(L);
+    const Tile4* tj = ti + 2;
+    float n0[C] = {}, n1[C] = {}, m[C] = {};
+    near_list<HALVES>(
+        ti, tj, near, lane, my_col, cut, lim2, scratch,
+        [&](int row, int col) { return Self::near_pair(ti, tj, row, col); },
+        [&](auto half, const float4& c, float mine) { Self::add_row(decltype(half)::value ? n1 : n0, c, mine); },
+        [&](const float4& c, float mine) { Self::add_col(m, c, mine); });
+    add_sums(rows, n0);
+    add_sums(rows, n1);
+    add_sums(cols, m);
+  }
+
+  // Share s: its rows' sums (zero in the other's lanes) and its columns' (lane = atom),
+  // far and then near. scratch: this wave's own.
+  __device__ __forceinline__ void share(int s, const float4* L, float4* scratch, float (&rows)[C],
+                                        float (&cols)[C]) const {
+    typename Self::template Run<kEdge> f{L, ni, nj, lane, cut2, thr2, s, nsub, 0, nullptr, {}, {}, 0};
+    by_class(tier, diag, cut, full, f);
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      rows[c] = f.rows[c];
+      cols[c] = f.cols[c];
+    }
+    if (diag) {
+      float d[C] = {};
+      near_atoms<false>(L, s, 0, d);
+      add_sums(cols, d);
+    } else if (f.near != 0) {
+      near_pairs<true>(L, scratch, f.near, lane, rows, cols);
+    }
+  }
+
+  // Share s0, or with LOOP the shares s0 .. s1 - 1: stores the rows' sums and
+  // returns the columns', share 0's plus share 1's.
+  template <bool LOOP>
+  __device__ __forceinline__ Sum run(const DeviceView& v, int s0, int s1, const float4* L, float4* scratch) const {
+    const int p = lane & 7, q = lane >> 3, mine = p & (nsub - 1);
+    Sum sum;
+    if constexpr (LOOP) {
+      float rows[C] = {};
+#pragma unroll 1
+      for (int s = s0; s < s1; ++s) {
+        float r[C], c[C];
+        share(s, L, scratch, r, c);
+        add_sums(rows, r);
+        add_sums(sum.v, c);
+      }
+      if (mine >= s0 && mine < s1) Self::put(v, w, 0, kEdge * p + q, rows);
+    } else {
+      float rows[C];
+      share(s0, L, scratch, rows, sum.v);
+      if (mine == s0) Self::put(v, w, 0, kEdge * p + q, rows);
+    }
+    return sum;
+  }
+
+  // The item by four waves: wave k = 2 s + h takes share s of the rows and half h
+  // of the columns. M: the group's memory (QuarterLds).
+  __device__ __forceinline__ Sum quarter(int k, float4* M) const {
+    typedef Quarter Q;
+    const int s = k >> 1, h = k & 1;
+    float4* const scratch = Q::scratch(M, k);
+    typename Self::template Run<kHalf> f{M, ni, nj, lane, cut2, thr2, s, nsub, h, Q::rows(M, k), {}, {}, 0};
+    by_class(tier, diag, cut, full, f);
+    Sum sum;
+    add_sums(sum.v, f.cols);
+    if (diag) {
+      float d[C] = {};
+      near_atoms<true>(M, s, h, d);
+      put_sums(reinterpret_cast<float*>(scratch), kTile, lane, d);
+      wave_lds_sync();
+#pragma unroll
+      for (int c = 0; c < C; ++c) sum.v[c] += reinterpret_cast<const float*>(scratch)[c * kTile + half_col(lane)];
+    } else {
+      float near[C] = {};  // of the rows
+      if (f.near != 0)
+        near_pairs<false>(M, scratch, f.near, half_atom(h, half_col(lane)), near, sum.v);
+      put_sums(reinterpret_cast<float*>(scratch), kTile, lane, near);
+    }
+    if (s == 1 && (lane & 8) == 0)
+      put_sums(reinterpret_cast<float*>(scratch) + C * kTile, kTile / 2, half_col(lane), sum.v);
+    return sum;
+  }
+
+  // Behind the barrier: wave k finishes two of its share's rows of patches, the
+  // waves of share 0 the columns of their half.
+  __device__ __forceinline__ void finish(const DeviceView& v, int k, float4* M, Sum& sum) const {
+    typedef Quarter Q;
+    const int s = k >> 1, h = k & 1, p = lane & 7, q = lane >> 3;
+    float rows[C] = {};
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const int i = 2 * h + n, b = s + 2 * i;
+      if (kEdge * b >= ni) break;
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const int at = (c * kHalf + i) * 64 + lane;
+        const float r = sum_p(Q::rows(M, 2 * s)[at] + Q::rows(M, 2 * s + 1)[at]);
+        rows[c] = p == b ? r : rows[c];
+      }
+    }
+    const float* const n0 = reinterpret_cast<const float*>(Q::scratch(M, 2 * s));
+    const float* const n1 = reinterpret_cast<const float*>(Q::scratch(M, 2 * s + 1));
+    if (!diag)
+#pragma unroll
+      for (int c = 0; c < C; ++c) rows[c] = (rows[c] + n0[c * kTile + lane]) + n1[c * kTile + lane];
+    if ((p & 1) == s && (p >> 2) == h) Self::put(v, w, 0, kEdge * p + q, rows);
+    if (s != 0) return;
+    const int half = half_col(lane);
+    const float* const c1 = reinterpret_cast<const float*>(Q::scratch(M, 2 + h)) + C * kTile;
+    float cols[C];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+      cols[c] = sum.v[c] + c1[c * (kTile / 2) + half];
+    }
+    if ((lane & 8) == 0) Self::put(v, w, 1, half_atom(h, half), cols);
+  }
+
+  __device__ __forceinline__ void store(const DeviceView& v, const Sum& s) const { Self::put(v, w, 1, lane, s.v); }
+};
+
+struct BornPass : ObcPass<BornPass, 1> {
+  template <int COLS>
+  using Run = BornRun<COLS>;
+  static constexpr int kRows = 1, kScratch = kObcScratch<1>;
+
+  __device__ __forceinline__ static float3 near_pair(const Tile4* ti, const Tile4* tj, int row, int col) {
+    return born_near_pair(ti, tj, row, col);
+  }
+  __device__ __forceinline__ static void add_row(float (&n)[1], const float4& c, float mine) {
+    n[0] = fmaf(mine, c.x, n[0]);
+  }
+  __device__ __forceinline__ static void add_col(float (&m)[1], const float4& c, float mine) {
+    m[0] = fmaf(mine, c.y, m[0]);
+  }
+  __device__ __forceinline__ static void near_two(const Tile4* t, int atom, const int (&o)[2], const bool (&on)[2],
+                                                  float (&even)[1], float (&odd)[1]) {
+    born_near_diag(t, atom, o, on, even, odd);
+  }
+  __device__ __forceinline__ static void put(const DeviceView& v, int w, int side, int at, const float (&x)[1]) {
+    part1(v, w, side)[at] = x[0];
+  }
 
   __device__ __forceinline__ bool stage(const DeviceView& v, int w_, const PairItem& it, bool rows, bool cols,
                                         float4* L) {
@@ -771,18 +1046,6 @@ struct BornPass {
     by_class(tier, diag, cut, full, put);
     return true;
   }
-
-  __device__ __forceinline__ BornSum run(const DeviceView& v, int sub, float4* L,
-                                         float4* scratch) const {
-    const int p = lane & 7, q = lane >> 3;
-    BornRun f{L, ni, nj, lane, cut2, thr2, sub, nsub, 0.0f, 0.0f, 0};
-    by_class(tier, diag, cut, full, f);
-    if (f.near != 0 || diag) born_near(L, scratch, f.near, lane, ni, diag, cut, lim2, sub, nsub, f.rows, f.cols);
-    if ((p & (nsub - 1)) == sub) part1(v, w, 0)[kEdge * p + q] = f.rows;
-    BornSum s;
-    s.c = f.cols;
-    return s;
-  }
 };
 
 // ---------------------------------------------------------------------------
@@ -800,19 +1063,23 @@ struct ForceSum {
     x += o.x; y += o.y; z += o.z; g += o.g;
     if (ENERGY) e += o.e;
   }
-  __device__ __forceinline__ void store(const DeviceView& v, int w, int lane) const {
-    part4(v, w, 1)[lane] = make_float4(x, y, z, g);
+  __device__ __forceinline__ void put_energies(const DeviceView& v, int w, int lane) const {
     if (ENERGY && lane < 48 && (lane & 15) == 0) v.e_items[(size_t)w * 3 + (lane == 0 ? 0 : (lane == 32 ? 1 : 2))] = e;
   }
-  __device__ __forceinline__ void to_lds(float4* at, int lane) const {
-    at[lane] = make_float4(x, y, z, g);
+  __device__ __forceinline__ void to_lds(float4* at, int lane, int atom) const {
+    at[atom] = make_float4(x, y, z, g);
     if (ENERGY && (lane & 15) == 0) reinterpret_cast<double*>(at + kTile)[lane >> 4] = e;
   }
-  __device__ __forceinline__ void from_lds(const float4* at, int lane) {
-    const float4 f = at[lane];
-    x = f.x; y = f.y; z = f.z; g = f.w;
-    if (ENERGY) e = reinterpret_cast<const double*>(at + kTile)[lane >> 4];
+  __device__ __forceinline__ void to_lds(float4* at, int lane) const { to_lds(at, lane, lane); }
+  __device__ __forceinline__ double energy_from_lds(const float4* at, int lane) const {
+    return ENERGY ? reinterpret_cast<const double*>(at + kTile)[lane >> 4] : 0.0;
   }
+  __device__ __forceinline__ void from_lds(const float4* at, int lane, int atom) {
+    const float4 f = at[atom];
+    x = f.x; y = f.y; z = f.z; g = f.w;
+    e = energy_from_lds(at, lane);
+  }
+  __device__ __forceinline__ void from_lds(const float4* at, int lane) { from_lds(at, lane, lane); }
 };
 
 // Three doubles summed over the wave, in the lanes of ForceSum::e: each
@@ -825,48 +1092,95 @@ __device__ __forceinline__ double sum_energies(double gb, double cl, double lj) 
   return e + dpp<kDppRor8 - 7>(e);
 }
 
+// Row sums of a patch row, from its lanes p.
+__device__ __forceinline__ void put_force_row(float* side0, int row, int p, float x, float y, float z, float db) {
+  const float s = sum_p4(x, y, z, -0.5f * db, p);
+  if ((p & 1) == 0) side0[row * 4 + comp_p(p)] = s;
+}
+
+// Three energies of this lane's pairs added to its sums in LDS.
+__device__ __forceinline__ void add_energies(double* en, int lane, const double (&e)[3]) {
+#pragma unroll
+  for (int c = 0; c < 3; ++c) en[c * 64 + lane] += e[c];
+}
+
 // What the pass takes from its system's constants and its item.
 struct ForceConst {
   float kc, gb2, cut2;  // cut2 > 0: the test r^2 < cut2 per pair
   bool gb_cut;          // of GB too
   float ev[4], ee[4];   // scales by exclusion class
-  const unsigned long long* excl;  // the tile's exclusion masks, or nullptr
+  const ulonglong2* excl;  // the rows' exclusion masks, or nullptr
 };
 
 // LJC = false: GB only (items entirely beyond the LJ/Coulomb cutoff). GEN:
 // ragged tiles, exclusions, and with cut2 > 0 the test r^2 < cut2 per pair, on
-// LJ/Coulomb and, if gb_cut, on GB too.
-template <bool GEN, bool DIAG, bool ENERGY, bool LJC>
+// LJ/Coulomb and, if gb_cut, on GB too. COLS, h and t as in born_tile. The energies too
+// are summed by halves, a row of patches at a time: with all eight columns the sums of
+// both halves wait in LDS (en: [half][term][lane]), where in registers they cost a
+// wave per SIMD, and a row takes the columns of half 0 first.
+template <bool GEN, bool DIAG, bool ENERGY, bool LJC, int COLS>
 __device__ __forceinline__ void force_tile(const ForceConst& S, int ni, int nj, int lane, float* side0, int sub,
-                                           int nsub, const float4* L, ForceSum<ENERGY>& out) {
+                                           int nsub, int h, float* t, const float4* L, double* en, ForceSum<ENERGY>& out) {
   const Tile4* ti = reinterpret_cast<const Tile4*>(L);
   const Tile4* tj = ti + 2;
   const float kc = S.kc, gb2 = S.gb2, cut2 = S.cut2;
   const bool has_cut = GEN && cut2 > 0.0f, gb_cut = S.gb_cut;
   const bool has_excl = GEN && LJC && S.excl != nullptr;
   const int p = lane & 7, q = lane >> 3;
-  float fxj[kEdge] = {}, fyj[kEdge] = {}, fzj[kEdge] = {}, dbj[kEdge] = {};
-  double egb = 0.0, ecl = 0.0, elj = 0.0;
+  float fxj[COLS] = {}, fyj[COLS] = {}, fzj[COLS] = {}, dbj[COLS] = {};
+  constexpr int kTerms = 3;
+  double e[kTerms] = {};  // GB, Coulomb, LJ / 4
+  if (ENERGY && COLS == kEdge)
+#pragma unroll
+    for (int k = 0; k < 2 * kTerms; ++k) en[k * 64 + lane] = 0.0;
   const int nb = GEN ? (ni + kEdge - 1) / kEdge : kEdge, na = GEN ? (nj + kEdge - 1) / kEdge : kEdge;
-  const int comp = comp_p(p);
+  ulonglong2 next = {};  // a short loop waits for these loads: half an item's are issued a row ahead
+  float4 half_a[kHalf], half_b[kHalf];  // columns of half h, kept over the rows
+  if (COLS == kHalf)
+#pragma unroll
+    for (int k = 0; k < kHalf; ++k) {
+      half_a[k] = tj[0][p + kEdge * (2 * k + h)];
+      half_b[k] = tj[1][p + kEdge * (2 * k + h)];
+    }
   PRX_UNROLL(PRX_UNROLL_FORCE)
   for (int b = sub; b < nb; b += nsub) {
     const int row = kEdge * b + q;
     const float4 ia = ti[0][row], ib = ti[1][row];
     const float q_kc = kc * ia.w, q_gb = gb2 * ia.w;
-    float fxi = 0.f, fyi = 0.f, fzi = 0.f, dbi = 0.f;
+    float fx[COLS / kHalf] = {}, fy[COLS / kHalf] = {}, fz[COLS / kHalf] = {}, db[COLS / kHalf] = {};
     unsigned long long m0 = 0, m1 = 0;  // the row's exclusion classes, column p of each patch at bit 8 a
     if (has_excl) {
-      m0 = S.excl[row * 2] >> p;
-      m1 = S.excl[row * 2 + 1] >> p;
+      if (COLS == kEdge || b == sub) next = S.excl[row];
+      m0 = next.x >> p;
+      m1 = next.y >> p;
+      if (COLS == kHalf && b + nsub < nb) next = S.excl[row + kEdge * nsub];
     }
-    int col = p;
+    int col = kByte * p;
+    double er[kTerms] = {};  // of the row's columns of one half
 #pragma unroll
-    for (int a = 0; a < kEdge; ++a) {
-      if (GEN && a >= na) break;
+    for (int n = 0; n < COLS; ++n) {
+      // place n's column: with energies half 0's before half 1's
+      const auto place = [](int n) { return ENERGY && COLS == kEdge ? 2 * (n % kHalf) + n / kHalf : n; };
+      const int k = place(n);
+      if (ENERGY && COLS == kEdge && n == kHalf) {
+        add_energies(en, lane, er);
+#pragma unroll
+        for (int c = 0; c < kTerms; ++c) er[c] = 0.0;
+      }
+      const int a = COLS == kHalf ? 2 * k + h : k;
+      if (GEN && a >= na) continue;
       if (DIAG && a < b) continue;
-      col = after(col, a < 2 ? fxi : fxj[a - 2]);
-      const float4 ja = tj[0][col + kEdge * a], jb = tj[1][col + kEdge * a];
+      const int o = half_of<COLS>(k);
+      float &fxi = fx[o], &fyi = fy[o], &fzi = fz[o], &dbi = db[o];
+      float4 ja, jb;
+      if constexpr (COLS == kHalf) {
+        ja = half_a[k];
+        jb = half_b[k];
+      } else {
+        col = after(col, n < 2 ? fxi : fxj[place(n - 2)]);
+        ja = at_byte(tj, 0, col + kByte * kEdge * k);
+        jb = at_byte(tj, 1, col + kByte * kEdge * k);
+      }
       const float dx = ja.x - ia.x, dy = ja.y - ia.y, dz = ja.z - ia.z;
       float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
       const bool once = !DIAG || a != b || p > q;  // each unordered pair once
@@ -883,7 +1197,8 @@ __device__ __forceinline__ void force_tile(const ForceConst& S, int ni, int nj, 
         const float s2 = sg * sg * rinv2;
         const float s6 = s2 * s2 * s2;
         float el = ep * fmaf(s6, s6, -s6);  // / 4
-        float fl = ep * s6 * fmaf(48.0f, s6, -24.0f);
+        const float es6 = ep * s6, f6 = fmaf(48.0f, s6, -24.0f);
+        float fl = es6 * f6;
         if (GEN) {
           if (has_excl) {
             const unsigned e0 = (unsigned)(m0 >> (kEdge * a)) & 1u, e1 = (unsigned)(m1 >> (kEdge * a)) & 1u;
@@ -904,10 +1219,10 @@ __device__ __forceinline__ void force_tile(const ForceConst& S, int ni, int nj, 
           }
         }
         if (ENERGY) {
-          ecl += once ? (double)ec : 0.0;
-          elj += once ? (double)el : 0.0;
+          er[1] += once ? (double)ec : 0.0;
+          er[2] += once ? (double)el : 0.0;
         }
-        lc = ec + fl;
+        lc = GEN ? ec + fl : fmaf(es6, f6, ec);
       }
       // GB over every pair
       const float BB = ib.z * jb.z;
@@ -916,39 +1231,53 @@ __device__ __forceinline__ void force_tile(const ForceConst& S, int ni, int nj, 
       const float f2 = fmaf(BB, ex, r2);
       const float finv = frsq(f2);
       const float eg = (q_gb * ja.w) * finv;
-      const float t = eg * (finv * finv);  // gb2 qq / f^3
-      const float te = t * ex;
-      float fgb = fmaf(-0.25f, te, t);     // -dE/dr / r
+      const float tg = eg * (finv * finv);  // gb2 qq / f^3
+      const float te = tg * ex;
+      float fgb = fmaf(-0.25f, te, tg);    // -dE/dr / r
       float g = te * fmaf(x, kLn2, 1.0f);  // dE/dB_i = -g B_j / 2, dE/dB_j = -g B_i / 2
       if (GEN && has_cut && gb_cut) {
         fgb = in ? fgb : 0.0f;
         g = in ? g : 0.0f;
-        if (ENERGY) egb += in && once ? (double)eg : 0.0;
+        if (ENERGY) er[0] += in && once ? (double)eg : 0.0;
       } else if (ENERGY) {
-        egb += once ? (double)eg : 0.0;
+        er[0] += once ? (double)eg : 0.0;
       }
       const float fr = LJC ? fmaf(lc, rinv2, fgb) : fgb;
       // F_i = -fr * (x_j - x_i)
       fxi = fmaf(-fr, dx, fxi); fyi = fmaf(-fr, dy, fyi); fzi = fmaf(-fr, dz, fzi);
       dbi = fmaf(g, jb.z, dbi);
-      fxj[a] = fmaf(fr, dx, fxj[a]); fyj[a] = fmaf(fr, dy, fyj[a]); fzj[a] = fmaf(fr, dz, fzj[a]);
-      dbj[a] = fmaf(g, ib.z, dbj[a]);
+      fxj[k] = fmaf(fr, dx, fxj[k]); fyj[k] = fmaf(fr, dy, fyj[k]); fzj[k] = fmaf(fr, dz, fzj[k]);
+      dbj[k] = fmaf(g, ib.z, dbj[k]);
     }
-    const float t = sum_p4(fxi, fyi, fzi, -0.5f * dbi, p);
-    if ((p & 1) == 0) side0[row * 4 + comp] = t;
+    if (ENERGY && COLS == kEdge) add_energies(en + kTerms * 64, lane, er);
+    if (ENERGY && COLS == kHalf)
+#pragma unroll
+      for (int c = 0; c < kTerms; ++c) e[c] += er[c];
+    if constexpr (COLS == kHalf) {
+      reinterpret_cast<float4*>(t)[(b >> 1) * 64 + lane] = make_float4(fx[0], fy[0], fz[0], db[0]);
+    } else {
+      put_force_row(side0, row, p, fx[0] + fx[1], fy[0] + fy[1], fz[0] + fz[1], db[0] + db[1]);
+    }
   }
   out.x = sum_q(fxj, lane);
   out.y = sum_q(fyj, lane);
   out.z = sum_q(fzj, lane);
   out.g = -0.5f * sum_q(dbj, lane);
-  if (ENERGY) out.e = sum_energies(egb, ecl, 4.0 * elj);
+  if (ENERGY && COLS == kHalf) out.e = sum_energies(e[0], e[1], 4.0 * e[2]);
+  if (ENERGY && COLS == kEdge) {
+    const double* e1 = en + kTerms * 64;
+    out.e = sum_energies(en[lane], en[64 + lane], 4.0 * en[128 + lane]);
+    out.e += sum_energies(e1[lane], e1[64 + lane], 4.0 * e1[128 + lane]);
+  }
 }
 
 // The force pass over one item (as BornPass).
 template <bool ENERGY>
 struct ForcePass {
   typedef ForceSum<ENERGY> Sum;
-  static constexpr int kLds = kForceLds;
+  static constexpr int kRows = 4, kScratch = kTile;               // columns
+  static constexpr int kLaneEnergies = ENERGY ? 2 * 3 * 64 / 2 : 0;  // the lanes' energies by half, later the wave's
+  typedef QuarterLds<kRows, kScratch + 2> Quarter;                   // with the wave's energies
   int w, lane, ni, nj, cls, nsub, flags;
   ForceConst K;
   float* side0;
@@ -976,7 +1305,7 @@ struct ForcePass {
     K.gb2 = S.gb2;
     K.cut2 = cls == kClsStraddle ? S.cutoff2 : 0.0f;
     K.gb_cut = S.gb_cut != 0;
-    K.excl = it.excl >= 0 ? v.excl_masks + (size_t)it.excl * 128 : nullptr;
+    K.excl = it.excl >= 0 ? reinterpret_cast<const ulonglong2*>(v.excl_masks) + (size_t)it.excl * kTile : nullptr;
     for (int k = 1; k < 4; ++k) {
       K.ev[k] = S.excl_v[k];
       K.ee[k] = S.excl_e[k];
@@ -1003,21 +1332,67 @@ struct ForcePass {
     return true;
   }
 
-  __device__ __forceinline__ Sum run(const DeviceView&, int sub, float4* L, float4*) const {
+  template <int COLS>
+  __device__ __forceinline__ Sum share(int sub, int h, float* t, const float4* L, double* en) const {
     Sum f;
     if (cls == kClsFar) {  // GB over every pair, nothing else (a far item is never diagonal)
       if (full)
-        force_tile<false, false, ENERGY, false>(K, ni, nj, lane, side0, sub, nsub, L, f);
+        force_tile<false, false, ENERGY, false, COLS>(K, ni, nj, lane, side0, sub, nsub, h, t, L, en, f);
       else
-        force_tile<true, false, ENERGY, false>(K, ni, nj, lane, side0, sub, nsub, L, f);
+        force_tile<true, false, ENERGY, false, COLS>(K, ni, nj, lane, side0, sub, nsub, h, t, L, en, f);
     } else if (flags & kFlagDiag) {
-      force_tile<true, true, ENERGY, true>(K, ni, nj, lane, side0, sub, nsub, L, f);
+      force_tile<true, true, ENERGY, true, COLS>(K, ni, nj, lane, side0, sub, nsub, h, t, L, en, f);
     } else if (full && !(flags & kFlagExcl) && K.cut2 == 0.0f) {
-      force_tile<false, false, ENERGY, true>(K, ni, nj, lane, side0, sub, nsub, L, f);
+      force_tile<false, false, ENERGY, true, COLS>(K, ni, nj, lane, side0, sub, nsub, h, t, L, en, f);
     } else {
-      force_tile<true, false, ENERGY, true>(K, ni, nj, lane, side0, sub, nsub, L, f);
+      force_tile<true, false, ENERGY, true, COLS>(K, ni, nj, lane, side0, sub, nsub, h, t, L, en, f);
     }
     return f;
+  }
+
+  // As in ObcPass.
+  template <bool LOOP>
+  __device__ __forceinline__ Sum run(const DeviceView&, int s0, int s1, const float4* L, float4* scratch) const {
+    double* const en = reinterpret_cast<double*>(scratch + kScratch);
+    if constexpr (!LOOP) return share<kEdge>(s0, 0, nullptr, L, en);
+    Sum sum;
+#pragma unroll 1
+    for (int sub = s0; sub < s1; ++sub) sum.add(share<kEdge>(sub, 0, nullptr, L, en));
+    return sum;
+  }
+
+  __device__ __forceinline__ Sum quarter(int k, float4* M) const {
+    const Sum sum = share<kHalf>(k >> 1, k & 1, Quarter::rows(M, k), M, nullptr);
+    if (k != 0) sum.to_lds(Quarter::scratch(M, k), lane, half_col(lane));
+    return sum;
+  }
+
+  __device__ __forceinline__ void finish(const DeviceView& v, int k, float4* M, Sum& sum) const {
+    const int s = k >> 1, h = k & 1, p = lane & 7, q = lane >> 3;
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      const int i = 2 * h + n, b = s + 2 * i;
+      if (kEdge * b >= ni) break;
+      const float4 x = reinterpret_cast<const float4*>(Quarter::rows(M, 2 * s))[i * 64 + lane];
+      const float4 y = reinterpret_cast<const float4*>(Quarter::rows(M, 2 * s + 1))[i * 64 + lane];
+      put_force_row(side0, kEdge * b + q, p, x.x + y.x, x.y + y.y, x.z + y.z, x.w + y.w);
+    }
+    if (s != 0) return;
+    const int half = half_col(lane);
+    Sum o;
+    o.from_lds(Quarter::scratch(M, 2 + h), lane, half);
+    if (ENERGY && h == 0) {
+      sum.e += sum.energy_from_lds(Quarter::scratch(M, 1), lane);
+      o.e += o.energy_from_lds(Quarter::scratch(M, 3), lane);
+    }
+    sum.add(o);
+    if ((lane & 8) == 0) part4(v, w, 1)[half_atom(h, half)] = make_float4(sum.x, sum.y, sum.z, sum.g);
+    if (h == 0) sum.put_energies(v, w, lane);
+  }
+
+  __device__ __forceinline__ void store(const DeviceView& v, const Sum& s) const {
+    part4(v, w, 1)[lane] = make_float4(s.x, s.y, s.z, s.g);
+    s.put_energies(v, w, lane);
   }
 };
 
@@ -1043,24 +1418,24 @@ struct ChainAtom {
       t[1][lane] = make_float4(b.z, b.w, b.x, b.y);
     }
   }
-  __device__ __forceinline__ void read(const Tile4* t, int e, bool row) {
-    const float4 a = t[0][e];
+  __device__ __forceinline__ void read(const Tile4* t, int byte, bool row) {
+    const float4 a = at_byte(t, 0, byte);
     x = a.x; y = a.y; z = a.z; c = a.w;
     if constexpr (kShort) {
-      const float4 b = t[1][e];
+      const float4 b = at_byte(t, 1, byte);
       w[0] = b.x; w[1] = b.y; w[2] = b.z;
       if constexpr (ChainW<CLS>::N > 3) w[3] = b.w;
     } else {
-      const float2 b = *reinterpret_cast<const float2*>(&t[1][e]);
+      const float2 b = *reinterpret_cast<const float2*>(&at_byte(t, 1, byte));
       s2 = b.x;
       s33 = b.y;
       if (row) obc_weights<ChainW<CLS>>(s2, s33, w);
     }
   }
-  // f sum_k w_k u^k
-  __device__ __forceinline__ float sum(float f, float u, bool row) const {
-    if (kShort || row) return f * horner(w, u);
-    return (f * s33) * obc_poly<ChainW<CLS>>(s2 * u);
+  // sum_k w_k u^k
+  __device__ __forceinline__ float sum(float u, bool row) const {
+    if (kShort || row) return horner(w, u);
+    return s33 * obc_poly<ChainW<CLS>>(s2 * u);
   }
 };
 
@@ -1074,71 +1449,65 @@ __device__ __forceinline__ float chain_one(float r2, float ci, const float4& bi,
   return fmaf(ci, d1, cj * d2) * rinv;
 }
 
-__device__ __forceinline__ void chain_near(float4* L, float4* scratch, unsigned long long near, int lane, int ni, bool diag, bool cut,
-                                           float lim2, int sub, int nsub, float3& rows, float3& cols) {
-  Tile4* ti = reinterpret_cast<Tile4*>(L);
-  Tile4* tj = ti + 2;
-  if (diag) {
-    const float4 me = ti[0][lane], mb = ti[1][lane];
-    near_diag(ti, lane, ni, sub, nsub, cut, lim2, [&](const int (&o)[2], const bool (&on)[2]) {
-      float g[2], dx[2], dy[2], dz[2];
+__device__ __forceinline__ void chain_near_diag(const Tile4* t, int atom, const int (&o)[2], const bool (&on)[2],
+                                                float (&even)[3], float (&odd)[3]) {
+  const float4 me = t[0][atom], mb = t[1][atom];
+  float g[2], dx[2], dy[2], dz[2];
 #pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const float4 a = ti[0][o[k]], b = ti[1][o[k]];
-        dx[k] = a.x - me.x; dy[k] = a.y - me.y; dz[k] = a.z - me.z;
-        const float r2 = fmaf(dx[k], dx[k], fmaf(dy[k], dy[k], dz[k] * dz[k]));
-        g[k] = chain_one(on[k] ? r2 : 1.0f, me.w, mb, a.w, b);
-      }
-#pragma unroll
-      for (int k = 0; k < 2; ++k) {
-        const float f = on[k] ? g[k] : 0.0f;
-        cols.x = fmaf(f, dx[k], cols.x);
-        cols.y = fmaf(f, dy[k], cols.y);
-        cols.z = fmaf(f, dz[k], cols.z);
-      }
-    });
-    return;
+  for (int k = 0; k < 2; ++k) {
+    const float4 a = t[0][o[k]], b = t[1][o[k]];
+    dx[k] = a.x - me.x; dy[k] = a.y - me.y; dz[k] = a.z - me.z;
+    const float r2 = fmaf(dx[k], dx[k], fmaf(dy[k], dy[k], dz[k] * dz[k]));
+    g[k] = chain_one(on[k] ? r2 : 1.0f, me.w, mb, a.w, b);
   }
-  near_list(
-      ti, tj, near, lane, cut, lim2, scratch,
-      [&](int row, int col) {
-        const float4 ai = ti[0][row], bi = ti[1][row], aj = tj[0][col], bj = tj[1][col];
-        const float dx = aj.x - ai.x, dy = aj.y - ai.y, dz = aj.z - ai.z;
-        const float gsc = chain_one(fmaf(dx, dx, fmaf(dy, dy, dz * dz)), ai.w, bi, aj.w, bj);
-        return make_float3(gsc * dx, gsc * dy, gsc * dz);
-      },
-      [&](const float4& c, float mine) {
-        rows.x = fmaf(mine, c.x, rows.x); rows.y = fmaf(mine, c.y, rows.y); rows.z = fmaf(mine, c.z, rows.z);
-      },
-      [&](const float4& c, float mine) {
-        cols.x = fmaf(-mine, c.x, cols.x); cols.y = fmaf(-mine, c.y, cols.y); cols.z = fmaf(-mine, c.z, cols.z);
-      });
+  const float f = on[0] ? g[0] : 0.0f, e = on[1] ? g[1] : 0.0f;
+  even[0] = fmaf(f, dx[0], even[0]); even[1] = fmaf(f, dy[0], even[1]); even[2] = fmaf(f, dz[0], even[2]);
+  odd[0] = fmaf(e, dx[1], odd[0]); odd[1] = fmaf(e, dy[1], odd[1]); odd[2] = fmaf(e, dz[1], odd[2]);
+}
+
+// Force of a near pair off the diagonal on its row atom.
+__device__ __forceinline__ float3 chain_near_pair(const Tile4* ti, const Tile4* tj, int row, int col) {
+  const float4 ai = ti[0][row], bi = ti[1][row], aj = tj[0][col], bj = tj[1][col];
+  const float dx = aj.x - ai.x, dy = aj.y - ai.y, dz = aj.z - ai.z;
+  const float gsc = chain_one(fmaf(dx, dx, fmaf(dy, dy, dz * dz)), ai.w, bi, aj.w, bj);
+  return make_float3(gsc * dx, gsc * dy, gsc * dz);
 }
 
 // As born_tile. Per pair: F_i = gsc (x_j - x_i), gsc = (c_i dI(rho_i, s_j)/dr +
 // c_j dI(rho_j, s_i)/dr) / r, in the far field u^3 (c_i P_j(u) + c_j P_i(u)).
-template <int CLS, bool DIAG, bool CUT, bool FULL>
+template <int CLS, bool DIAG, bool CUT, bool FULL, int COLS>
 __device__ __forceinline__ void chain_tile(const float4* L, int ni, int nj, int lane, float cut2, float thr2, int sub,
-                                           int nsub, float3& rows, float3& cols, unsigned long long& near) {
+                                           int nsub, int h, float* t, float (&rows)[3], float (&cols)[3],
+                                           unsigned long long& near) {
   const Tile4* ti = reinterpret_cast<const Tile4*>(L);
   const Tile4* tj = ti + 2;
   const int p = lane & 7, q = lane >> 3;
-  float fxj[kEdge] = {}, fyj[kEdge] = {}, fzj[kEdge] = {};
+  float fxj[COLS] = {}, fyj[COLS] = {}, fzj[COLS] = {};
+  ChainAtom<CLS> half_cols[kHalf];
+  if (COLS == kHalf)
+#pragma unroll
+    for (int k = 0; k < kHalf; ++k) half_cols[k].read(tj, kByte * (p + kEdge * (2 * k + h)), false);
   const int nb = FULL ? kEdge : (ni + kEdge - 1) / kEdge, na = FULL ? kEdge : (nj + kEdge - 1) / kEdge;
   PRX_UNROLL(PRX_UNROLL_CHAIN)
   for (int b = sub; b < nb; b += nsub) {
     ChainAtom<CLS> i;
-    float fxi = 0.f, fyi = 0.f, fzi = 0.f;
-    i.read(ti, kEdge * b + q, true);
+    float fx[2] = {}, fy[2] = {}, fz[2] = {};
+    i.read(ti, kByte * (kEdge * b + q), true);
     unsigned marks = 0;
-    int col = p;
+    int col = kByte * p;
 #pragma unroll
-    for (int a = 0; a < kEdge; ++a) {
-      if (!FULL && a >= na) break;
+    for (int k = 0; k < COLS; ++k) {
+      const int a = COLS == kHalf ? 2 * k + h : k;
+      if (!FULL && a >= na) continue;
       if (DIAG && a < b) continue;
+      float &fxi = fx[half_of<COLS>(k)], &fyi = fy[half_of<COLS>(k)], &fzi = fz[half_of<COLS>(k)];
       ChainAtom<CLS> j;
-      col = after(col, a < 2 ? fxi : fxj[a - 2]);
-      j.read(tj, col + kEdge * a, false);
+      if constexpr (COLS == kHalf) {
+        j = half_cols[k];
+      } else {
+        col = after(col, k < 2 ? fxi : fxj[k - 2]);
+        j.read(tj, col + kByte * kEdge * k, false);
+      }
       const float dx = j.x - i.x, dy = j.y - i.y, dz = j.z - i.z;
       float r2 = fmaf(dx, dx, fmaf(dy, dy, dz * dz));
       if (DIAG && a == b) r2 = p > q ? r2 : 1e30f;
@@ -1151,55 +1520,64 @@ __device__ __forceinline__ void chain_tile(const float4* L, int ni, int nj, int 
       }
       float u = frcp(r2);
       if (CUT || CLS == kMixed) u = on ? u : 0.0f;
-      const float gsc = (u * u * u) * (j.sum(i.c, u, false) + i.sum(j.c, u, true));
+      const float gsc = (u * u * u) * fmaf(i.c, j.sum(u, false), j.c * i.sum(u, true));
       fxi = fmaf(gsc, dx, fxi); fyi = fmaf(gsc, dy, fyi); fzi = fmaf(gsc, dz, fzi);
-      fxj[a] = fmaf(-gsc, dx, fxj[a]); fyj[a] = fmaf(-gsc, dy, fyj[a]); fzj[a] = fmaf(-gsc, dz, fzj[a]);
+      fxj[k] = fmaf(-gsc, dx, fxj[k]); fyj[k] = fmaf(-gsc, dy, fyj[k]); fzj[k] = fmaf(-gsc, dz, fzj[k]);
     }
-    const float x = sum_p(fxi), y = sum_p(fyi), z = sum_p(fzi);
-    rows.x = p == b ? x : rows.x; rows.y = p == b ? y : rows.y; rows.z = p == b ? z : rows.z;
+    if constexpr (COLS == kHalf) {
+      const float x[3] = {fx[0], fy[0], fz[0]};
+#pragma unroll
+      for (int c = 0; c < 3; ++c) t[(c * kHalf + (b >> 1)) * 64 + lane] = x[c];
+    } else {
+      const float x = sum_p(fx[0] + fx[1]), y = sum_p(fy[0] + fy[1]), z = sum_p(fz[0] + fz[1]);
+      rows[0] = p == b ? x : rows[0]; rows[1] = p == b ? y : rows[1]; rows[2] = p == b ? z : rows[2];
+    }
     if (CLS == kMixed && !DIAG) near |= (unsigned long long)marks << (kEdge * b);
   }
-  cols = make_float3(sum_q(fxj, lane), sum_q(fyj, lane), sum_q(fzj, lane));
+  cols[0] = sum_q(fxj, lane);
+  cols[1] = sum_q(fyj, lane);
+  cols[2] = sum_q(fzj, lane);
 }
 
+template <int COLS>
 struct ChainRun {
   const float4* L;
   int ni, nj, lane;
   float cut2, thr2;
-  int sub, nsub;
-  float3 rows, cols;
+  int sub, nsub, h;
+  float* t;
+  float rows[3], cols[3];
   unsigned long long near;
   template <int CLS, bool DIAG, bool CUT, bool FULL>
   __device__ __forceinline__ void run() {
-    chain_tile<CLS, DIAG, CUT, FULL>(L, ni, nj, lane, cut2, thr2, sub, nsub, rows, cols, near);
+    chain_tile<CLS, DIAG, CUT, FULL, COLS>(L, ni, nj, lane, cut2, thr2, sub, nsub, h, t, rows, cols, near);
   }
 };
 
-__device__ __forceinline__ void put_part3(const DeviceView& v, int w, int side, int at, float x, float y, float z) {
-  float* pc = part3(v, w, side);
-  pc[at] = x;
-  pc[kTile + at] = y;
-  pc[2 * kTile + at] = z;
-}
+struct ChainPass : ObcPass<ChainPass, 3> {
+  template <int COLS>
+  using Run = ChainRun<COLS>;
+  static constexpr int kRows = 3, kScratch = kObcScratch<3>;
 
-struct ChainSum {
-  float x = 0.0f, y = 0.0f, z = 0.0f;
-  __device__ __forceinline__ void add(const ChainSum& o) { x += o.x; y += o.y; z += o.z; }
-  __device__ __forceinline__ void store(const DeviceView& v, int w, int lane) const { put_part3(v, w, 1, lane, x, y, z); }
-  __device__ __forceinline__ void to_lds(float4* at, int lane) const { at[lane] = make_float4(x, y, z, 0.0f); }
-  __device__ __forceinline__ void from_lds(const float4* at, int lane) {
-    const float4 f = at[lane];
-    x = f.x; y = f.y; z = f.z;
+  __device__ __forceinline__ static float3 near_pair(const Tile4* ti, const Tile4* tj, int row, int col) {
+    return chain_near_pair(ti, tj, row, col);
   }
-};
-
-// The chain pass over one item (as BornPass).
-struct ChainPass {
-  typedef ChainSum Sum;
-  static constexpr int kLds = kChainLds;
-  int w, lane, ni, nj, tier, nsub;
-  float cut2, thr2, lim2;
-  bool diag, full, cut;
+  __device__ __forceinline__ static void add_row(float (&n)[3], const float4& c, float mine) {
+    n[0] = fmaf(mine, c.x, n[0]); n[1] = fmaf(mine, c.y, n[1]); n[2] = fmaf(mine, c.z, n[2]);
+  }
+  __device__ __forceinline__ static void add_col(float (&m)[3], const float4& c, float mine) {
+    m[0] = fmaf(-mine, c.x, m[0]); m[1] = fmaf(-mine, c.y, m[1]); m[2] = fmaf(-mine, c.z, m[2]);
+  }
+  __device__ __forceinline__ static void near_two(const Tile4* t, int atom, const int (&o)[2], const bool (&on)[2],
+                                                  float (&even)[3], float (&odd)[3]) {
+    chain_near_diag(t, atom, o, on, even, odd);
+  }
+  __device__ __forceinline__ static void put(const DeviceView& v, int w, int side, int at, const float (&x)[3]) {
+    float* pc = part3(v, w, side);
+    pc[at] = x[0];
+    pc[kTile + at] = x[1];
+    pc[2 * kTile + at] = x[2];
+  }
 
   __device__ __forceinline__ bool stage(const DeviceView& v, int w_, const PairItem& it, bool rows, bool cols,
                                         float4* L) {
@@ -1229,69 +1607,55 @@ struct ChainPass {
     by_class(tier, diag, cut, full, put);
     return true;
   }
-
-  __device__ __forceinline__ ChainSum run(const DeviceView& v, int sub, float4* L,
-                                          float4* scratch) const {
-    const int p = lane & 7, q = lane >> 3;
-    const float3 zero = make_float3(0.f, 0.f, 0.f);
-    ChainRun f{L, ni, nj, lane, cut2, thr2, sub, nsub, zero, zero, 0};
-    by_class(tier, diag, cut, full, f);
-    if (f.near != 0 || diag) chain_near(L, scratch, f.near, lane, ni, diag, cut, lim2, sub, nsub, f.rows, f.cols);
-    if ((p & (nsub - 1)) == sub) put_part3(v, w, 0, kEdge * p + q, f.rows.x, f.rows.y, f.rows.z);
-    ChainSum s;
-    s.x = f.cols.x; s.y = f.cols.y; s.z = f.cols.z;
-    return s;
-  }
 };
 
 // ---------------------------------------------------------------------------
 // Items to waves
 // ---------------------------------------------------------------------------
-// The items of a small system are cut into shares by rows (PairItem.nsub: share
-// s has the rows b = s, s + nsub, ... of the patches), whose column sums are
-// added in their order. How many depends on the system's own size alone, so
-// its sums are the same in any pack and on either path:
-// - pair_wave: one wave takes an item, its shares one after the other. For work
-//   lists that fill the chip: a wave's registers and LDS are free as soon as its
-//   own item is done, and no wave waits for another.
-// - pair_unit: a group of kUnitWaves waves takes a unit (prx_common.h): a wave
-//   per share. The first two waves of an item bring its two tiles into LDS,
-//   for all. For short work lists, whose time is that of one item.
-// SYNC: every unit holds exactly two workgroup barriers, also one of whole
-// items or of items without work, so that groups of one workgroup meet the same
-// barriers whatever their units are; without it only cut items hold them.
-
+// The rows of an item are one share or two (PairItem.nsub, by the system's size: share s
+// has the rows of patches b = s, s + nsub, ...), whose column sums are added in their
+// order, and a row's sum is that of its half 0 plus that of its half 1. So one, two or
+// four waves give the same sums bit for bit, in any pack and on any path:
+// - a wave takes the item, its shares one after the other;
+// - two waves take a share each, and the second's column sums go through LDS;
+// - four waves take a half of the columns of a share each: they keep their four columns in
+//   registers, and the lanes of their rows meet in LDS.
+// Four row shares, whose column sums a wave alone formed four times over with four lists
+// of near pairs, cost the packs 4 to 12% that a lone system gained (us a step of 303 systems
+// of 700 atoms: 374, now 336; of one of 2,500: 54, now 53).
+// The first two waves of an item bring its two tiles into LDS, for all. Waves of
+// one, two or four items form a unit (prx_common.h).
 template <class Pass>
-__device__ __forceinline__ void pair_wave(const DeviceView& v, int w, float4* L) {
-  const PairItem it = v.items[w];
-  Pass f;
-  if (!f.stage(v, w, it, true, true, L)) return;
-  wave_lds_sync();
-  typename Pass::Sum s;
-  for (int sub = 0; sub < it.nsub; ++sub) s.add(f.run(v, sub, L, L + 4 * kTile));
-  s.store(v, w, f.lane);
+constexpr int kWaveLds = kTilesLds + Pass::kScratch + Pass::kLaneEnergies;  // a wave's memory where it takes an item or a share
+template <class Pass>
+constexpr int kGroupLds =
+    kUnitWaves * kWaveLds<Pass> > Pass::Quarter::kSize ? kUnitWaves * kWaveLds<Pass> : Pass::Quarter::kSize;
+constexpr int kAnyWaveLds = kWaveLds<ChainPass>;                // of any pass
+constexpr int kAnyGroupLds = kGroupLds<ForcePass<false>>;
+static_assert(kAnyWaveLds >= kWaveLds<BornPass> && kAnyWaveLds >= kWaveLds<ForcePass<false>>, "");
+static_assert(kAnyGroupLds >= kGroupLds<BornPass> && kAnyGroupLds >= kGroupLds<ChainPass> &&
+                  kAnyGroupLds >= kUnitWaves * kAnyWaveLds, "");
+
+// Unit i of the list (of items in four quarters each, no list is kept).
+__device__ __forceinline__ PairUnit unit_of(const DeviceView& v, int i) {
+  return v.units != nullptr ? v.units[i] : PairUnit{i, 1, kUnitWaves};
 }
 
-// Workgroup memory of one group: per wave two tiles (used by the first wave of
-// each item) and the wave's scratch, which takes its column sums at the end.
-template <int N, int WAVES = kUnitWaves>
-struct UnitLds {
-  static constexpr int kWaves = WAVES;
-  float4 wave[WAVES][N];
-};
-
-// k: the wave's index in the group. Groups of kUnitWaves take the units of the
-// list, smaller ones the item of the unit's index, in as many shares.
-template <bool SYNC, class Pass, class Lds>
-__device__ __forceinline__ void pair_unit(const DeviceView& v, int unit, int k, Lds& L) {
-  constexpr int W = Lds::kWaves;
-  const PairUnit u = W == kUnitWaves && v.units != nullptr ? v.units[unit] : PairUnit{unit, 1, W};
-  const int sh = u.shares;
+// Wave k of a group of W takes its part of unit u; M: the group's memory. meet: the
+// unit holds exactly two workgroup barriers, also one of whole items or of items
+// without work (groups of one workgroup, and waves of one group, meet the same
+// barriers whatever their units are); else none, and all its items are whole. LOOP:
+// a wave that takes a whole item may find two shares in it. QUAD: every unit of the
+// list is an item on four waves.
+template <class Pass, int W, bool LOOP, bool QUAD = false>
+__device__ __forceinline__ void pair_unit(const DeviceView& v, const PairUnit& u, int k, bool meet, float4* M) {
+  constexpr int kWave = kWaveLds<Pass>;
+  const int sh = QUAD ? kUnitWaves : u.shares;  // waves per item
+  const bool four = W == kUnitWaves && sh == kUnitWaves;
   const int m = sh == W ? 0 : (sh == 1 ? k : k / 2), sub = k - m * sh;
   const int w = u.first + m;
-  float4* const tiles = L.wave[m * sh];
-  float4* const own = L.wave[k] + 4 * kTile;
-  const bool meet = SYNC || sh > 1;
+  float4* const tiles = M + (four ? 0 : m * sh * kWave);
+  float4* const own = M + k * kWave + kTilesLds;
   PairItem it;
   Pass f;
   bool on = m < u.n;
@@ -1305,17 +1669,31 @@ __device__ __forceinline__ void pair_unit(const DeviceView& v, int unit, int k, 
     wave_lds_sync();
   typename Pass::Sum s;
   if (on) {
-    s.add(f.run(v, sub, tiles, own));
-    if (sub > 0) s.to_lds(own, f.lane);
+    if (four) {
+      s = f.quarter(k, M);
+    } else {
+      s = f.template run<LOOP>(v, sub, sh > 1 ? sub + 1 : it.nsub, tiles, own);
+      if (sub > 0) s.to_lds(own, f.lane);
+    }
   }
   if (meet) __syncthreads();
-  if (!on || sub > 0) return;
-  for (int n = 1; n < sh; ++n) {
-    typename Pass::Sum o;
-    o.from_lds(L.wave[k + n] + 4 * kTile, f.lane);
-    s.add(o);
+  if (!on) return;
+  if (four) {
+    f.finish(v, k, M, s);
+  } else if (sub == 0) {
+    if (sh > 1) {
+      typename Pass::Sum o;
+      o.from_lds(own + kWave, f.lane);
+      s.add(o);
+    }
+    f.store(v, s);
   }
-  s.store(v, w, f.lane);
+}
+
+// An item on one wave; L: the wave's memory.
+template <class Pass>
+__device__ __forceinline__ void pair_wave(const DeviceView& v, int w, float4* L) {
+  pair_unit<Pass, 1, false>(v, PairUnit{w, 1, 1}, 0, false, L);
 }
 
 // Item or unit of block b of nb. Workgroups are dispatched to the 8 XCDs round-robin
@@ -1347,3 +1725,5 @@ __device__ __forceinline__ int unit_wave() {
 }
 
 }  // namespace prx
+
+#pragma clang fp contract(fast)

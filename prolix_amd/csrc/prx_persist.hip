@@ -71,20 +71,19 @@ __device__ __forceinline__ bool grid_sync(GridBarrier* bar, unsigned& gen) {
 // the blocks, whose number the grid barriers' time grows with (2,500 atoms 201 us
 // a step, 480 with units).
 template <class Pass>
-__device__ __forceinline__ void pair_pass(const DeviceView& v, int wave, int n_waves, int uw, UnitLds<kPairLds>& L) {
-  if (persist_by_unit(v)) {
-    for (int u = blockIdx.x; u < v.n_units; u += gridDim.x) {
-      pair_unit<true, Pass>(v, u, uw, L);
-      __syncthreads();
-    }
-  } else {
-    for (int w = wave; w < v.n_items; w += n_waves) pair_wave<Pass>(v, w, L.wave[uw]);
+__device__ __forceinline__ void pair_pass(const DeviceView& v, int wave, int n_waves, int uw, float4* L) {
+  const bool units = persist_by_unit(v);
+  const int end = units ? v.n_units : v.n_items, step = units ? (int)gridDim.x : n_waves;
+  for (int k = units ? (int)blockIdx.x : wave; k < end; k += step) {
+    const PairUnit u = units ? unit_of(v, k) : PairUnit{k, 1, 1};
+    pair_unit<Pass, kUnitWaves, true>(v, u, units ? uw : 0, units, units ? L : L + uw * kAnyWaveLds);
+    if (units) __syncthreads();
   }
 }
 
 __global__ __launch_bounds__(kPersistThreads) void k_persist_steps(DeviceView v, const int32_t* ranges, int n_slots,
                                                                     int n_steps, int has_nl, GridBarrier* bar) {
-  __shared__ UnitLds<kPairLds> L;
+  __shared__ float4 L[kAnyGroupLds];
   const int uw = unit_wave();
   __shared__ GatherLds G;
   unsigned gen = 0;  // the barrier's generation, tracked by thread 0
