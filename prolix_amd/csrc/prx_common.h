@@ -55,8 +55,11 @@ constexpr int kHalfTiles = 128;
 // faster in the longest lists: 303 systems of 700 atoms (20,000 items) 361 and 338
 // with two, 31 of 5,000 (97,960) 1,113 and 1,064.
 constexpr int kQuarterItems = 5000;
-// The persistent kernel runs units up to this many, else an item per wave.
-constexpr int kPersistUnits = 64;
+// The persistent kernel has four waves per item up to kPersistQuads items, two up to
+// kPersistPairs, else one; the time of its barriers grows with the blocks. us a step on
+// four, two and one: 700 atoms (66 items) 79, 74, 95; 1,000 (136) 122, 87, 94; 1,250 (210)
+// 171, 108, 101.
+constexpr int kPersistQuads = 64, kPersistPairs = 150;
 
 constexpr int kFlagDiag = 1;
 constexpr int kFlagExcl = 2;
@@ -100,7 +103,6 @@ struct SlotConst {
   int32_t caps;         // 1: batched-step safety caps (velocity, displacement, force)
   int32_t tile0;        // global index of the system's first tile
   uint64_t seed;
-  int32_t unit0, n_units;  // the system's units
   int32_t pack0;        // packed index of the system's first atom
   // neighbour-list systems (gb_cut with a cutoff): list build and reuse
   int32_t nl;           // 1: pair work from the list (chunk items), 0: all tile pairs
@@ -247,7 +249,10 @@ struct GridBarrier {
   int pad;
 };
 
-inline __host__ __device__ bool persist_by_unit(const DeviceView& v) { return v.n_units <= kPersistUnits; }
+// Waves per item in the persistent kernel (v.shares > 1: every item has two shares).
+inline __host__ __device__ int persist_shares(const DeviceView& v) {
+  return v.shares < 2 || v.n_items > kPersistPairs ? 1 : (v.n_items > kPersistQuads ? 2 : kUnitWaves);
+}
 
 // Launchers (defined in the .hip translation units).
 void launch_tile_boxes(const DeviceView& v, hipStream_t s);                // -> tbox (every evaluation)
@@ -293,7 +298,9 @@ void launch_tick(unsigned long long* out, hipStream_t s);
 int persist_max_blocks();
 // Fused step kernel (prx_fused.hip): n_steps steps of every listed system,
 // one workgroup per system (slot_ranges rows as for launch_kinetic).
-void launch_fused_steps(const DeviceView& v, const int32_t* slot_ranges, int n_slots, int n_steps, hipStream_t s);
+// max_atoms: of the largest listed system
+void launch_fused_steps(const DeviceView& v, const int32_t* slot_ranges, int n_slots, int max_atoms, int n_steps,
+                        hipStream_t s);
 hipError_t launch_persist_steps(const DeviceView& v, const int32_t* slot_ranges, int n_slots, int n_steps,
                                 bool has_nl, GridBarrier* bar, int n_blocks, hipStream_t s);
 

@@ -370,15 +370,16 @@ struct prx_engine {
   bool has_skin = false;          // and one of these has a skin
   // step path: 0 = auto (the fused kernel when every system fits in
   // kFusedAutoAtoms atoms and none uses a neighbour list, else graphs: on
-  // MI355X the fused kernel beats graphs only on systems of one tile. us a step,
-  // fused / graphs: 64 atoms 32 / 43, 100 atoms 52 / 43, 138 atoms 77 / 44; 192
-  // systems of 64 atoms 34 / 47, of 100 atoms 57 / 54), 1 = captured graphs,
+  // MI355X the fused kernel beats graphs on systems of one tile, unless
+  // there are thousands. us a step, fused / graphs: 64 atoms 31 / 39, 100 atoms 47 / 40,
+  // 138 atoms 56 / 41; 192 systems of 64 atoms 32 / 44, of 100 atoms 48 / 51; 2,000
+  // systems of 64 atoms 142 / 105), 1 = captured graphs,
   // 2 = the persistent kernel, 3 = the fused kernel (one workgroup per system)
   int32_t step_mode = 0;
   static constexpr int32_t kFusedAutoAtoms = prx::kTile;
   // Steps recorded into a caller's own graph, in which no step graph can be
   // captured or launched: systems up to this size, as the passes themselves (138
-  // atoms 44 us a step, 78 fused), or fused in calls of more than kGraphSteps.
+  // atoms 41 us a step, 56 fused), or fused in calls of more than kGraphSteps.
   static constexpr int32_t kRecordAtoms = 3 * prx::kTile;
   static constexpr int kGraphSteps = 50;  // steps per step graph
   int32_t max_system_atoms = 0;   // largest live system (rebuild)
@@ -958,11 +959,9 @@ struct prx_engine {
       s.c.item_base = ib;
       s.c.tile0 = (int32_t)tiles.size();
       const int nT = (s.n + prx::kTile - 1) / prx::kTile;
-      s.c.unit0 = (int32_t)units.size();
       s.c.pack0 = offsets.back();
       const int32_t sh = prx::append_units(s.items, nT, n_list, ib, units);
       shares = shares < 0 || shares == sh ? sh : 0;
-      s.c.n_units = (int32_t)units.size() - s.c.unit0;
       push_const(sid, s.c);
       for (int T = 0; T < nT; ++T) {
         tiles.push_back(make_int4(s.a0 + T * prx::kTile, std::min(prx::kTile, s.n - T * prx::kTile), sid, T));
@@ -1216,8 +1215,8 @@ struct prx_engine {
   // The persistent kernel: at most one unit, or one item per wave, and one tile
   // per block in each pass, within the co-resident grid.
   void steps_persistent(int n_steps, hipStream_t s) {
-    const int64_t pair_blocks =
-        prx::persist_by_unit(v) ? v.n_units : ((int64_t)v.n_items + prx::kUnitWaves - 1) / prx::kUnitWaves;
+    const int per = prx::kUnitWaves / prx::persist_shares(v);  // items of a block
+    const int64_t pair_blocks = ((int64_t)v.n_items + per - 1) / per;
     const int64_t want = std::max<int64_t>({(int64_t)v.n_tiles, pair_blocks, 1});
     const int blocks = (int)std::min<int64_t>(want, persist_blocks);
     for (int left = n_steps; left > 0;) {
@@ -1252,7 +1251,7 @@ struct prx_engine {
       if (use_fused(recorded)) {
         for (int left = n_steps; left > 0;) {
           const int k = std::min(left, kPersistChunk);
-          prx::launch_fused_steps(v, d_ranges, (int)order.size(), k, stream);
+          prx::launch_fused_steps(v, d_ranges, (int)order.size(), max_system_atoms, k, stream);
           HIPCHECK(hipGetLastError());
           left -= k;
         }

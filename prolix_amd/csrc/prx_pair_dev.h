@@ -1636,11 +1636,6 @@ static_assert(kAnyWaveLds >= kWaveLds<BornPass> && kAnyWaveLds >= kWaveLds<Force
 static_assert(kAnyGroupLds >= kGroupLds<BornPass> && kAnyGroupLds >= kGroupLds<ChainPass> &&
                   kAnyGroupLds >= kUnitWaves * kAnyWaveLds, "");
 
-// Unit i of the list (of items in four quarters each, no list is kept).
-__device__ __forceinline__ PairUnit unit_of(const DeviceView& v, int i) {
-  return v.units != nullptr ? v.units[i] : PairUnit{i, 1, kUnitWaves};
-}
-
 // Wave k of a group of W takes its part of unit u; M: the group's memory. meet: the
 // unit holds exactly two workgroup barriers, also one of whole items or of items
 // without work (groups of one workgroup, and waves of one group, meet the same

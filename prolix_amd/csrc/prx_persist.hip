@@ -4,8 +4,8 @@
 // A step of the graph path is 6 dependent kernel launches (plus the bonded
 // branch and, for neighbour-list systems, the list build). For an engine
 // with little pair work (one system of a few thousand atoms) the step time is
-// then set by launch and dependency latency, not by the work: ~90 us per step
-// at 138 or 2,500 atoms against ~10 us of kernels. Here one launch runs K
+// then set by launch and dependency latency, not by the work: 41 us per step
+// at 138 atoms, 53 at 2,500, against ~10 us of kernels. Here one launch runs K
 // steps; each pass is a grid-stride loop over the same per-item and per-tile
 // device functions the graph's kernels call (prx_*_dev.h), so every result
 // is bit for bit the graph path's.
@@ -66,16 +66,14 @@ __device__ __forceinline__ bool grid_sync(GridBarrier* bar, unsigned& gen) {
   return s_ok != 0;
 }
 
-// One pair pass over the grid: short lists a unit per block (138 atoms 48 us a
-// step, 72 with an item per wave), longer ones an item per wave, with a quarter of
-// the blocks, whose number the grid barriers' time grows with (2,500 atoms 201 us
-// a step, 480 with units).
+// One pair pass over the grid (persist_shares: waves per item).
 template <class Pass>
 __device__ __forceinline__ void pair_pass(const DeviceView& v, int wave, int n_waves, int uw, float4* L) {
-  const bool units = persist_by_unit(v);
-  const int end = units ? v.n_units : v.n_items, step = units ? (int)gridDim.x : n_waves;
-  for (int k = units ? (int)blockIdx.x : wave; k < end; k += step) {
-    const PairUnit u = units ? unit_of(v, k) : PairUnit{k, 1, 1};
+  const int shares = persist_shares(v), per = kUnitWaves / shares;  // waves per item, items per block
+  const bool units = shares > 1;
+  const int step = units ? (int)gridDim.x * per : n_waves;
+  for (int k = units ? (int)blockIdx.x * per : wave; k < v.n_items; k += step) {
+    const PairUnit u = {k, (int16_t)(units ? min(per, v.n_items - k) : 1), (int16_t)shares};
     pair_unit<Pass, kUnitWaves, true>(v, u, units ? uw : 0, units, units ? L : L + uw * kAnyWaveLds);
     if (units) __syncthreads();
   }
