@@ -263,9 +263,9 @@ def main():
     t_k = prof[pair_pass] * 1e-3
     achieved = FLOPS_PER_PAIR[pair_pass] * pairs_per_step / t_k / 1e12
     pair_total_s = sum(prof[k] for k in FLOPS_PER_PAIR) * 1e-3
-    full_name = {"born_pairs": "void prx::k_born_pairs<1>(prx::DeviceView)",
-                 "force_pairs": "void prx::k_force_pairs<1, false>(prx::DeviceView)",
-                 "chain_pairs": "void prx::k_chain_pairs<1>(prx::DeviceView)"}[pair_pass]
+    full_name = {"born_pairs": "void prx::k_born_pairs<2>(prx::DeviceView)",
+                 "force_pairs": "void prx::k_force_pairs<2, false>(prx::DeviceView)",
+                 "chain_pairs": "void prx::k_chain_pairs<2>(prx::DeviceView)"}[pair_pass]
     traffic = None
     traffic_file = os.path.join(ROOT, "profiles", "hbm_traffic_batch256.json")
     if os.path.exists(traffic_file) and a.n_systems == 256:
@@ -273,8 +273,8 @@ def main():
             traffic = json.load(fh)["kernels"].get(full_name, {}).get("bytes")
     roofline = {
         "bound": "valu",
-        "kernel": {"born_pairs": "k_born_pairs<1>", "force_pairs": "k_force_pairs<1, false>",
-                   "chain_pairs": "k_chain_pairs<1>"}[pair_pass],
+        "kernel": {"born_pairs": "k_born_pairs<2>", "force_pairs": "k_force_pairs<2, false>",
+                   "chain_pairs": "k_chain_pairs<2>"}[pair_pass],
         "achieved": achieved,
         "peak": PEAK_FP32,
         "unit": "TFLOP/s",

@@ -239,8 +239,9 @@ int prx_engine_set_nl_skin(prx_engine* eng, double skin);
  *     side; PRX_ERR_STATE if a system uses a neighbour list;
  * 0 = auto (default): fused when every system has at most 64 atoms and
  *     none uses a neighbour list (measured fastest there on MI355X), graphs
- *     otherwise; steps recorded into a caller's own graph are fused up to
- *     192 atoms (no graph can be launched there).
+ *     otherwise. Steps recorded into a caller's own graph, where no graph can
+ *     be launched, are recorded as the passes themselves for systems up to
+ *     192 atoms and 50 steps a call, and fused in longer calls.
  * PRX_ERR_STATE for 2 where cooperative launches are unavailable. No
  * counterpart in prolix (its loop is jax.lax.fori_loop,
  * physics/simulate.py:253-254). */

@@ -179,9 +179,9 @@ struct DeviceView {
   // pair work
   const PairItem* items;
   int32_t n_items;
-  const PairUnit* units;  // nullptr: unit = item, every item cut
+  const PairUnit* units;  // written and read where systems differ in waves per item (shares 0)
   int32_t n_units;
-  int32_t shares;  // of every item, or 0 where systems differ
+  int32_t shares;  // waves of every item, or 0 where systems differ
   float4* part;        // partial sums, 2 * 64 float4 per item (part1 / part3 / part4 below)
   const int4* tiles;   // per tile: (first atom, atoms in tile, slot, tile index T)
   int32_t n_tiles;

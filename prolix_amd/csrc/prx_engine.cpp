@@ -1034,14 +1034,14 @@ struct prx_engine {
       HIPCHECK(hipMemcpy(d_tiles, tiles.data(), tiles.size() * sizeof(int4), hipMemcpyHostToDevice));
     if (!items.empty())
       HIPCHECK(hipMemcpy(d_items, items.data(), items.size() * sizeof(prx::PairItem), hipMemcpyHostToDevice));
-    if (!units.empty() && shares != prx::kUnitWaves)  // else unit k is item k, and no list is read
+    if (!units.empty() && shares == 0)  // else blocks take items, and no list is read
       HIPCHECK(hipMemcpy(d_units, units.data(), units.size() * sizeof(prx::PairUnit), hipMemcpyHostToDevice));
     if (!ranges.empty())
       HIPCHECK(hipMemcpy(d_ranges, ranges.data(), ranges.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     if (!map.empty()) HIPCHECK(hipMemcpy(d_map, map.data(), map.size() * sizeof(int32_t), hipMemcpyHostToDevice));
     v.items = d_items;
     v.n_items = (int32_t)items.size();
-    v.units = shares == prx::kUnitWaves ? nullptr : d_units;
+    v.units = d_units;
     v.shares = std::max(shares, 0);
     v.n_units = (int32_t)units.size();
     v.e_items = d_e_items;

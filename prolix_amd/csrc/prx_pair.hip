@@ -102,8 +102,8 @@ __global__ __launch_bounds__(kThreads<BLOCKS>) PRX_OCCUPANCY void k_born_pairs_b
   if (e < bonded_entries(v)) bonded_entry<ENERGY>(v, e);
 }
 
-// Blocks of a list: an item per wave in a long list or where every item is
-// whole, two or four waves per item where every item takes as many, else units.
+// Blocks of a list: one, two or four waves per item where every item takes as many,
+// else units.
 // Two-wave blocks free their slots as soon as one item is done, and read no unit list:
 // 8,000 atoms 144 us an evaluation, 148 with units of two items.
 static inline int list_blocks(const DeviceView& v) { return v.shares; }
